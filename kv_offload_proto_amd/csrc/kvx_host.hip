@@ -984,19 +984,18 @@ int kvx_sieve_ht_init(uint64_t device_buffer_tokens, uint64_t device_buffer_ht, 
         a.paddedBufferSize = padded_buffer_size;
         a.htSize = ht_size;
         if (static_cast<uint64_t>(num_reqs) * layer_num == 0) return;
-        // the parallel build when its LDS form fits, else the batched wave
-        // build (larger tables), else one lane per table on the table in LDS
-        // or in HBM
-        const size_t ldsPar = kvx::sieve_ht_init_par_lds(ht_size, device_buffer_size);
-        const size_t ldsWave = kvx::sieve_ht_init_wave_lds(ht_size, device_buffer_size);
+        // the parallel build with the table, or the part that holds homes, in
+        // LDS; else one lane per table on the table in LDS or in HBM
+        const size_t ldsSmall = kvx::sieve_ht_init_small_lds(ht_size, device_buffer_size);
+        const size_t ldsLarge = kvx::sieve_ht_init_large_lds(ht_size, device_buffer_size);
         kvx::InitForm form = kvx::InitForm::kInOrder;
         size_t lds = static_cast<size_t>(ht_size) * 2;
-        if (ldsPar != 0 && ldsPar <= g.ldsLimit) {
-            form = kvx::InitForm::kParallel;
-            lds = ldsPar;
-        } else if (ldsWave != 0 && ldsWave <= g.ldsLimit) {
-            form = kvx::InitForm::kWave;
-            lds = ldsWave;
+        if (ldsSmall != 0 && ldsSmall <= g.ldsLimit) {
+            form = kvx::InitForm::kSmall;
+            lds = ldsSmall;
+        } else if (ldsLarge != 0 && ldsLarge <= g.ldsLimit) {
+            form = kvx::InitForm::kLarge;
+            lds = ldsLarge;
         } else if (lds > g.ldsLimit) {
             lds = 0;
         }

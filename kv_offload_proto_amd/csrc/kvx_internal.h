@@ -319,16 +319,16 @@ constexpr uint32_t kTblLdsBytes = kTblHistBytes + kTblWinWords * 8u;
 // Launchers (implemented next to their kernels).
 hipError_t launch_sieve_update(const HispSieveUpdateArgs &a, uint64_t overflowSlot, int variant,
                                size_t ldsBytes, hipStream_t stream);
-// Forms of the admission build: kParallel (ldsBytes =
-// sieve_ht_init_par_lds(htSize, dbs)), kWave (ldsBytes =
-// sieve_ht_init_wave_lds(htSize, dbs)), kInOrder (one lane per table; the
+// Forms of the admission build: kSmall (ldsBytes =
+// sieve_ht_init_small_lds(htSize, dbs)), kLarge (ldsBytes =
+// sieve_ht_init_large_lds(htSize, dbs)), kInOrder (one lane per table; the
 // table in LDS when ldsBytes = 2 htSize, in HBM when 0).  The size functions
 // return 0 where their form does not apply.
-enum class InitForm { kParallel, kWave, kInOrder };
+enum class InitForm { kSmall, kLarge, kInOrder };
 hipError_t launch_sieve_ht_init(const HispSieveHtInitArgs &a, uint64_t overflowSlot, size_t ldsBytes,
                                 hipStream_t stream, InitForm form);
-size_t sieve_ht_init_par_lds(uint32_t htSize, uint32_t dbs);
-size_t sieve_ht_init_wave_lds(uint32_t htSize, uint32_t dbs);
+size_t sieve_ht_init_small_lds(uint32_t htSize, uint32_t dbs);
+size_t sieve_ht_init_large_lds(uint32_t htSize, uint32_t dbs);
 hipError_t sieve_set_lds_limit(size_t bytes);
 hipError_t sieve_fast_set_lds_limit(size_t bytes);
 hipError_t launch_sieve_update_wave(const HispSieveUpdateArgs &a, uint64_t overflowSlot, int32_t *shadow,

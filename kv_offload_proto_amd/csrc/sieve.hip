@@ -147,205 +147,163 @@ __global__ __launch_bounds__(256) void kvx_sieve_ht_init(KvxLaunch<HispSieveHtIn
     }
 }
 
-// Parallel form of the same build for tables that fit LDS, one 256-lane
-// workgroup per (layer, pool row).  Linear probing fills the same set of
-// cells whatever the insertion order: with n(c) keys homed at cell c, the
-// backlog b(c) = max(0, b(c-1) + n(c) - 1) counts the keys homed at or before
-// c still waiting for a cell, and c is in use iff b(c-1) + n(c) >= 1.  A key
-// never leaves the cluster (maximal run of used cells) holding its home, so
-// inserting each cluster's keys alone, in slot order, gives the sequential
-// layout.  A later slot with a token already inserted meets the earlier entry
-// on its probe path and is skipped (hisp_kernel_common.h:97-112); both share
-// a home, so it is dropped from its home's list instead.
+// Parallel form of the same build.  Sequential first-come-first-served
+// inserts leave every key in the first cell from its home that no earlier key
+// took, so the table is the stable matching in which keys prefer cells nearer
+// their home and every cell prefers the smaller slot (deferred acceptance,
+// Gale and Shapley 1962).  It does not depend on the order of the proposals:
+// every lane proposes its slots to their cells with an atomic min, and carries
+// the slot that a cell gives up (its own or the one it displaced) to the next
+// cell.  The proposals number the keys plus the sum of their distances from
+// home, whatever the order.
 //
-// LDS: table (2H B), per-home list ends (2H B, 16-bit, paired for atomics),
-// the slots bucketed by home (2 B each), the used-cell bitmap (H/8 B), the
-// scans' lane values (2 KiB); nothing static.
-constexpr int32_t kInitThreads = 256;
+// A later slot with a token already inserted meets the earlier entry on its
+// probe path and is skipped (hisp_kernel_common.h:97-112).  With such slots
+// inserted as keys of their own, each lies behind its token's first slot (same
+// home, which that slot left no nearer cell free for), so a walk from the home
+// finds every one of them; the table is then built again without them.
+//
+// A table of up to kInitLdsCells cells stands in LDS as 32-bit cells (the
+// slot, all ones = empty): one returning atomic per proposal.  The bound is
+// latency: a lane's chain of LDS round trips, four slots each at 4096 slots.
+// The form it replaced (per-home counts, two scans of a contiguous run of
+// cells per lane, a lane per cluster) read the table at strides that put half
+// a wave on one bank: an admission of 61 such tables took 157 us, now 67.
+constexpr int32_t kInitThreads = 1024;
+constexpr int32_t kInitLdsCells = 32768;
+constexpr int32_t kInitSmallThreads = 256;  // rows of up to kInitSmallSlots slots
+constexpr int32_t kInitSmallSlots = 1024;
+constexpr int kInitUnroll = 4;              // slots whose tokens a lane loads together
 
-__global__ __launch_bounds__(kInitThreads) void kvx_sieve_ht_init_par(KvxLaunch<HispSieveHtInitArgs> L)
+typedef __attribute__((address_space(1))) const int32_t GTok;
+typedef __attribute__((address_space(1))) uint16_t GCell;
+typedef uint32_t Chunk __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) Chunk GChunk;
+
+// The tokens of a row: read from the state, or, at admission, slot s holds
+// token s for s < n0 (no token is held twice then).
+template <bool kIdentity>
+struct RowTokens {
+    GTok *tok;
+    int32_t n0;
+    __device__ __forceinline__ int32_t operator()(int32_t s) const
+    {
+        if constexpr (kIdentity) return s < n0 ? s : -1;
+        else return tok[s];
+    }
+};
+
+template <bool kIdentity>
+__device__ __forceinline__ void init_table_lds(uint8_t *smem, const RowTokens<kIdentity> token, GCell *gHt, int32_t dbs,
+                                               int32_t H)
 {
-    extern __shared__ __align__(16) uint8_t smem[];
-    const HispSieveHtInitArgs &a = L.a;
-    const int32_t numReqs = static_cast<int32_t>(a.numReqs);
-    const int32_t layerNum = static_cast<int32_t>(a.layerNum);
-    const int32_t poolSize = static_cast<int32_t>(a.poolSize);
-    const int32_t dbs = static_cast<int32_t>(a.deviceBufferSize);
-    const int32_t padded = static_cast<int32_t>(a.paddedBufferSize);
-    const int32_t H = static_cast<int32_t>(a.htSize);
-    const int32_t mask = H - 1;
-    const int32_t b = blockIdx.x;
-    if (b >= layerNum * numReqs) return;
-    const int32_t layer = b / numReqs;
-    const int64_t reqIdx = static_cast<int64_t>(a.reqStart) + b % numReqs;
-    if (reqIdx < 0 || reqIdx >= poolSize) return;
-    const int32_t *tok = reinterpret_cast<const int32_t *>(a.deviceBufferTokens) +
-                         (static_cast<int64_t>(layer) * poolSize + reqIdx) * padded;
-    uint16_t *gHt = reinterpret_cast<uint16_t *>(a.deviceBufferHt) +
-                    (static_cast<int64_t>(layer) * poolSize + reqIdx) * H;
-
-    const int32_t tid = threadIdx.x;
-    const int32_t per = H / kInitThreads;  // cells (homes) per lane, >= 4 (H >= 1024)
-    const int32_t c0 = tid * per;
-    uint16_t *ht = reinterpret_cast<uint16_t *>(smem);
-    uint16_t *ends = ht + H;  // per home: inclusive prefix of the counts, then (after the scatter) the list start
-    uint32_t *ends32 = reinterpret_cast<uint32_t *>(ends);
-    uint16_t *keys = ends + H;
-    uint32_t *used = reinterpret_cast<uint32_t *>(keys + ((dbs + 7) & ~7));
-    int32_t *sP = reinterpret_cast<int32_t *>(used + H / 32);  // the scans' lane values
-    int32_t *sQ = sP + kInitThreads;
-    int32_t &sTotal = sQ[kInitThreads];
-    constexpr uint16_t kGone = 0xFFFF;  // a dropped duplicate or an inserted slot
-    auto is_used = [&](int32_t c) { return (used[c >> 5] >> (c & 31)) & 1u; };
-
-    // clear the table, the counts and the bitmap
-    for (int32_t i = tid; i < H / 4; i += kInitThreads) reinterpret_cast<uint4 *>(smem)[i] = make_uint4(0, 0, 0, 0);  // 4H bytes
-    for (int32_t i = tid; i < H / 32; i += kInitThreads) used[i] = 0u;
-    __syncthreads();
-    // keys per home (two 16-bit counts per word; a count stays below 2^16)
-    for (int32_t s = tid; s < dbs; s += kInitThreads) {
-        const int32_t t = tok[s];
-        if (t >= 0) {
-            const int32_t h = static_cast<int32_t>(ht_hash(t)) & mask;
-            atomicAdd(ends32 + (h >> 1), 1u << ((h & 1) * 16));
-        }
+    constexpr uint32_t kEmpty = 0xFFFFFFFFu;
+    const int32_t mask = H - 1, tid = threadIdx.x, nt = blockDim.x;
+    uint32_t *cell = reinterpret_cast<uint32_t *>(smem);
+    uint32_t *drop = cell + H;  // slots whose token an earlier slot holds
+    const int32_t dropWords = (dbs + 31) / 32;
+    if constexpr (!kIdentity) {
+        for (int32_t i = tid; i < dropWords; i += nt) drop[i] = 0u;
     }
-    __syncthreads();
-    // inclusive prefix over the homes: lane sums, a scan of the lane sums, then the lane's run
-    int32_t sum = 0;
-    for (int32_t i = 0; i < per; ++i) sum += ends[c0 + i];
-    sP[tid] = sum;
-    __syncthreads();
-    for (int32_t o = 1; o < kInitThreads; o <<= 1) {
-        const int32_t v = tid >= o ? sP[tid - o] : 0;
-        __syncthreads();
-        sP[tid] += v;
-        __syncthreads();
-    }
-    int32_t run = sP[tid] - sum;
-    for (int32_t i = 0; i < per; ++i) {
-        run += ends[c0 + i];
-        ends[c0 + i] = static_cast<uint16_t>(run);
-    }
-    if (tid == kInitThreads - 1) sTotal = sP[kInitThreads - 1];
-    __syncthreads();
-    // bucket the slots by home: each key takes the next position down from
-    // its home's end, so the entry ends as the home's list start
-    for (int32_t s = tid; s < dbs; s += kInitThreads) {
-        const int32_t t = tok[s];
-        if (t >= 0) {
-            const int32_t h = static_cast<int32_t>(ht_hash(t)) & mask;
-            const uint32_t sh = static_cast<uint32_t>(h & 1) * 16u;
-            const uint32_t old = atomicSub(ends32 + (h >> 1), 1u << sh);
-            keys[((old >> sh) & 0xFFFFu) - 1u] = static_cast<uint16_t>(s);
-        }
-    }
-    __syncthreads();
-    const int32_t total = sTotal;
-    auto list_end = [&](int32_t h) { return h + 1 < H ? static_cast<int32_t>(ends[h + 1]) : total; };
-    // per home: slot order, duplicates dropped, the count kept in the (still
-    // empty) table cell; the lane's segment as a backlog map x -> max(P, x + Q)
-    int32_t P = 0, Q = 0;
-    for (int32_t i = 0; i < per; ++i) {
-        const int32_t h = c0 + i;
-        const int32_t st = ends[h], en = list_end(h);
-        for (int32_t j = st + 1; j < en; ++j) {
-            const uint16_t v = keys[j];
-            int32_t k = j;
-            for (; k > st && keys[k - 1] > v; --k) keys[k] = keys[k - 1];
-            keys[k] = v;
-        }
-        int32_t n = 0;
-        for (int32_t j = st; j < en; ++j) {
-            bool dup = false;
-            if (j > st) {
-                const int32_t tj = tok[keys[j]];
-                for (int32_t k = st; k < j && !dup; ++k) dup = keys[k] != kGone && tok[keys[k]] == tj;
-            }
-            if (dup) keys[j] = kGone;
-            else ++n;
-        }
-        ht[h] = static_cast<uint16_t>(n);
-        P = max(0, P + n - 1);
-        Q += n - 1;
-    }
-    sP[tid] = P;
-    sQ[tid] = Q;
-    __syncthreads();
-    // compose the segment maps in cell order (inclusive scan); the ring's map
-    // has Q < 0 (fewer keys than cells), so its fixed point -- the backlog
-    // entering cell 0 -- is its P
-    for (int32_t o = 1; o < kInitThreads; o <<= 1) {
-        const bool has = tid >= o;
-        const int32_t pe = has ? sP[tid - o] : 0, qe = has ? sQ[tid - o] : 0;
-        __syncthreads();
-        if (has) {
-            const int32_t pc = sP[tid], qc = sQ[tid];
-            sP[tid] = max(pc, pe + qc);
-            sQ[tid] = qe + qc;
+    for (int attempt = 0; attempt < 2; ++attempt) {
+        for (int32_t i = tid; i < H / 4; i += nt) {
+            reinterpret_cast<uint4 *>(cell)[i] = make_uint4(kEmpty, kEmpty, kEmpty, kEmpty);
         }
         __syncthreads();
-    }
-    const int32_t x0 = sP[kInitThreads - 1];
-    int32_t x = tid == 0 ? x0 : max(sP[tid - 1], x0 + sQ[tid - 1]);
-    for (int32_t i = 0; i < per; ++i) {
-        const int32_t h = c0 + i;
-        const int32_t n = ht[h];
-        if (x + n >= 1) atomicOr(used + (h >> 5), 1u << (h & 31));
-        x = max(0, x + n - 1);
-        ht[h] = 0;
-    }
-    __syncthreads();
-    // each cluster, by the lane holding its first cell: its keys in slot
-    // order, each to the first free cell from its home (a cluster of L cells
-    // costs O(L^2) LDS reads: short at these load factors, at most H/2 keys)
-    for (int32_t i = 0; i < per; ++i) {
-        const int32_t c = c0 + i;
-        if (!is_used(c) || is_used((c - 1) & mask)) continue;
-        int32_t len = 0;
-        while (len < H && is_used((c + len) & mask)) ++len;
-        for (;;) {
-            int32_t best = 0x10000, bj = -1, bh = 0;
-            for (int32_t u = 0; u < len; ++u) {
-                const int32_t h = (c + u) & mask;
-                const int32_t en = list_end(h);
-                for (int32_t j = ends[h]; j < en; ++j) {
-                    const int32_t v = keys[j];
-                    if (v == kGone) continue;
-                    if (v < best) {
-                        best = v;
-                        bj = j;
-                        bh = h;
-                    }
-                    break;  // the home's list is in slot order
+        for (int32_t s0 = tid; s0 < dbs; s0 += kInitUnroll * nt) {
+            int32_t t[kInitUnroll];
+#pragma unroll
+            for (int q = 0; q < kInitUnroll; ++q) t[q] = s0 + q * nt < dbs ? token(s0 + q * nt) : -1;
+#pragma unroll
+            for (int q = 0; q < kInitUnroll; ++q) {
+                const int32_t s = s0 + q * nt;
+                if (t[q] < 0) continue;
+                if (!kIdentity && attempt != 0 && ((drop[s >> 5] >> (s & 31)) & 1u)) continue;
+                uint32_t v = static_cast<uint32_t>(s);
+                for (uint32_t c = ht_hash(t[q]) & static_cast<uint32_t>(mask);;) {
+                    const uint32_t old = atomicMin(cell + c, v);
+                    if (old == kEmpty) break;  // fewer keys than cells: every chain ends
+                    v = old > v ? old : v;
+                    c = (c + 1u) & static_cast<uint32_t>(mask);
                 }
             }
-            if (bj < 0) break;
-            keys[bj] = kGone;
-            int32_t y = bh;
-            for (int32_t n = 0; n < len && ht[y] != 0; ++n) y = (y + 1) & mask;
-            ht[y] = static_cast<uint16_t>(best + 1);
+        }
+        __syncthreads();
+        if constexpr (kIdentity) {
+            break;
+        } else {
+            if (attempt != 0) break;
+            int dup = 0;
+            for (int32_t s0 = tid; s0 < dbs; s0 += kInitUnroll * nt) {
+                int32_t t[kInitUnroll];
+#pragma unroll
+                for (int q = 0; q < kInitUnroll; ++q) t[q] = s0 + q * nt < dbs ? token(s0 + q * nt) : -1;
+#pragma unroll
+                for (int q = 0; q < kInitUnroll; ++q) {
+                    const int32_t s = s0 + q * nt;
+                    if (t[q] < 0) continue;
+                    uint32_t c = ht_hash(t[q]) & static_cast<uint32_t>(mask);
+                    for (uint32_t e = cell[c]; e != static_cast<uint32_t>(s) && e != kEmpty;) {
+                        if (token(static_cast<int32_t>(e)) == t[q]) {
+                            dup = 1;
+                            atomicOr(drop + (s >> 5), 1u << (s & 31));
+                            break;
+                        }
+                        c = (c + 1u) & static_cast<uint32_t>(mask);
+                        e = cell[c];
+                    }
+                }
+            }
+            if (__syncthreads_or(dup) == 0) break;
         }
     }
-    __syncthreads();
-    block_copy16(gHt, ht, static_cast<uint32_t>(H) * 2u);
+    // an entry is slot + 1, 0 = empty: all ones plus one
+    GChunk *out = reinterpret_cast<GChunk *>(gHt);
+    for (int32_t i = tid; i < H / 8; i += nt) {
+        const uint4 lo = reinterpret_cast<const uint4 *>(cell)[2 * i], hi = reinterpret_cast<const uint4 *>(cell)[2 * i + 1];
+        auto two = [](uint32_t x, uint32_t y) { return ((x + 1u) & 0xFFFFu) | ((y + 1u) << 16); };
+        out[i] = Chunk{two(lo.x, lo.y), two(lo.z, lo.w), two(hi.x, hi.y), two(hi.z, hi.w)};
+    }
 }
 
-// Admission build for tables beyond the parallel form's LDS budget, one
-// 256-lane workgroup per (layer, pool row); the table of the sequential
-// inserts (hisp_sieve_ht_init.cpp:14-60).  Every lane first marks its slots'
-// tokens in an LDS bitmap: a token met twice (a later slot would meet the
-// earlier entry and insert nothing) or one beyond the bitmap sends the row to
-// the one-lane inserts.  Otherwise one wave inserts 64 slots at a time over a
-// three-level bitmap of used cells: each key's first free cell at or after its
-// home in the table before the batch, then the free cells in increasing
-// order, each taken by the earliest key of the batch whose first free cell is
-// at or before it -- linear probing's cells in slot order.  A batch whose
-// probe wraps past the table's end, or that has fewer free cells than keys at
-// or after its last first-free cell (its sweep could wrap), inserts its keys
-// one by one.
+// The same build for tables beyond kInitLdsCells (65536 cells and more).  A
+// hash has 16 bits, so every home lies in the first 65536 cells: those stand
+// in LDS as the table's own 16-bit entries (compare and swap on the
+// containing word), and the keys that run past them, in larger tables, take
+// the cells from 65536 on in slot order (no key is homed there, so each cell
+// takes the smallest slot waiting; they never wrap: a row holds fewer than
+// 65536 keys).
+//
+// The slots go in increasing passes, each half of the cells left free, so
+// that the proposals of a pass stay few however full the table gets; a cell
+// taken in an earlier pass holds a smaller slot and is skipped by a bitmap
+// (occ, with a bit per full word in `full`).  A chain of more than
+// kInitMaxHops proposals (homes packed into few cells) sends the row to the
+// one-wave sweep below, whose time does not depend on the distances.
+//
+// A token held twice, or one beyond the bitmap that finds those, sends the
+// row to the one-lane inserts.
+//
+// Against the sweep alone: four tables of 65518 slots, admission pattern, 4541
+// -> 175 us with the calls around the build; 64 tables of 16000 random tokens
+// 1379 -> 21 us; four of 60000 random tokens 4221 -> 368 us.
 constexpr int32_t kWaveInitTokenBits = 1 << 20;
 constexpr int32_t kFreeCap = 4;  // free cells counted between neighbouring first-free cells
+constexpr int32_t kInitHomes = 65536;
+constexpr int32_t kInitMaxHops = 512;
+constexpr int32_t kInitWords = kInitHomes / 64;           // words of the occ and spill bitmaps
+constexpr int32_t kInitTailEnd = 2 * kInitHomes;          // no cell at or past it is ever taken
+constexpr int32_t kInitHelpers = 3;                       // workgroups per row beside the one that builds
+
+struct InitLargeLds {
+    uint32_t cells[kInitHomes / 2];
+    uint64_t occ[kInitWords], spill[kInitWords];
+    uint64_t full[kInitWords / 64];
+    uint32_t part[kInitThreads / 64 + 1];
+    int32_t inOrder, stop;
+};
+static_assert(kWaveInitTokenBits / 8 <= sizeof(InitLargeLds::cells), "the token bitmap takes the cells' place");
+static_assert(kInitWords == kInitThreads, "one bitmap word per lane");
 
 __device__ __forceinline__ void wave_lds_sync()
 {
@@ -354,68 +312,36 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__global__ __launch_bounds__(kInitThreads) void kvx_sieve_ht_init_wave(KvxLaunch<HispSieveHtInitArgs> L)
+// Entry v proposes to cell c: 0 when the cell was empty, else the entry that
+// goes on to the next cell.
+__device__ __forceinline__ uint32_t propose16(uint32_t *cells, uint32_t c, uint32_t v)
 {
-    extern __shared__ __align__(16) uint8_t smem[];
-    __shared__ int32_t sInOrder;
-    const HispSieveHtInitArgs &a = L.a;
-    const int32_t numReqs = static_cast<int32_t>(a.numReqs);
-    const int32_t layerNum = static_cast<int32_t>(a.layerNum);
-    const int32_t poolSize = static_cast<int32_t>(a.poolSize);
-    const int32_t dbs = static_cast<int32_t>(a.deviceBufferSize);
-    const int32_t padded = static_cast<int32_t>(a.paddedBufferSize);
-    const int32_t H = static_cast<int32_t>(a.htSize);  // a power of two in [65536, 2^20] (launcher)
+    uint32_t *w = cells + (c >> 1);
+    const uint32_t sh = (c & 1u) * 16u;
+    uint32_t old = *w;
+    for (;;) {
+        const uint32_t cur = (old >> sh) & 0xFFFFu;
+        if (cur != 0u && cur < v) return v;
+        const uint32_t prev = atomicCAS(w, old, (old & ~(0xFFFFu << sh)) | (v << sh));
+        if (prev == old) return cur;
+        old = prev;
+    }
+}
+
+// One wave inserts 64 slots at a time over a three-level bitmap of used
+// cells: each key's first free cell at or after its home in the table before
+// the batch, then the free cells in increasing order, each taken by the
+// earliest key of the batch whose first free cell is at or before it -- linear
+// probing's cells in slot order.  A batch whose probe wraps past the table's
+// end, or that has fewer free cells than keys at or after its last first-free
+// cell (its sweep could wrap), inserts its keys one by one.  The table is
+// zeroed before.
+template <bool kIdentity>
+__device__ void init_table_sweep(uint8_t *smem, const RowTokens<kIdentity> token, GCell *gHt, int32_t dbs, int32_t H,
+                                 uint64_t overflowSlot)
+{
     const int32_t mask = H - 1;
-    const int32_t b = blockIdx.x;
-    if (b >= layerNum * numReqs) return;
-    const int32_t layer = b / numReqs;
-    const int64_t reqIdx = static_cast<int64_t>(a.reqStart) + b % numReqs;
-    if (reqIdx < 0 || reqIdx >= poolSize) return;
-    // global-space pointers: flat accesses would also count against the LDS
-    // wait counter, and every bitmap read would wait for the table's stores
-    typedef __attribute__((address_space(1))) const int32_t GTok;
-    typedef __attribute__((address_space(1))) uint16_t GCell;
-    typedef uint32_t Chunk __attribute__((ext_vector_type(4)));
-    typedef __attribute__((address_space(1))) Chunk GChunk;
-    GTok *tok = reinterpret_cast<GTok *>(a.deviceBufferTokens) + (static_cast<int64_t>(layer) * poolSize + reqIdx) * padded;
-    GCell *gHt = reinterpret_cast<GCell *>(a.deviceBufferHt) + (static_cast<int64_t>(layer) * poolSize + reqIdx) * H;
-    const int32_t tid = threadIdx.x;
     const int32_t lane = static_cast<int32_t>(__lane_id());
-
-    // ---- clear the table; repeated and out-of-range tokens
-    uint32_t *tbits = reinterpret_cast<uint32_t *>(smem);
-    for (int32_t i = tid; i < H / 8; i += kInitThreads) reinterpret_cast<GChunk *>(gHt)[i] = Chunk{0u, 0u, 0u, 0u};
-    for (int32_t i = tid; i < kWaveInitTokenBits / 128; i += kInitThreads) {
-        reinterpret_cast<uint4 *>(smem)[i] = make_uint4(0, 0, 0, 0);
-    }
-    if (tid == 0) sInOrder = 0;
-    __syncthreads();
-    bool inOrder = false;
-    for (int32_t s = tid; s < dbs; s += kInitThreads) {
-        const int32_t t = tok[s];
-        if (t < 0) continue;
-        if (t >= kWaveInitTokenBits) {
-            inOrder = true;
-            continue;
-        }
-        const uint32_t bit = 1u << (t & 31);
-        if (atomicOr(tbits + (t >> 5), bit) & bit) inOrder = true;
-    }
-    if (__ballot(inOrder) != 0ull && lane == 0) atomicOr(&sInOrder, 1);
-    __syncthreads();
-    if (sInOrder) {
-        if (tid == 0) {
-            Guard g;
-            for (int32_t s = 0; s < dbs && g.code == 0; ++s) {
-                const int32_t t = tok[s];
-                if (t >= 0) ht_insert((uint16_t *)gHt, (const int32_t *)tok, padded, t, s, mask, g);
-            }
-            report_overflow(L.overflowSlot, g.code);
-        }
-        return;
-    }
-    if (tid >= 64) return;  // one wave from here on (no more workgroup barriers)
-
     // ---- used cells: word w bit i = cell 64w+i; full1 bit w = word w full;
     // full2 bit q = full1 word q full (bits past the last full1 word set)
     const int32_t nW = H >> 6, nS = nW >> 6, nT = (nS + 63) >> 6;
@@ -469,11 +395,11 @@ __global__ __launch_bounds__(kInitThreads) void kvx_sieve_ht_init_wave(KvxLaunch
 
     Guard g;
     const int32_t nb = (dbs + 63) >> 6;
-    int32_t tNext = lane < dbs ? tok[lane] : -1;
+    int32_t tNext = lane < dbs ? token(lane) : -1;
     for (int32_t bi = 0; bi < nb && g.code == 0; ++bi) {
         const int32_t s = (bi << 6) + lane;
         const int32_t t = tNext;
-        tNext = s + 64 < dbs ? tok[s + 64] : -1;  // the next batch's tokens, in flight meanwhile
+        tNext = s + 64 < dbs ? token(s + 64) : -1;  // the next batch's tokens, in flight meanwhile
         const bool valid = s < dbs && t >= 0;
         const uint64_t keys = __ballot(valid);
         if (keys == 0ull) continue;
@@ -629,7 +555,203 @@ __global__ __launch_bounds__(kInitThreads) void kvx_sieve_ht_init_wave(KvxLaunch
             }
         }
     }
-    if (lane == 0) report_overflow(L.overflowSlot, g.code);
+    if (lane == 0) report_overflow(overflowSlot, g.code);
+}
+
+template <bool kIdentity>
+__device__ __forceinline__ void init_table_large(uint8_t *smem, const RowTokens<kIdentity> token, GCell *gHt,
+                                                 int32_t padded, int32_t dbs, int32_t H, uint64_t overflowSlot)
+{
+    InitLargeLds &l = *reinterpret_cast<InitLargeLds *>(smem);
+    const int32_t tid = threadIdx.x;
+    constexpr int32_t NT = kInitThreads;
+    const int32_t zeroEnd = H < kInitTailEnd ? H : kInitTailEnd;  // the helpers clear the rest
+    auto clear_cells = [&]() {
+        for (int32_t i = tid; i < kInitHomes / 8; i += NT) reinterpret_cast<uint4 *>(l.cells)[i] = make_uint4(0, 0, 0, 0);
+    };
+    auto clear_table = [&]() {
+        for (int32_t i = tid; i < zeroEnd / 8; i += NT) reinterpret_cast<GChunk *>(gHt)[i] = Chunk{0u, 0u, 0u, 0u};
+    };
+    clear_cells();
+    l.spill[tid] = 0ull;
+    if (tid == 0) l.inOrder = l.stop = 0;
+    __syncthreads();
+    if constexpr (!kIdentity) {
+        // repeated and out-of-range tokens
+        bool inOrder = false;
+        for (int32_t s0 = tid; s0 < dbs; s0 += kInitUnroll * NT) {
+            int32_t t[kInitUnroll];
+#pragma unroll
+            for (int q = 0; q < kInitUnroll; ++q) t[q] = s0 + q * NT < dbs ? token(s0 + q * NT) : -1;
+#pragma unroll
+            for (int q = 0; q < kInitUnroll; ++q) {
+                if (t[q] < 0) continue;
+                if (t[q] >= kWaveInitTokenBits) {
+                    inOrder = true;
+                    continue;
+                }
+                const uint32_t bit = 1u << (t[q] & 31);
+                if (atomicOr(l.cells + (t[q] >> 5), bit) & bit) inOrder = true;
+            }
+        }
+        if (__syncthreads_or(inOrder ? 1 : 0)) {
+            clear_table();
+            __threadfence_block();
+            __syncthreads();
+            if (tid == 0) {
+                Guard g;
+                const int32_t *tok = (const int32_t *)token.tok;
+                for (int32_t s = 0; s < dbs && g.code == 0; ++s) {
+                    const int32_t t = tok[s];
+                    if (t >= 0) ht_insert((uint16_t *)gHt, tok, padded, t, s, H - 1, g);
+                }
+                report_overflow(overflowSlot, g.code);
+            }
+            return;
+        }
+        clear_cells();
+        __syncthreads();
+    }
+    const bool wraps = H == kInitHomes;
+    // the first cell at or after c that no earlier pass took, or kInitHomes
+    auto next_free = [&](uint32_t c) -> uint32_t {
+        uint32_t w = c >> 6;
+        if (w >= static_cast<uint32_t>(kInitWords)) return kInitHomes;
+        const uint64_t x = ~l.occ[w] & (~0ull << (c & 63u));
+        if (x) return (w << 6) + static_cast<uint32_t>(__builtin_ctzll(x));
+        for (++w; w < static_cast<uint32_t>(kInitWords); w = (w | 63u) + 1u) {
+            const uint64_t f = ~l.full[w >> 6] & (~0ull << (w & 63u));
+            if (f) {
+                w = (w & ~63u) + static_cast<uint32_t>(__builtin_ctzll(f));
+                return (w << 6) + static_cast<uint32_t>(__builtin_ctzll(~l.occ[w]));
+            }
+        }
+        return kInitHomes;
+    };
+    for (int32_t done = 0; done < dbs;) {
+        const int32_t half = (kInitHomes - done) / 2;
+        const int32_t end = min(dbs, done + (half > NT ? half : NT));
+        const bool later = done > 0;
+        for (int32_t s0 = done + tid; s0 < end; s0 += kInitUnroll * NT) {
+            int32_t t[kInitUnroll];
+#pragma unroll
+            for (int q = 0; q < kInitUnroll; ++q) t[q] = s0 + q * NT < end ? token(s0 + q * NT) : -1;
+#pragma unroll
+            for (int q = 0; q < kInitUnroll; ++q) {
+                if (t[q] < 0) continue;
+                uint32_t v = static_cast<uint32_t>(s0 + q * NT) + 1u;
+                uint32_t c = ht_hash(t[q]);  // 16 bits: the home
+                for (int32_t hops = 0;; ++hops) {
+                    if (later) c = next_free(c);
+                    if (c >= static_cast<uint32_t>(kInitHomes)) {
+                        if (!wraps) {
+                            atomicOr(reinterpret_cast<unsigned long long *>(l.spill) + ((v - 1u) >> 6), 1ull << ((v - 1u) & 63u));
+                            break;
+                        }
+                        c = 0u;  // (fewer keys than cells: one is free)
+                        continue;
+                    }
+                    v = propose16(l.cells, c, v);
+                    if (v == 0u) break;
+                    ++c;
+                    if (hops >= kInitMaxHops) {
+                        l.stop = 1;
+                        break;
+                    }
+                }
+            }
+            if (*const_cast<volatile int32_t *>(&l.stop)) break;
+        }
+        __syncthreads();
+        if (l.stop) {
+            clear_table();
+            __threadfence_block();
+            __syncthreads();
+            if (tid < 64) init_table_sweep<kIdentity>(smem, token, gHt, dbs, H, overflowSlot);
+            return;
+        }
+        done = end;
+        if (done < dbs) {
+            uint8_t *occ8 = reinterpret_cast<uint8_t *>(l.occ);
+            for (int32_t i = tid; i < kInitHomes / 8; i += NT) {
+                const uint4 v = reinterpret_cast<const uint4 *>(l.cells)[i];
+                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+                uint32_t m = 0u;
+#pragma unroll
+                for (int h = 0; h < 4; ++h) {
+                    m |= ((w[h] & 0xFFFFu) != 0u ? 1u : 0u) << (2 * h);
+                    m |= ((w[h] >> 16) != 0u ? 1u : 0u) << (2 * h + 1);
+                }
+                occ8[i] = static_cast<uint8_t>(m);
+            }
+            __syncthreads();
+            const uint64_t fm = __ballot(l.occ[tid] == ~0ull);
+            if ((tid & 63) == 0) l.full[tid >> 6] = fm;
+            __syncthreads();
+        }
+    }
+    for (int32_t i = tid; i < kInitHomes / 8; i += NT) {
+        const uint4 v = reinterpret_cast<const uint4 *>(l.cells)[i];
+        reinterpret_cast<GChunk *>(gHt)[i] = Chunk{v.x, v.y, v.z, v.w};
+    }
+    if (wraps) return;
+    // the spilled slots in increasing order from cell 65536 on
+    uint64_t sp = l.spill[tid];
+    uint32_t inc = static_cast<uint32_t>(__builtin_popcountll(sp));
+    const uint32_t mine = inc, lane = static_cast<uint32_t>(__lane_id());
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = static_cast<uint32_t>(__shfl_up(static_cast<int>(inc), d));
+        if (lane >= static_cast<uint32_t>(d)) inc += o;
+    }
+    if (lane == 63u) l.part[tid >> 6] = inc;
+    __syncthreads();
+    uint32_t before = 0, total = 0;
+    for (int w = 0; w < NT / 64; ++w) {
+        if (w < (tid >> 6)) before += l.part[w];
+        total += l.part[w];
+    }
+    uint32_t at = kInitHomes + before + inc - mine;
+    for (; sp != 0ull; sp &= sp - 1ull) {
+        gHt[at++] = static_cast<uint16_t>((static_cast<uint32_t>(tid) << 6) + static_cast<uint32_t>(__builtin_ctzll(sp)) + 1u);
+    }
+    // the empty cells after them: the cells up to the next chunk one by one
+    const uint32_t end = kInitHomes + total, chunk0 = (end + 7u) / 8u;
+    if (static_cast<uint32_t>(tid) < chunk0 * 8u - end) gHt[end + static_cast<uint32_t>(tid)] = 0;
+    for (uint32_t i = chunk0 + static_cast<uint32_t>(tid); i < static_cast<uint32_t>(zeroEnd) / 8u; i += NT) {
+        reinterpret_cast<GChunk *>(gHt)[i] = Chunk{0u, 0u, 0u, 0u};
+    }
+}
+
+// kLarge: the form for tables beyond kInitLdsCells; workgroup y > 0 of a row
+// clears its share of the cells that no key reaches.
+template <bool kLarge>
+__global__ __launch_bounds__(kInitThreads) void kvx_sieve_ht_init_par(KvxLaunch<HispSieveHtInitArgs> L)
+{
+    extern __shared__ __align__(16) uint8_t smem[];
+    const HispSieveHtInitArgs &a = L.a;
+    const int32_t numReqs = static_cast<int32_t>(a.numReqs);
+    const int32_t poolSize = static_cast<int32_t>(a.poolSize);
+    const int32_t padded = static_cast<int32_t>(a.paddedBufferSize);
+    const int32_t H = static_cast<int32_t>(a.htSize);
+    const int32_t b = blockIdx.x;  // the grid is exactly layerNum * numReqs
+    const int32_t layer = b / numReqs;
+    const int64_t reqIdx = static_cast<int64_t>(a.reqStart) + b % numReqs;
+    if (reqIdx < 0 || reqIdx >= poolSize) return;
+    const int64_t row = static_cast<int64_t>(layer) * poolSize + reqIdx;
+    const RowTokens<false> token{reinterpret_cast<GTok *>(a.deviceBufferTokens) + row * padded, 0};
+    GCell *gHt = reinterpret_cast<GCell *>(a.deviceBufferHt) + row * H;
+    if constexpr (kLarge) {
+        if (blockIdx.y != 0) {
+            for (int32_t i = kInitTailEnd / 8 + (static_cast<int32_t>(blockIdx.y) - 1) * kInitThreads + threadIdx.x; i < H / 8;
+                 i += kInitHelpers * kInitThreads) {
+                reinterpret_cast<GChunk *>(gHt)[i] = Chunk{0u, 0u, 0u, 0u};
+            }
+            return;
+        }
+        init_table_large<false>(smem, token, gHt, padded, static_cast<int32_t>(a.deviceBufferSize), H, L.overflowSlot);
+    } else {
+        init_table_lds<false>(smem, token, gHt, static_cast<int32_t>(a.deviceBufferSize), H);
+    }
 }
 
 }  // namespace
@@ -642,10 +764,10 @@ hipError_t sieve_set_lds_limit(size_t bytes)
     e = hipFuncSetAttribute(reinterpret_cast<const void *>(&kvx_sieve_ht_init<true>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
     if (e != hipSuccess) return e;
-    e = hipFuncSetAttribute(reinterpret_cast<const void *>(&kvx_sieve_ht_init_par),
+    e = hipFuncSetAttribute(reinterpret_cast<const void *>(&kvx_sieve_ht_init_par<false>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
     if (e != hipSuccess) return e;
-    return hipFuncSetAttribute(reinterpret_cast<const void *>(&kvx_sieve_ht_init_wave),
+    return hipFuncSetAttribute(reinterpret_cast<const void *>(&kvx_sieve_ht_init_par<true>),
                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
 }
 
@@ -662,19 +784,19 @@ hipError_t launch_sieve_update(const HispSieveUpdateArgs &a, uint64_t overflowSl
     return hipGetLastError();
 }
 
-size_t sieve_ht_init_par_lds(uint32_t htSize, uint32_t dbs)
+size_t sieve_ht_init_small_lds(uint32_t htSize, uint32_t dbs)
 {
-    if (htSize < 1024u || dbs >= htSize) return 0;  // 4+ cells per lane; fewer keys than cells
-    return static_cast<size_t>(htSize) * 4u + static_cast<size_t>((dbs + 7u) & ~7u) * 2u + htSize / 8u +
-           (2u * kInitThreads + 4u) * 4u;
+    // fewer keys than cells, or a chain of proposals would not end
+    if (htSize < 1024u || htSize > static_cast<uint32_t>(kInitLdsCells) || dbs >= htSize) return 0;
+    return static_cast<size_t>(htSize) * 4u + (dbs + 31u) / 32u * 4u;
 }
 
-size_t sieve_ht_init_wave_lds(uint32_t htSize, uint32_t dbs)
+size_t sieve_ht_init_large_lds(uint32_t htSize, uint32_t dbs)
 {
-    if (htSize < 65536u || htSize > (1u << 20) || (htSize & (htSize - 1u)) != 0 || dbs >= htSize) return 0;
-    const size_t cells = htSize / 8u + htSize / 512u + 8u * ((htSize + 262143u) / 262144u);
-    const size_t tokens = kWaveInitTokenBits / 8u;
-    return cells > tokens ? cells : tokens;
+    // slots below 65535: an entry is 16 bits
+    if (htSize < static_cast<uint32_t>(kInitHomes) || htSize > (1u << 20) || dbs > 65535u) return 0;
+    const size_t sweep = htSize / 8u + htSize / 512u + 8u * ((htSize + 262143u) / 262144u);
+    return sweep > sizeof(InitLargeLds) ? sweep : sizeof(InitLargeLds);
 }
 
 hipError_t launch_sieve_ht_init(const HispSieveHtInitArgs &a, uint64_t overflowSlot, size_t ldsBytes,
@@ -682,10 +804,12 @@ hipError_t launch_sieve_ht_init(const HispSieveHtInitArgs &a, uint64_t overflowS
 {
     KvxLaunch<HispSieveHtInitArgs> L{a, overflowSlot};
     const dim3 grid(a.layerNum * a.numReqs), block(256);
-    if (form == InitForm::kParallel) {
-        hipLaunchKernelGGL(kvx_sieve_ht_init_par, grid, dim3(kInitThreads), ldsBytes, stream, L);
-    } else if (form == InitForm::kWave) {
-        hipLaunchKernelGGL(kvx_sieve_ht_init_wave, grid, dim3(kInitThreads), ldsBytes, stream, L);
+    if (form == InitForm::kSmall) {
+        const uint32_t threads = a.deviceBufferSize <= static_cast<uint32_t>(kInitSmallSlots) ? kInitSmallThreads : kInitThreads;
+        hipLaunchKernelGGL(kvx_sieve_ht_init_par<false>, grid, dim3(threads), ldsBytes, stream, L);
+    } else if (form == InitForm::kLarge) {
+        const uint32_t parts = a.htSize > static_cast<uint32_t>(kInitTailEnd) ? 1u + kInitHelpers : 1u;
+        hipLaunchKernelGGL(kvx_sieve_ht_init_par<true>, dim3(grid.x, parts), dim3(kInitThreads), ldsBytes, stream, L);
     } else if (ldsBytes != 0) {
         hipLaunchKernelGGL(kvx_sieve_ht_init<true>, grid, block, ldsBytes, stream, L);
     } else {

@@ -151,6 +151,35 @@ def test_ht_init_wave_parity(kvops, dbs, top_k, mode):
     assert kvops.read_overflow() == 0
 
 
+@pytest.mark.parametrize("homes", ["first", "last"])
+@pytest.mark.parametrize("dbs,top_k", [(16000, 2048), (32000, 2048), (65518, 8192)])
+def test_ht_init_packed_homes(kvops, dbs, top_k, homes):
+    """Large tables whose keys are homed in 64 cells: the first ones (chains of
+    proposals past the parallel build's limit, so the one-wave sweep) or the
+    last of the 65536 homes (keys that run past them: cells from 65536 on, or
+    around the end of a 65536-cell table)."""
+    import torch
+
+    rng = np.random.default_rng(dbs + len(homes))
+    st = orc.SieveState(1, 2, dbs, top_k)
+    t = np.arange(0, 1 << 20, dtype=np.int64)
+    h = _home(t, 65536)
+    cand = t[h < 64] if homes == "first" else t[h >= 65536 - 64]
+    st.tokens[:] = -1
+    for r in range(2):
+        vals = rng.permutation(cand)[:900]
+        st.tokens[0, r, rng.choice(dbs, size=len(vals), replace=False)] = vals
+    dev = DevSieve(st)
+    dev.ht.fill_(77)
+    st.ht[:] = 77
+    orc.sieve_ht_init(st.tokens, st.ht, 0, 2, 1, 2, dbs, st.padded, st.ht_size)
+    kvops.sieve_ht_init(dev.tokens.data_ptr(), dev.ht.data_ptr(), dev.prefill.data_ptr(), 0, 2, 1, 2, dbs, st.padded,
+                        st.ht_size, 0, 0)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(dev.ht.cpu().numpy().view(np.uint16), st.ht)
+    assert kvops.read_overflow() == 0
+
+
 def test_ht_init_small_table_parity(kvops):
     """A 512-cell table (under the parallel form's 1024): the one-lane build."""
     import torch

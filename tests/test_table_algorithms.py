@@ -7,13 +7,15 @@
   also the table of inserting the survivors in their insertion order; and so
   does the kernel's windowed form of the pass (events found one at a time,
   holes in a few queue lanes or a set, a window's writes after it).
-* Parallel admission build (kvx_sieve_ht_init_par, csrc/sieve.hip): keys
-  bucketed by home with later duplicates dropped, the used cells from the
-  backlog recursion (the ring's fixed point entering cell 0), then each
-  cluster's keys in slot order; equal to the oracle's sequential inserts
-  (hisp_sieve_ht_init.cpp:14-60).
-
-* Batched admission build for tables larger than LDS (kvx_sieve_ht_init_wave,
+* Parallel admission build (kvx_sieve_ht_init_par, csrc/sieve.hip): every slot
+  proposes to the cells from its home on, a cell keeps the smallest slot, in
+  any order of the proposals; slots whose token an earlier slot holds are found
+  on the walk from their home and left out of a second build.  Equal to the
+  oracle's sequential inserts (hisp_sieve_ht_init.cpp:14-60).
+* Parallel build by clusters: keys bucketed by home with later duplicates
+  dropped, the used cells from the backlog recursion (the ring's fixed point
+  entering cell 0), then each cluster's keys in slot order; the same table.
+* Batched build (the one-wave sweep of kvx_sieve_ht_init_par's large form,
   csrc/sieve.hip): with distinct tokens, 64 keys at a time; keys whose
   backlog is zero take their own first free cell at once, the rest sweep the
   free cells in increasing order, earliest slot first; a batch whose probes
@@ -284,6 +286,59 @@ def test_parallel_table_build_equals_sequential_inserts(mode):
         want = np.zeros((1, 1, H), dtype=np.uint16)
         orc.sieve_ht_init(tok.reshape(1, 1, padded).copy(), want, 0, 1, 1, 1, dbs, padded, H)
         np.testing.assert_array_equal(_parallel_build(tok, dbs, H), want[0, 0], err_msg="{} {}".format(mode, trial))
+
+
+def _proposal_build(tok, dbs, H, rng):
+    """Deferred acceptance with the proposals in a random order."""
+    mask = H - 1
+    live = [s for s in range(dbs) if tok[s] >= 0]
+    for _ in range(2):
+        cell = [None] * H
+        wait = [(s, _knuth_home(int(tok[s]), H)) for s in live]
+        while wait:
+            s, c = wait.pop(int(rng.integers(0, len(wait))))
+            if cell[c] is None:
+                cell[c] = s
+            else:
+                keep, go = min(cell[c], s), max(cell[c], s)
+                cell[c] = keep
+                wait.append((go, (c + 1) & mask))
+        again = set()
+        for s in live:
+            c = _knuth_home(int(tok[s]), H)
+            while cell[c] != s:
+                if tok[cell[c]] == tok[s]:
+                    again.add(s)
+                    break
+                c = (c + 1) & mask
+        if not again:
+            break
+        live = [s for s in live if s not in again]
+    return np.array([0 if s is None else s + 1 for s in cell], dtype=np.uint16)
+
+
+@pytest.mark.parametrize("mode", ["unique", "dups", "few_homes", "wrap"])
+def test_proposal_build_equals_sequential_inserts(mode):
+    rng = np.random.default_rng(40 + len(mode))
+    for trial in range(6):
+        dbs = int(rng.choice([1, 64, 300, 500]))
+        padded = (dbs + 15) // 16 * 16
+        H = orc.ht_size(padded, 8)
+        tok = np.full(padded, -1, dtype=np.int32)
+        n = int(rng.integers(0, dbs + 1))
+        if mode == "unique":
+            vals = rng.choice(1 << 22, size=n, replace=False)
+        elif mode == "dups":
+            vals = rng.integers(-3, max(4, n // 3), size=n)
+        else:
+            t = np.arange(0, 1 << 20, dtype=np.int64)
+            h = ((t * 2654435761) & 0xFFFFFFFF) >> 16 & (H - 1)
+            cand = t[np.isin(h, rng.choice(H, size=4, replace=False))] if mode == "few_homes" else t[h >= H - 24]
+            vals = rng.choice(cand, size=min(n, len(cand)), replace=False)
+        tok[rng.choice(dbs, size=len(vals), replace=False)] = vals
+        want = np.zeros((1, 1, H), dtype=np.uint16)
+        orc.sieve_ht_init(tok.reshape(1, 1, padded).copy(), want, 0, 1, 1, 1, dbs, padded, H)
+        np.testing.assert_array_equal(_proposal_build(tok, dbs, H, rng), want[0, 0], err_msg="{} {}".format(mode, trial))
 
 
 def _batch_sweep_build(tok, dbs, H, batch=64, cap=4):
