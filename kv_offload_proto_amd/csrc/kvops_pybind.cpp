@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "kvx/kvx.h"
+#include "kvx_admit.h"
 
 namespace py = pybind11;
 
@@ -196,6 +197,23 @@ PYBIND11_MODULE(_kvops, m)
             return addr;
         },
         py::arg("nbytes"), py::arg("coherent") = false);
+    m.def(
+        "admit_request",
+        [](uint64_t device_buffer_tokens, uint64_t device_buffer_visited, uint64_t device_buffer_ht,
+           uint64_t sieve_hand, uint64_t prefill_lens, uint64_t req_host_base, uint32_t req_batch_idx,
+           uint32_t req_pool_idx, int32_t prefill_len, int64_t host_base_row, uint32_t layer_num, uint32_t pool_size,
+           uint32_t device_buffer_size, uint32_t padded_buffer_size, uint32_t visited_stride_b, uint32_t ht_size,
+           uint64_t stream) {
+            Check(kvx_admit_request(device_buffer_tokens, device_buffer_visited, device_buffer_ht, sieve_hand,
+                                    prefill_lens, req_host_base, req_batch_idx, req_pool_idx, prefill_len,
+                                    host_base_row, layer_num, pool_size, device_buffer_size, padded_buffer_size,
+                                    visited_stride_b, ht_size, stream));
+        },
+        py::arg("device_buffer_tokens"), py::arg("device_buffer_visited"), py::arg("device_buffer_ht"),
+        py::arg("sieve_hand"), py::arg("prefill_lens"), py::arg("req_host_base"), py::arg("req_batch_idx"),
+        py::arg("req_pool_idx"), py::arg("prefill_len"), py::arg("host_base_row"), py::arg("layer_num"),
+        py::arg("pool_size"), py::arg("device_buffer_size"), py::arg("padded_buffer_size"),
+        py::arg("visited_stride_b"), py::arg("ht_size"), py::arg("stream") = 0);
     m.def("host_free", [](uint64_t addr) { Check(kvx_host_free(addr)); }, py::arg("addr"));
     m.def(
         "host_alloc_node",

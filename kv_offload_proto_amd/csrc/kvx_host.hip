@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "kvx/kvx.h"
+#include "kvx_admit.h"
 #include "kvx_internal.h"
 
 namespace {
@@ -1001,6 +1002,58 @@ int kvx_sieve_ht_init(uint64_t device_buffer_tokens, uint64_t device_buffer_ht, 
         }
         hipCheck(kvx::launch_sieve_ht_init(a, reinterpret_cast<uint64_t>(g.overflow), lds, AsStream(stream), form),
                  "hisp_sieve_ht_init launch");
+    });
+}
+
+int kvx_admit_request(uint64_t device_buffer_tokens, uint64_t device_buffer_visited, uint64_t device_buffer_ht,
+                      uint64_t sieve_hand, uint64_t prefill_lens, uint64_t req_host_base, uint32_t req_batch_idx,
+                      uint32_t req_pool_idx, int32_t prefill_len, int64_t host_base_row, uint32_t layer_num,
+                      uint32_t pool_size, uint32_t device_buffer_size, uint32_t padded_buffer_size,
+                      uint32_t visited_stride_b, uint32_t ht_size, uint64_t stream)
+{
+    return Guarded([&] {
+        EnsureInited();
+        if (ht_size < 1024 || (ht_size & (ht_size - 1)) != 0 || ht_size > (1u << 20)) {
+            throw Error("admit_request: ht_size must be a power of two in [1024, 2^20]");
+        }
+        if (padded_buffer_size % 16 != 0 || padded_buffer_size > 65535 || device_buffer_size > padded_buffer_size ||
+            padded_buffer_size >= ht_size) {
+            throw Error("admit_request: padded_buffer_size must be a multiple of 16 below 65536 and ht_size, and cover "
+                        "device_buffer_size");
+        }
+        if (visited_stride_b % 64 != 0 || visited_stride_b < (padded_buffer_size + 7) / 8) {
+            throw Error("admit_request: visited bitmap stride must be 64B aligned and cover padded");
+        }
+        if (prefill_len < 0) throw Error("admit_request: prefill_len must not be negative");
+        if (req_pool_idx >= pool_size) throw Error("admit_request: req_pool_idx out of range");
+        CheckAligned16(device_buffer_tokens, "admit_request: device_buffer_tokens");
+        CheckAligned16(device_buffer_visited, "admit_request: device_buffer_visited");
+        CheckAligned16(device_buffer_ht, "admit_request: device_buffer_ht");
+        CheckAligned16(sieve_hand, "admit_request: sieve_hand");
+        kvx::AdmitArgs a{};
+        a.deviceBufferTokens = device_buffer_tokens;
+        a.deviceBufferVisited = device_buffer_visited;
+        a.deviceBufferHt = device_buffer_ht;
+        a.sieveHand = sieve_hand;
+        a.prefillLens = prefill_lens;
+        a.reqHostBase = req_host_base;
+        a.hostBaseRow = host_base_row;
+        a.poolSize = pool_size;
+        a.paddedBufferSize = padded_buffer_size;
+        a.visitedStrideB = visited_stride_b;
+        a.htSize = ht_size;
+        a.reqPoolIdx = req_pool_idx;
+        a.reqBatchIdx = req_batch_idx;
+        a.prefillLen = prefill_len;
+        a.liveSlots = static_cast<int32_t>(std::min<int64_t>(prefill_len, device_buffer_size));
+        if (layer_num == 0) return;
+        const size_t ldsSmall = kvx::sieve_ht_init_small_lds(ht_size, device_buffer_size);
+        const size_t ldsLarge = kvx::sieve_ht_init_large_lds(ht_size, device_buffer_size);
+        const bool large = ldsSmall == 0;
+        const size_t lds = large ? ldsLarge : ldsSmall;
+        if (lds == 0 || lds > g.ldsLimit) throw Error("admit_request: table too large for the device's LDS");
+        hipCheck(kvx::launch_admit(a, layer_num, reinterpret_cast<uint64_t>(g.overflow), lds, large, AsStream(stream)),
+                 "admit_request launch");
     });
 }
 

@@ -327,6 +327,19 @@ hipError_t launch_sieve_update(const HispSieveUpdateArgs &a, uint64_t overflowSl
 enum class InitForm { kSmall, kLarge, kInOrder };
 hipError_t launch_sieve_ht_init(const HispSieveHtInitArgs &a, uint64_t overflowSlot, size_t ldsBytes,
                                 hipStream_t stream, InitForm form);
+// One request's admission in every layer (state tensors as sieve_update takes
+// them, base addresses of layer 0); forms and LDS sizes as above, by the slots
+// in use.
+struct AdmitArgs {
+    uint64_t deviceBufferTokens, deviceBufferVisited, deviceBufferHt, sieveHand, prefillLens, reqHostBase;
+    int64_t hostBaseRow;
+    uint32_t poolSize, paddedBufferSize, visitedStrideB, htSize;
+    uint32_t reqPoolIdx, reqBatchIdx;
+    int32_t prefillLen;
+    int32_t liveSlots;  // min(prefill, device buffer slots)
+};
+hipError_t launch_admit(const AdmitArgs &a, uint32_t layers, uint64_t overflowSlot, size_t ldsBytes, bool large,
+                        hipStream_t stream);
 size_t sieve_ht_init_small_lds(uint32_t htSize, uint32_t dbs);
 size_t sieve_ht_init_large_lds(uint32_t htSize, uint32_t dbs);
 hipError_t sieve_set_lds_limit(size_t bytes);

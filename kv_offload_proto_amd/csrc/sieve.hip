@@ -754,6 +754,49 @@ __global__ __launch_bounds__(kInitThreads) void kvx_sieve_ht_init_par(KvxLaunch<
     }
 }
 
+// One request's state in every layer at admission, in one launch: slot s holds
+// token s for s < n0 and none past it, the visited bits and the hand records
+// cleared, the tables of those tokens, the request's lengths.  Workgroup x is
+// layer x; in the large form workgroup y > 0 writes a share of everything but
+// the cells below kInitTailEnd, which workgroup 0 builds meanwhile.  The
+// tokens need not be read back: their slots are their numbers.  (As eight
+// launches -- fills, a range, two copies of a scalar from the host, the table
+// build -- an admission was bound by their submission, ~45 us of it.)
+template <bool kLarge>
+__global__ __launch_bounds__(kInitThreads) void kvx_admit(AdmitArgs a, uint64_t overflowSlot)
+{
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int32_t padded = static_cast<int32_t>(a.paddedBufferSize), H = static_cast<int32_t>(a.htSize);
+    const int32_t tid = threadIdx.x, n0 = a.liveSlots;
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * a.poolSize + a.reqPoolIdx;
+    GCell *gHt = reinterpret_cast<GCell *>(a.deviceBufferHt) + row * H;
+    if (!kLarge || blockIdx.y != 0) {
+        const int32_t parts = kLarge ? kInitHelpers : 1, part = kLarge ? static_cast<int32_t>(blockIdx.y) - 1 : 0;
+        const int32_t step = parts * static_cast<int32_t>(blockDim.x), first = part * static_cast<int32_t>(blockDim.x) + tid;
+        GChunk *tok4 = reinterpret_cast<GChunk *>(a.deviceBufferTokens + static_cast<uint64_t>(row) * padded * 4u);
+        for (int32_t i = first; i < padded / 4; i += step) {
+            auto at = [&](int32_t s) { return static_cast<uint32_t>(s < n0 ? s : -1); };
+            tok4[i] = Chunk{at(4 * i), at(4 * i + 1), at(4 * i + 2), at(4 * i + 3)};
+        }
+        GChunk *vis4 = reinterpret_cast<GChunk *>(a.deviceBufferVisited + static_cast<uint64_t>(row) * a.visitedStrideB);
+        for (int32_t i = first; i < static_cast<int32_t>(a.visitedStrideB) / 16; i += step) vis4[i] = Chunk{0u, 0u, 0u, 0u};
+        if (part == 0 && tid < kHandStride / 4) {
+            reinterpret_cast<GChunk *>(a.sieveHand + static_cast<uint64_t>(row) * kHandStride * 4u)[tid] = Chunk{0u, 0u, 0u, 0u};
+        }
+        if (blockIdx.x == 0 && part == 0 && tid == 0) {
+            reinterpret_cast<__attribute__((address_space(1))) int32_t *>(a.prefillLens)[a.reqPoolIdx] = a.prefillLen;
+            reinterpret_cast<__attribute__((address_space(1))) int64_t *>(a.reqHostBase)[a.reqBatchIdx] = a.hostBaseRow;
+        }
+        if constexpr (kLarge) {
+            for (int32_t i = kInitTailEnd / 8 + first; i < H / 8; i += step) reinterpret_cast<GChunk *>(gHt)[i] = Chunk{0u, 0u, 0u, 0u};
+            return;
+        }
+    }
+    const RowTokens<true> token{nullptr, n0};
+    if constexpr (kLarge) init_table_large<true>(smem, token, gHt, padded, n0, H, overflowSlot);
+    else init_table_lds<true>(smem, token, gHt, n0, H);
+}
+
 }  // namespace
 
 hipError_t sieve_set_lds_limit(size_t bytes)
@@ -767,8 +810,12 @@ hipError_t sieve_set_lds_limit(size_t bytes)
     e = hipFuncSetAttribute(reinterpret_cast<const void *>(&kvx_sieve_ht_init_par<false>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
     if (e != hipSuccess) return e;
-    return hipFuncSetAttribute(reinterpret_cast<const void *>(&kvx_sieve_ht_init_par<true>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+    for (const void *f : {reinterpret_cast<const void *>(&kvx_sieve_ht_init_par<true>),
+                          reinterpret_cast<const void *>(&kvx_admit<false>), reinterpret_cast<const void *>(&kvx_admit<true>)}) {
+        e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_sieve_update(const HispSieveUpdateArgs &a, uint64_t overflowSlot, int variant, size_t ldsBytes,
@@ -797,6 +844,18 @@ size_t sieve_ht_init_large_lds(uint32_t htSize, uint32_t dbs)
     if (htSize < static_cast<uint32_t>(kInitHomes) || htSize > (1u << 20) || dbs > 65535u) return 0;
     const size_t sweep = htSize / 8u + htSize / 512u + 8u * ((htSize + 262143u) / 262144u);
     return sweep > sizeof(InitLargeLds) ? sweep : sizeof(InitLargeLds);
+}
+
+hipError_t launch_admit(const AdmitArgs &a, uint32_t layers, uint64_t overflowSlot, size_t ldsBytes, bool large,
+                        hipStream_t stream)
+{
+    if (large) {
+        hipLaunchKernelGGL(kvx_admit<true>, dim3(layers, 1u + kInitHelpers), dim3(kInitThreads), ldsBytes, stream, a, overflowSlot);
+    } else {
+        const uint32_t threads = a.paddedBufferSize <= static_cast<uint32_t>(kInitSmallSlots) ? kInitSmallThreads : kInitThreads;
+        hipLaunchKernelGGL(kvx_admit<false>, dim3(layers), dim3(threads), ldsBytes, stream, a, overflowSlot);
+    }
+    return hipGetLastError();
 }
 
 hipError_t launch_sieve_ht_init(const HispSieveHtInitArgs &a, uint64_t overflowSlot, size_t ldsBytes,

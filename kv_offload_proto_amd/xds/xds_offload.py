@@ -67,6 +67,15 @@ class XdsOffloadCoordinator:
             raise ValueError("req_pool_idx out of range: {}".format(req_pool_idx))
         if req_batch_idx < 0 or req_batch_idx >= self.max_num_reqs:
             raise ValueError("req_batch_idx out of range: {}".format(req_batch_idx))
+        handle = _stream_handle(stream)
+        if self._one_launch(prefill_len, host_base_row, handle):
+            _kvops.admit_request(self.device_buffer_tokens.data_ptr(), self.device_buffer_visited.data_ptr(),
+                                 self.device_buffer_ht.data_ptr(), self.sieve_hand.data_ptr(),
+                                 self.prefill_lens.data_ptr(), self.req_host_base.data_ptr(), req_batch_idx,
+                                 req_pool_idx, prefill_len, host_base_row, self.layer_num, self.pool_size,
+                                 self.device_buffer_size, self.padded_buffer_size, self.visited_stride_b,
+                                 self.ht_size, handle)
+            return
         init_n = min(prefill_len, self.device_buffer_size)
         row = self.device_buffer_tokens[:, req_pool_idx, :]
         row.fill_(-1)
@@ -77,8 +86,32 @@ class XdsOffloadCoordinator:
         self.req_host_base[req_batch_idx] = host_base_row
         _kvops.sieve_ht_init(self.device_buffer_tokens.data_ptr(), self.device_buffer_ht.data_ptr(),
                              self.prefill_lens.data_ptr(), req_pool_idx, 1, self.layer_num, self.pool_size,
-                             self.device_buffer_size, self.padded_buffer_size, self.ht_size,
-                             _stream_handle(stream), self.layer_num)
+                             self.device_buffer_size, self.padded_buffer_size, self.ht_size, handle, self.layer_num)
+
+    def _one_launch(self, prefill_len, host_base_row, handle: int) -> bool:
+        """Whether the admission can go as one launch on `handle`: plain
+        lengths, state tensors as constructed (a caller may have replaced
+        them), sizes the launch takes, and the stream that the separate calls
+        would use throughout (their tensor writes go to the current one)."""
+        if type(prefill_len) is not int or type(host_base_row) is not int:
+            return False
+        if not (0 <= prefill_len < 1 << 31 and -(1 << 63) <= host_base_row < 1 << 63 and self.device_buffer_size > 0):
+            return False
+        if self.ht_size > 1 << 20 or self.padded_buffer_size > 65535:
+            return False
+        L, p = self.layer_num, self.pool_size
+        for t, shape, dtype in ((self.device_buffer_tokens, (L, p, self.padded_buffer_size), torch.int32),
+                                (self.device_buffer_visited, (L, p, self.visited_stride_b), torch.uint8),
+                                (self.device_buffer_ht, (L, p, self.ht_size), torch.int16),
+                                (self.sieve_hand, (L, p, 16), torch.int32),
+                                (self.prefill_lens, (p,), torch.int32),
+                                (self.req_host_base, (self.max_num_reqs,), torch.int64)):
+            if type(t) is not torch.Tensor or t.dtype is not dtype or t.shape != shape or not t.is_contiguous():
+                return False
+            if not t.is_cuda or t.data_ptr() % 16:
+                return False
+        dev = self.device_buffer_tokens.device
+        return dev.index == torch.cuda.current_device() and handle == torch.cuda.current_stream(dev).cuda_stream
 
     def set_batch(self, req_pool_indices: torch.Tensor, seq_lens: torch.Tensor) -> None:
         """Batch context of the next decode steps (xds_offload.py:79-87)."""

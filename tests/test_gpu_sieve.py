@@ -180,6 +180,45 @@ def test_ht_init_packed_homes(kvops, dbs, top_k, homes):
     assert kvops.read_overflow() == 0
 
 
+@pytest.mark.parametrize("dbs,top_k,prefills", [
+    (1, 16, [0, 1, 5]), (64, 64, [63, 64, 256]), (1000, 333, [1, 999, 3777]), (8192, 2048, [8191, 8192, 16384]),
+    (16370, 8, [16370, 40000]), (16384, 2048, [16383, 131072]), (65518, 8192, [300, 65518, 131072])])
+def test_admit_one_launch(kvops, dbs, top_k, prefills):
+    """admit_request as one launch leaves what the separate calls leave (and
+    those, the oracle): every state tensor, the rows of other requests
+    untouched."""
+    import torch
+
+    from kv_offload_proto_amd.xds import XdsOffloadCoordinator
+
+    layers, pool = 3, 4
+    one = XdsOffloadCoordinator("cuda", layers, pool, dbs, top_k, 3, 1 << 17)
+    two = XdsOffloadCoordinator("cuda", layers, pool, dbs, top_k, 3, 1 << 17)
+    names = ("device_buffer_tokens", "device_buffer_visited", "device_buffer_ht", "sieve_hand", "prefill_lens",
+             "req_host_base")
+    two._one_launch = lambda *a: False
+    st = orc.SieveState(layers, pool, dbs, top_k)
+    for c in (one, two):
+        for n in names:
+            getattr(c, n).fill_(77)
+    rows = [2, 0, 3][:len(prefills)]
+    for i, (r, n) in enumerate(zip(rows, prefills)):
+        assert one._one_launch(n, 7 << 33, torch.cuda.current_stream().cuda_stream)
+        for c in (one, two):
+            c.admit_request(2 - i, r, n, (7 << 33) + i)
+        st.admit(r, n)
+    torch.cuda.synchronize()
+    for n in names:
+        np.testing.assert_array_equal(getattr(one, n).cpu().numpy(), getattr(two, n).cpu().numpy(), err_msg=n)
+    for r in rows:
+        np.testing.assert_array_equal(one.device_buffer_ht[:, r].cpu().numpy().view(np.uint16), st.ht[:, r])
+        np.testing.assert_array_equal(one.device_buffer_tokens[:, r].cpu().numpy(), st.tokens[:, r])
+    side = torch.cuda.Stream()
+    assert not one._one_launch(5, 0, side.cuda_stream)
+    assert not one._one_launch(np.int64(5), 0, torch.cuda.current_stream().cuda_stream)
+    assert kvops.read_overflow() == 0
+
+
 def test_ht_init_small_table_parity(kvops):
     """A 512-cell table (under the parallel form's 1024): the one-lane build."""
     import torch
