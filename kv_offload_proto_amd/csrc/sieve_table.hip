@@ -456,6 +456,102 @@ __device__ __forceinline__ uint32_t select_bit64(uint64_t x, uint32_t r)  // off
     return base;
 }
 
+// Key i of n, in insertion order, takes the first of the cells 0 .. n-1 at or
+// after L.res[i] that no earlier key took (every key finds one): its cell goes
+// to L.sortedH[i].  By halving: the cells that the first half of the keys take
+// do not depend on their order (the backlog of their counts); those cells, in
+// order, and the rest are two problems of half the size, and a key's first
+// candidate in its half is the number of that half's cells before it.  Eight
+// levels of a scan in place of 256 searches one after another on one wave
+// (100k of a chunk's 130k cycles in a long cluster): the launch 315 -> 176 us at
+// 4 rows of 65518 slots in long clusters.  All threads call it; n <= kTblChunkCells,
+// the arrays are padded with keys that each take a cell of their own.
+__device__ __forceinline__ void match_cells(const PlaceLds &L, uint32_t n)
+{
+    constexpr uint32_t NP = kTblChunkCells, NPW = NP / 64u;
+    static_assert(NP <= kTT && (NP & (NP - 1u)) == 0u && NP >= 64u, "one key per thread");
+    __shared__ MP sTot[NPW];
+    __shared__ uint32_t sUsed[NPW];
+    uint32_t *cnt = L.own, *next = L.home, *before = L.ent;  // saved in registers meanwhile
+    const uint32_t tid = threadIdx.x, lane = static_cast<uint32_t>(__lane_id()), wave = tid >> 6;
+    const bool on = tid < NP;
+    uint32_t keepOwn = 0, keepEnt = 0, lo = tid, cell = tid;
+    if (on) {
+        keepOwn = L.own[tid];
+        keepEnt = L.ent[tid];
+        if (tid < n) lo = L.res[tid] < NP ? L.res[tid] : NP - 1u;
+    }
+    __syncthreads();
+    if (on) cnt[tid] = 0u;
+    __syncthreads();
+    for (uint32_t g = NP; g > 1u; g >>= 1) {
+        const uint32_t half = g >> 1, base = tid & ~(g - 1u);
+        const bool first = (tid & half) == 0u;
+        if (on && first) atomicAdd(&cnt[base + lo], 1u);
+        __syncthreads();
+        MP m{kNegInf, 0}, ex{kNegInf, 0};
+        int32_t c = 0;
+        const uint32_t seg = g < 64u ? g : 64u, at = lane & (seg - 1u);
+        if (on) {
+            c = static_cast<int32_t>(cnt[tid]);
+            m = mp_cell(c);
+            for (uint32_t d = 1; d < seg; d <<= 1) {
+                MP o;
+                o.p = __shfl_up(m.p, d);
+                o.q = __shfl_up(m.q, d);
+                if (at >= d) m = mp_then(o, m);
+            }
+            ex.p = __shfl_up(m.p, 1);
+            ex.q = __shfl_up(m.q, 1);
+            if (at == 0u) ex = MP{kNegInf, 0};
+            if (lane == 63u) sTot[wave] = m;
+        }
+        const uint32_t w0 = base >> 6;  // the group's first wave
+        if (g > 64u) {
+            __syncthreads();
+            if (on) {
+                MP run{kNegInf, 0};
+                for (uint32_t w = w0; w < wave; ++w) run = mp_then(run, sTot[w]);
+                ex = mp_then(run, ex);
+            }
+        }
+        const bool used = on && mp_apply(ex, 0) + c >= 1;
+        const uint64_t um = __ballot(used);
+        uint32_t u = 0;  // the group's used cells before this one
+        if (on) {
+            const uint64_t below = um & ((1ull << lane) - 1ull);
+            u = static_cast<uint32_t>(__builtin_popcountll(seg < 64u ? below >> (lane & ~(seg - 1u)) : below));
+            if (lane == 0u) sUsed[wave] = static_cast<uint32_t>(__builtin_popcountll(um));
+        }
+        if (g > 64u) {
+            __syncthreads();
+            if (on) {
+                for (uint32_t w = w0; w < wave; ++w) u += sUsed[w];
+            }
+        }
+        if (on) {
+            const uint32_t to = used ? base + u : base + half + (tid - base - u);
+            next[to & (NP - 1u)] = cell;
+            before[tid] = u;
+        }
+        __syncthreads();
+        if (on) {
+            const uint32_t ub = before[base + lo];
+            lo = first ? ub : lo - ub;
+            lo = lo < half ? lo : half - 1u;  // (always below: each half's cells number its keys)
+            cell = next[tid];
+            cnt[tid] = 0u;
+        }
+        __syncthreads();
+    }
+    if (on) {
+        L.sortedH[tid] = cell;
+        L.own[tid] = keepOwn;
+        L.ent[tid] = keepEnt;
+    }
+    __syncthreads();
+}
+
 // All threads; the items are in L.home/ent/own [0, n).  Returns through L.res
 // the window cell of each item.  False: a key found no cell (not reachable).
 __device__ bool place_chunk(const PlaceLds &L, const uint64_t *win, uint32_t n, MP *sPart, int32_t *sMax)
@@ -542,39 +638,9 @@ __device__ bool place_chunk(const PlaceLds &L, const uint64_t *win, uint32_t n, 
         L.res[tid] = lo;
     }
     __syncthreads();
-    // in insertion order, the first untaken candidate (one wave, 256-bit mask)
-    if (tid < 64) {
-        uint64_t tk0 = 0, tk1 = 0, tk2 = 0, tk3 = 0;
-        uint32_t q4[4], r4[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const uint32_t i = static_cast<uint32_t>(g) * 64u + lane;
-            q4[g] = i < n ? L.res[i] : 0u;
-        }
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const uint32_t lim = n > static_cast<uint32_t>(g) * 64u ? n - static_cast<uint32_t>(g) * 64u : 0u;
-            for (uint32_t l = 0; l < (lim < 64u ? lim : 64u); ++l) {
-                const uint32_t q = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(q4[g]), static_cast<int>(l)));
-                const uint32_t wq = q >> 6;
-                const uint64_t m0 = wq == 0u ? (~tk0 & (~0ull << (q & 63u))) : 0ull;
-                const uint64_t m1 = wq <= 1u ? (~tk1 & (wq == 1u ? (~0ull << (q & 63u)) : ~0ull)) : 0ull;
-                const uint64_t m2 = wq <= 2u ? (~tk2 & (wq == 2u ? (~0ull << (q & 63u)) : ~0ull)) : 0ull;
-                const uint64_t m3 = ~tk3 & (wq == 3u ? (~0ull << (q & 63u)) : ~0ull);
-                uint32_t idx;
-                if (m0) { idx = static_cast<uint32_t>(__builtin_ctzll(m0)); tk0 |= 1ull << idx; }
-                else if (m1) { idx = 64u + static_cast<uint32_t>(__builtin_ctzll(m1)); tk1 |= 1ull << (idx - 64u); }
-                else if (m2) { idx = 128u + static_cast<uint32_t>(__builtin_ctzll(m2)); tk2 |= 1ull << (idx - 128u); }
-                else { idx = 192u + static_cast<uint32_t>(__builtin_ctzll(m3)); tk3 |= 1ull << (idx - 192u); }
-                if (lane == l) r4[g] = idx;
-            }
-        }
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const uint32_t i = static_cast<uint32_t>(g) * 64u + lane;
-            if (i < n) L.res[i] = L.z[r4[g]];
-        }
-    }
+    // in insertion order, the first untaken candidate
+    match_cells(L, n);
+    if (tid < n) L.res[tid] = L.z[L.sortedH[tid]];
     __syncthreads();
     return true;
 }
