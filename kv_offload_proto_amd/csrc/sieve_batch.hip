@@ -18,12 +18,12 @@
 //     row whose consistency flag (sieve_hand[row][1]) is set, which this
 //     kernel and the LDS kernel set when they leave the row consistent, only
 //     has its live tokens and entries counted, and its tokens' fingerprint
-//     compared with the one written with the flag (sieve_hand[row][3]);
+//     compared with the one written with the flag (sieve_hand[row][3]): a
+//     difference sends it to the full check or the in-order recurrence;
 //  2. decide: each position's first occurrence in the batch and the initial
-//     slot of its token are found in parallel first (for a flagged row whose
-//     tokens lie below the table size the pre-passes mark the step's tokens
-//     in a bitmap and find their slots in one pass over the slots instead of
-//     a token map); up to the first miss every position is a hit, applied in
+//     slot of its token are found in parallel first (for a flagged row
+//     the pre-passes mark the step's tokens in a bitmap and find their slots
+//     in one pass over the slots instead of a token map); up to the first miss every position is a hit, applied in
 //     parallel; a step whose hand does not come back to where it started is
 //     then decided in parallel (decide_parallel); otherwise one wave decides
 //     in order, from LDS only: a token is resident at the slot it was last
@@ -186,16 +186,15 @@ __device__ __forceinline__ bool batch_row_head(const HispSieveUpdateArgs &a, int
 }
 
 // Second level: the request's flag and prefill length.  True when the batch
-// kernel takes the row in its bitmap form (flagged, tokens below the table size).
+// kernel takes the row in its bitmap form (flagged).
 __device__ __forceinline__ bool batch_row_bitmap(const HispSieveUpdateArgs &a, int64_t reqIdx, int32_t &prefill,
-                                                 uint32_t mapCap)
+                                                 int32_t &mapLim, uint32_t mapCap)
 {
     const int32_t flag = ((KVX_CM const int32_t *)(a.sieveHand))[reqIdx * kHandStride + 1];
     prefill = ((KVX_CM const int32_t *)(a.prefillLens))[reqIdx];
     asm volatile("" : : "s"(flag), "s"(prefill));
-    if (flag != kCanonFlag) return false;
-    const int32_t mapLim = prefill < static_cast<int32_t>(mapCap) ? prefill : static_cast<int32_t>(mapCap);
-    return mapLim <= static_cast<int32_t>(a.htSize);
+    mapLim = prefill < static_cast<int32_t>(mapCap) ? prefill : static_cast<int32_t>(mapCap);
+    return flag == kCanonFlag;
 }
 
 __global__ __launch_bounds__(kPreThreads) void kvx_sieve_batch_pre(BatchParams P)
@@ -232,8 +231,8 @@ __global__ __launch_bounds__(kPreThreads) void kvx_sieve_batch_pre(BatchParams P
         const uint32_t c = c0 + static_cast<uint32_t>(tid + q * kPreThreads);
         if (c < c1) cv[q] = t16[c];
     }
-    if (!batch_row_bitmap(a, reqIdx, prefill, P.mapCap)) return;
-    const int32_t mapLim = prefill < static_cast<int32_t>(P.mapCap) ? prefill : static_cast<int32_t>(P.mapCap);
+    int32_t mapLim = 0;
+    if (!batch_row_bitmap(a, reqIdx, prefill, mapLim, P.mapCap)) return;
     KVX_GM uint32_t *first = (KVX_GM uint32_t *)P.aux + static_cast<uint64_t>(bid) * P.auxWords + P.mapCap;
     KVX_GM uint32_t *bits = first + P.mapCap;
     KVX_GM uint32_t *counts = bits + P.mapCap / 32u;
@@ -303,8 +302,8 @@ __global__ __launch_bounds__(kPreThreads) void kvx_sieve_batch_slots(BatchParams
         const int32_t q = q0 + tid + j * kPreThreads;
         if (q < q1) tv[j] = t4[q];
     }
-    if (!batch_row_bitmap(a, reqIdx, prefill, P.mapCap)) return;
-    const int32_t mapLim = prefill < static_cast<int32_t>(P.mapCap) ? prefill : static_cast<int32_t>(P.mapCap);
+    int32_t mapLim = 0;
+    if (!batch_row_bitmap(a, reqIdx, prefill, mapLim, P.mapCap)) return;
     KVX_GM uint32_t *first = (KVX_GM uint32_t *)P.aux + static_cast<uint64_t>(bid) * P.auxWords + P.mapCap;
     const KVX_GM uint32_t *bits = first + P.mapCap;
     KVX_GM uint32_t *counts = first + P.mapCap + P.mapCap / 32u;
@@ -731,6 +730,8 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
 {
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ int32_t sScan[BT];
+    __shared__ int32_t sBits;  // the pre-passes' bitmap form holds for the row
+    __shared__ int32_t sRing;  // the hand made no full turn: the misses took their slots in ring order
     __shared__ int32_t sBad, sWrap, sLive, sOcc, sNamed, sNdel, sHand, sE0, sTableBad, sFirstMiss, sMisses;
     __shared__ uint32_t sFp, sFpD;  // the pre-step tokens' fingerprint; its change by the step's new tokens
 
@@ -808,12 +809,6 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
     // a row this kernel (or the LDS kernel) left consistent: the table scans
     // of the check are skipped, its live tokens and entries still counted
     const bool flagged = flagWord == kCanonFlag;
-    // such a row, with its tokens below the table size, needs no map: the
-    // step's tokens are marked in a bitmap over [0, mapLim) (the LDS of the
-    // deleted-cell bits, unused until the outputs), and one pass over the
-    // slots finds the resident ones
-    const bool useBits = flagged && mapLim <= H;
-
     const BatchLayout &y = P.lay;
     uint64_t *visB = reinterpret_cast<uint64_t *>(lds + y.vis);
     uint64_t *evB = reinterpret_cast<uint64_t *>(lds + y.ev);
@@ -849,6 +844,7 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
         sTableBad = 0;
         sFirstMiss = K;
         sMisses = 0;
+        sRing = 1;
         sFp = sFpD = 0u;
     }
     for (uint32_t w = tid; w < nVisW; w += BT) {
@@ -856,7 +852,26 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
         evB[w] = 0ull;
     }
     for (uint32_t w = tid; w < nCellW; w += BT) delB[w] = 0ull;
+    // Such a row needs no map: the pre-passes marked the step's tokens in a
+    // bitmap over [0, mapLim), found the resident ones in one pass over the
+    // slots, and counted its tokens and entries.  A token past the map, a live
+    // token without an entry (or the reverse), tokens changed since the flag
+    // was written (an edit in place), or a table without an empty cell, where
+    // probes never stop, take the full check, or the in-order recurrence where
+    // the tokens lie below the table size.
+    if (tid == 0) {
+        const bool good = pc[3] == 0u && pc[2] == pc[0] && pc[4] == static_cast<uint32_t>(fpWord) && pc[1] != 0u;
+        sBits = flagged && (good || mapLim <= H) ? 1 : 0;
+        if (sBits) {
+            if (!good) sBad = 1;
+            sOcc = sNamed = static_cast<int32_t>(pc[0]);
+            sE0 = static_cast<int32_t>(pc[1]) - 1;
+            sLive = static_cast<int32_t>(pc[2]);
+            sFp = pc[4];
+        }
+    }
     __syncthreads();
+    const bool useBits = sBits != 0;
     if (!useBits) {
         // the map by plain stores; a token held by two slots is found when
         // the map is read back below (one of them reads the other's slot).
@@ -888,16 +903,6 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
         if (bad) sBad = 1;
         for (int d = 32; d > 0; d >>= 1) fp += __shfl_xor(fp, d);
         if (lane == 0 && fp) atomicAdd(&sFp, fp);
-    }
-    // a flagged row whose tokens changed since the flag was written (an edit
-    // in place) is checked in full like an unflagged one (in the bitmap form,
-    // without a map, it takes the in-order recurrence instead, below)
-    bool full = !flagged;
-    if (flagged && !useBits) {
-        __syncthreads();
-        full = sFp != static_cast<uint32_t>(fpWord);
-    }
-    if (full) {
         __syncthreads();
         {
             int32_t bad = 0;
@@ -1008,50 +1013,6 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
             int32_t cnt = 0;
             for (int32_t w = tid; w < (dbs + 31) / 32; w += BT) cnt += __builtin_popcount(named[w]);
             if (cnt) atomicAdd(&sNamed, cnt);
-        }
-    } else {
-        // the entries counted and the last empty cell found, 8 cells a load
-        // (counted by the pre-pass for a row in the bitmap form)
-        int32_t occ = 0, last = -1;
-        if (useBits && tid == 0) {
-            occ = static_cast<int32_t>(pc[0]);
-            last = static_cast<int32_t>(pc[1]) - 1;
-            sLive = static_cast<int32_t>(pc[2]);
-            sFp = pc[4];
-            // a token past the map, or a live token without an entry (or the
-            // reverse), or tokens changed since the flag was written: the
-            // in-order recurrence instead
-            if (pc[3] != 0u || pc[2] != pc[0] || pc[4] != static_cast<uint32_t>(fpWord)) sBad = 1;
-        }
-        const uint32_t nChunk = static_cast<uint32_t>(H) / 8u;
-        const KVX_GM u32x4 *t16 = reinterpret_cast<const KVX_GM u32x4 *>(r.ht);
-        for (uint32_t c0 = tid; c0 < nChunk && !useBits; c0 += BT * kCheckUnroll) {
-            u32x4 v[kCheckUnroll];
-#pragma unroll
-            for (int q = 0; q < kCheckUnroll; ++q) {
-                const uint32_t c = c0 + static_cast<uint32_t>(q) * BT;
-                if (c < nChunk) v[q] = t16[c];
-            }
-#pragma unroll
-            for (int q = 0; q < kCheckUnroll; ++q) {
-                if (c0 + static_cast<uint32_t>(q) * BT >= nChunk) continue;
-                const uint32_t c = (c0 + static_cast<uint32_t>(q) * BT) * 8u;
-                const uint32_t w[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
-#pragma unroll
-                for (int h = 0; h < 4; ++h) {
-                    const uint32_t lo = w[h] & 0xFFFFu, hi = w[h] >> 16;
-                    occ += (lo != 0u) + (hi != 0u);
-                    if (lo == 0u) last = static_cast<int32_t>(c + 2u * h);
-                    if (hi == 0u) last = static_cast<int32_t>(c + 2u * h + 1u);
-                }
-            }
-        }
-        if (occ) atomicAdd(&sOcc, occ);
-        if (last >= 0) atomicMax(&sE0, last);
-        __syncthreads();
-        if (tid == 0) {
-            sNamed = sOcc;
-            if (sE0 < 0) sBad = 1;  // no empty cell: probes never stop
         }
     }
     __syncthreads();
@@ -1285,6 +1246,7 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
         if (lane == 0) {
             visB[cwIdx] = cwVal;
             sHand = hand;
+            sRing = passed <= dbs ? 1 : 0;
             sWrap = bail ? 1 : 0;
             sMisses = nMiss;
         }
@@ -1316,7 +1278,7 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
         const int32_t t = rt[k];
         if (t >= 0 && t < seqLen && t < prefill && t < mapLim) first[t] = 0u;
     }
-    if (useBits) {
+    if (flagged) {  // what the pre-passes left
         for (int32_t w = tid; w < (mapLim + 31) / 32; w += BT) gBits[w] = 0u;
         for (int32_t k = tid; k < K; k += BT) gResSlot[k] = 0u;
         if (tid < static_cast<int>(kBatchCounts)) gCounts[tid] = 0u;
@@ -1355,12 +1317,10 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
     __syncthreads();  // code[] is dead from here on (its LDS becomes the bitmaps)
     if (P.tbl != nullptr && sMisses > 0) {
         // The table's deletions and inserts go to the rebuild kernels: the
-        // step's evicted slots, its new keys in event order with their homes
-        // (zeroed per-home counts for them to fill), then the new tokens.
-        const uint32_t HH = static_cast<uint32_t>(H) < 65536u ? static_cast<uint32_t>(H) : 65536u;
+        // step's evicted slots, its new keys in event order with their homes,
+        // then the new tokens.
         KVX_GM uint64_t *ev64 = (KVX_GM uint64_t *)(tbl + P.t.evict);
         for (uint32_t w = tid; w < nVisW; w += BT) ev64[w] = evB[w];
-        for (uint32_t i = tid; i < HH; i += BT) tbl[P.t.hist + i] = 0u;
         // the misses' ranks in position order: a contiguous run of positions per thread
         const int32_t per = (K + BT - 1) / BT;
         const int32_t k0 = tid * per, k1 = k0 + per < K ? k0 + per : K;
@@ -1411,6 +1371,8 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
         __syncthreads();
         if (tid == 0) {
             tbl[P.t.meta + 1] = static_cast<uint32_t>(sMisses);
+            tbl[P.t.meta + 3] = sRing ? 1u : 0u;
+            tbl[P.t.meta + 4] = static_cast<uint32_t>(hand0 < 0 || hand0 >= dbs ? 0 : hand0);
             tbl[P.t.meta] = 1u;
             gHand[1] = kCanonFlag;  // the rebuild leaves the table consistent
             gHand[kFingerprintWord] = static_cast<int32_t>(sFp + sFpD);

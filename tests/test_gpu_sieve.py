@@ -1209,6 +1209,48 @@ def test_sieve_batch_scratch_across_shapes(kvops, form):
     assert kvops.read_overflow() == 0
 
 
+@pytest.mark.parametrize("dbs,top_k,last", [(40, 16, False), (480, 31, True), (3000, 512, False), (9000, 1200, True),
+                                            (16384, 2048, False), (16384, 2048, True), (33000, 900, True)])
+def test_sieve_table_short_clusters(kvops, dbs, top_k, last):
+    """The one-workgroup table update of steps that change short clusters:
+    tokens spread over the table, or half of them homed in its last 1/64 of
+    homes (clusters around a table's end, or past cell 65535 in a larger one,
+    which the rebuild takes), 1 to all misses a row; full state against the
+    oracle after every step."""
+    rng = np.random.default_rng(dbs + top_k + last)
+    req, prefill = 3, 1 << 18
+    st = orc.SieveState(1, req, dbs, top_k)
+    homes = min(st.ht_size, 65536)
+    t = np.arange(prefill, dtype=np.int64)
+    near = t[_home(t, st.ht_size) >= homes - homes // 64] if last else t
+    for r in range(req):
+        st.admit(r, prefill)
+        vals = np.unique(np.concatenate([rng.choice(near, size=min(dbs // 64 + 1, len(near)), replace=False),
+                                         rng.choice(t, size=dbs, replace=False)]))
+        st.tokens[0, r, :dbs] = rng.permutation(vals)[:dbs]
+    orc.sieve_ht_init(st.tokens, st.ht, 0, req, 1, req, dbs, st.padded, st.ht_size)
+    dev = DevSieve(st)
+    kvops.sieve_force_variant(5)
+    try:
+        for step, misses in enumerate([1, top_k // 3, top_k - 2, 0, top_k // 5]):
+            batch = np.empty((req, top_k), dtype=np.int32)
+            for r in range(req):
+                live = st.tokens[0, r, :dbs]
+                fresh = np.setdiff1d(near if step % 2 else t, live)
+                batch[r] = rng.permutation(np.concatenate([rng.choice(live, size=top_k - misses),
+                                                           rng.choice(fresh, size=misses)]))
+            seq = np.full(req, prefill)
+            e_slots, e_miss = st.update(0, batch, np.arange(req), seq, req)
+            g_slots, g_miss, _ = dev.update(kvops, 0, batch, np.arange(req), seq, req, req, top_k)
+            assert kvops.last_sieve_variant() == 5
+            np.testing.assert_array_equal(g_miss, e_miss, err_msg="step {}".format(step))
+            np.testing.assert_array_equal(g_slots, e_slots, err_msg="step {}".format(step))
+            dev.assert_state_equal()
+    finally:
+        kvops.sieve_force_variant(-1)
+    assert kvops.read_overflow() == 0
+
+
 @pytest.mark.parametrize("case", ["wrap", "past-2^16"])
 def test_sieve_table_rebuild_cluster_edges(kvops, case):
     """The parallel table rebuild where the cell order matters most: "wrap"
