@@ -284,15 +284,23 @@ StreamScratch &ScratchFor(uint64_t stream, const ScratchNeed &need, const char *
 }
 
 // The SIEVE kernel a row shape launches: 2 = parallel LDS kernel, 4 = the same
-// with the compact LDS layout (token hashes in LDS, tokens in HBM), 0 =
-// sequential LDS kernel, 5 = batch HBM-resident kernel (state in HBM,
-// decisions and bitmaps in LDS), 3 = sequential HBM-resident kernel with
-// wave-wide probes (1 = the single-lane HBM kernel, only when forced).
+// with the compact LDS layout (token hashes in LDS, tokens in HBM), 5 = batch
+// HBM-resident kernel (state in HBM, decisions and bitmaps in LDS), 0 =
+// sequential LDS kernel, 3 = sequential HBM-resident kernel with wave-wide
+// probes (1 = the single-lane HBM kernel, only when forced).  A row that fits
+// LDS but neither parallel layout (about 9000 to 15000 slots at 900 and more
+// positions) takes the batch kernel: 9 rows of 9370 slots and 1655 positions
+// 1060 us a call on the sequential one, 70 on the batch kernel.  With as many
+// positions as slots a slot can be evicted twice in a step, which the batch
+// kernel leaves to a recurrence on HBM, so such a row stays on the sequential
+// LDS kernel; and so does a call whose stream has no scratch for the batch
+// kernel and cannot get it (capture, memory).
 struct SievePlan {
     int variant = 0;
     size_t ldsLaunch = 0;   // dynamic LDS of the launch
     uint32_t invCap = 0;    // entries of the parallel kernel's token -> slot map
     bool rebuild = false;   // variant 5: a step's table changes by the rebuild kernels
+    size_t ldsInOrder = 0;  // variant 5: LDS of variant 0, which takes the row without scratch (0: it cannot)
 };
 
 SievePlan PlanSieve(uint32_t top_k, uint32_t dbs, uint32_t padded, uint32_t visStrideB, uint32_t poolSize,
@@ -309,14 +317,19 @@ SievePlan PlanSieve(uint32_t top_k, uint32_t dbs, uint32_t padded, uint32_t visS
     const bool compactOk = fastShape && ldsCompact <= g.ldsLimit && lds <= g.ldsLimit;
     const size_t ldsBatch = kvx::batch_layout(dbs, htSize, top_k).total;
     const bool batchOk = top_k >= 1 && top_k < (1u << 24) && dbs <= 65535 && htSize >= 1024 && ldsBatch <= g.ldsBatch;
-    int v = fastOk ? 2 : (compactOk ? 4 : (lds <= g.ldsLimit ? 0 : (batchOk ? 5 : 3)));
+    const bool inOrderOk = lds <= g.ldsLimit;
+    int v = fastOk ? 2 : (compactOk ? 4 : (inOrderOk && !(batchOk && top_k < dbs) ? 0 : (batchOk ? 5 : 3)));
+    if (v == 5 && inOrderOk) p.ldsInOrder = lds;
     const int f = g.forcedSieveVariant;
-    if (f == 0 && lds <= g.ldsLimit) v = 0;
+    if (f == 0 && inOrderOk) v = 0;
     if (f == 1) v = 1;
     if (f == 2 && fastOk) v = 2;
     if (f == 3) v = 3;
     if (f == 4 && compactOk) v = 4;
-    if ((f == 5 || f == 6) && batchOk) v = 5;
+    if ((f == 5 || f == 6) && batchOk) {
+        v = 5;
+        p.ldsInOrder = 0;
+    }
     p.variant = v;
     // the batch kernel hands a step's table changes to the rebuild kernels
     // where their windows fit (force 6: it applies them itself)
@@ -929,8 +942,18 @@ int kvx_sieve_update(uint64_t topk_indices, uint64_t req_pool_indices, uint64_t 
         a.reqsPerCore = static_cast<uint32_t>(rpc);
         a.htSize = static_cast<uint32_t>(htSize);
         a.poolSize = pool_size;
-        const SievePlan plan = PlanSieve(top_k, device_buffer_size, padded_buffer_size, visited_stride_b, pool_size,
-                                         static_cast<uint32_t>(htSize));
+        SievePlan plan = PlanSieve(top_k, device_buffer_size, padded_buffer_size, visited_stride_b, pool_size,
+                                   static_cast<uint32_t>(htSize));
+        if (plan.variant == 5 && plan.ldsInOrder != 0) {
+            std::lock_guard<std::mutex> lk(g_scratchMu);
+            try {
+                (void)ScratchFor(stream, SieveScratchNeed(plan, max_num_reqs, static_cast<uint32_t>(htSize)), "sieve_update");
+            } catch (const Error &) {
+                (void)hipGetLastError();  // a failed allocation is not the launch's error
+                plan.variant = 0;
+                plan.ldsLaunch = plan.ldsInOrder;
+            }
+        }
         a.reserved = static_cast<uint32_t>(plan.variant) | (plan.invCap << 8);
         g.lastSieveVariant = plan.variant;
         if (max_num_reqs == 0) return;

@@ -1296,3 +1296,64 @@ def test_sieve_table_rebuild_cluster_edges(kvops, case):
     finally:
         kvops.sieve_force_variant(-1)
     assert kvops.read_overflow() == 0
+
+
+@pytest.mark.parametrize("dbs,top_k,want", [(9370, 1655, 5), (12000, 1200, 5), (15000, 1000, 5), (700, 16383, 0)])
+def test_sieve_rows_between_the_layouts(kvops, dbs, top_k, want):
+    """Rows that fit LDS but neither layout of the parallel kernel: the batch
+    kernel, or the sequential one with as many positions as slots; full state
+    against the oracle after every step."""
+    rng = np.random.default_rng(dbs)
+    req, prefill = 2, dbs + 3000
+    st = orc.SieveState(1, req, dbs, top_k)
+    for r in range(req):
+        st.admit(r, prefill)
+    dev = DevSieve(st)
+    for step in range(3):
+        batch = _random_state_stream(rng, st, top_k, prefill, miss_frac=0.25)
+        seq = np.full(req, prefill + 3)
+        e_slots, e_miss = st.update(0, batch, np.arange(req), seq, req)
+        g_slots, g_miss, _ = dev.update(kvops, 0, batch, np.arange(req), seq, req, req, top_k)
+        assert kvops.last_sieve_variant() == want
+        np.testing.assert_array_equal(g_miss, e_miss, err_msg="step {}".format(step))
+        np.testing.assert_array_equal(g_slots, e_slots, err_msg="step {}".format(step))
+        dev.assert_state_equal()
+    assert kvops.read_overflow() == 0
+
+
+def test_sieve_between_the_layouts_captured_without_scratch(kvops):
+    """Such a row under capture on a stream without scratch runs the
+    sequential kernel, as it needs none; each replay against the oracle."""
+    import torch
+
+    rng = np.random.default_rng(77)
+    dbs, top_k, req = 9370, 1655, 2
+    prefill = dbs + 3000
+    st = orc.SieveState(1, req, dbs, top_k)
+    for r in range(req):
+        st.admit(r, prefill)
+    dev = DevSieve(st)
+    topk = torch.empty((req, top_k), dtype=torch.int32, device="cuda")
+    slots = torch.empty_like(topk)
+    miss = torch.empty((req, top_k), dtype=torch.int8, device="cuda")
+    pool = torch.arange(req, device="cuda")
+    seq = torch.full((req,), prefill, dtype=torch.int32, device="cuda")
+    real = torch.full((1,), req, dtype=torch.int32, device="cuda")
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=stream):
+        kvops.sieve_update(topk.data_ptr(), pool.data_ptr(), seq.data_ptr(), dev.prefill.data_ptr(),
+                           dev.tokens.data_ptr(), dev.vis.data_ptr(), dev.ht.data_ptr(), dev.hand.data_ptr(),
+                           slots.data_ptr(), miss.data_ptr(), real.data_ptr(), top_k, dbs, st.padded,
+                           st.vis.shape[-1], req, req, stream.cuda_stream)
+    assert kvops.last_sieve_variant() == 0
+    for _ in range(3):
+        batch = _random_state_stream(rng, st, top_k, prefill, miss_frac=0.25)
+        topk.copy_(torch.from_numpy(batch.astype(np.int32)))
+        g.replay()
+        torch.cuda.synchronize()
+        e_slots, e_miss = st.update(0, batch, np.arange(req), np.full(req, prefill), req)
+        np.testing.assert_array_equal(slots.cpu().numpy(), e_slots)
+        np.testing.assert_array_equal(miss.cpu().numpy(), e_miss)
+        dev.assert_state_equal()
