@@ -5,16 +5,17 @@
 // kvc_scatter_rows_alllayer.cpp:11-67 of the reference, with the row
 // ownership of kv_layout.h.  The reference moves each row with one HCOMM
 // ReadNbi/WriteNbi; here the host segments are pinned host memory mapped
-// into the device address space.  The import runs in two launches: winners
-// (the last miss position per destination row), then the listing and the
-// copy, where 64 workgroups claim 256 positions at a time, list their rows in
-// LDS with the reference's queued counts, and move them as 16-byte chunks, 8
-// chunks in flight per lane.  A small batch (up to 4096 positions) takes one
-// launch instead (below).
+// into the device address space.  The import is one launch: each workgroup
+// finds the winners (the last miss position per destination row) among its own
+// positions, lists their rows in LDS with the reference's queued counts, and
+// moves them as 16-byte chunks, 8 chunks in flight per lane.  Calls whose
+// requests share rows over more than 8192 positions take two launches: winners
+// in memory, then the listing and the copy, where 64 workgroups claim 256
+// positions at a time.
 //
 // Completion: the last workgroup to finish (atomicInc ticket) stores the
 // status words with a system-scope release, after every workgroup fenced its
-// own row stores.  The reference's per-block Commit/Drain + MTE3 flush has the
+// own row stores, or waited for stores that go through the caches.  The reference's per-block Commit/Drain + MTE3 flush has the
 // same meaning: all rows of the launch have landed.
 #include <cstddef>
 
@@ -56,6 +57,7 @@ struct GatherExtra {
     uint32_t fused;
     uint32_t spanRows;
     uint32_t statusWords;
+    uint32_t groupSize, span, parts, blocks;  // one launch: positions of a group and of a span, spans of a group and in all
 };
 
 struct GatherParams {
@@ -90,6 +92,18 @@ __device__ __forceinline__ void store_status(uint64_t addr, uint64_t word)
 {
     __hip_atomic_store(reinterpret_cast<uint64_t *>(addr), word, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
+
+// A 16-byte store that goes through the caches to memory.  Once a workgroup's
+// stores of this kind are done (wait_stores) its rows are visible everywhere,
+// and it can report them without a fence: a device-scope release writes back
+// the whole L2 of its XCD, and one per workgroup, while others still copy,
+// took a fifth of the import (131072 positions from 1024 workgroups 859 -> 671
+// us without it, 1665 positions from 105 27 -> 19).
+__device__ __forceinline__ void store_through(uint64_t addr, u32x4 v)
+{
+    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt" : : "v"(addr), "v"(v) : "memory");
+}
+__device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" : : : "memory"); }
 
 // Copy `n` rows whose byte addresses sit in src[0..n), dst[0..n) (LDS or
 // global) with the whole wave: chunk c covers bytes [16*(c%cpr), +16) of row
@@ -284,161 +298,209 @@ __global__ __launch_bounds__(256) void kvx_gather_span(GatherParams P)
         for (uint64_t i = tid; i < x.winEntries; i += blockDim.x) x.win[i] = 0ull;
     }
     if (tid == 0) *x.epoch = sEpoch + 1u;
-    if (a.status == 0) return;
     __threadfence();
     const uint32_t n0 = x.fused ? 0u : a.myNode;
     const uint32_t n1 = x.fused ? a.nodeNum : a.myNode + 1u;
-    for (uint32_t i = tid; i < (n1 - n0) * x.statusWords; i += blockDim.x) {
-        const uint32_t node = n0 + i / x.statusWords, b = i % x.statusWords;
+    for (uint32_t i = tid; i < (n1 - n0) * 8u; i += blockDim.x) {
+        const uint32_t node = n0 + i / 8u, b = i % 8u;
+        const uint32_t q = __hip_atomic_load(&x.counters[node * 8u + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t e = __hip_atomic_load(&x.errs[node * 8u + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        x.counters[node * 8u + b] = 0u;  // the one-launch import finds them zeroed
+        x.errs[node * 8u + b] = 0u;
+        if (a.status == 0 || b >= x.statusWords) continue;
         uint64_t word = 1ull << 32;  // kvc_gather_rows.cpp:29-33, :93
         if (static_cast<int64_t>(b * ppc) < total) {
-            const uint32_t q = __hip_atomic_load(&x.counters[node * 8u + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const uint32_t e = __hip_atomic_load(&x.errs[node * 8u + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             word |= (static_cast<uint64_t>(q) << 40) | (e == 0xFFFFFFFFu ? 0u : row_error_code(e));
         }
         store_status(a.status + node * 64ull + b * 8ull, word);
     }
 }
 
-// Small batches (max_num_reqs * top_k <= kSmallMaxPositions): the three
-// passes in one launch.  A winner is the last miss on its destination row;
-// the rows of request b start at b * spanRows, so a row that a later request
-// can also reach is one whose slot is at or past spanRows.  Each workgroup
-// loads the slots of the requests its own kSmallSpan positions belong to
-// into LDS; when none of its own positions has such a slot (the usual case),
-// eight lanes per own position look for a later position of the same
-// request with the same slot, and no global tags are needed.  Otherwise the
-// workgroup tags every position of the call (relaxed device-scope max, as
-// the two-launch path does) and reads its own positions' tags.  Each
-// workgroup counts the queued rows and errors of all positions in its own
-// LDS, then moves the winners among its own positions: the rows spread over
-// ceil(positions / kSmallSpan) CUs (one CU reads only a few GB/s from host
-// memory), with no counters shared between workgroups.  The last workgroup
-// (ticket) advances the epoch and stores the status words.
-constexpr uint32_t kSmallMaxPositions = 4096;
-constexpr uint32_t kSmallSpan = 32;
+// The import in one launch, where a group -- the positions that can share a
+// destination row -- is short: a request (rows of request b start at
+// b * spanRows), or the whole call where every request has the same rows
+// (spanRows 0).  A winner is the last miss on its destination row.  Each
+// workgroup takes `span` consecutive positions of one group and marks the
+// slots of the group's later positions in a bitmap; an own position wins when
+// its slot is neither there nor at a later own position.  A slot at or past
+// spanRows also reaches rows of later requests: such positions (none in a
+// buffer of spanRows slots a request) are looked for in those requests one by
+// one.  The workgroup counts its own queued rows and errors, adds them to the
+// call's counters and moves its rows; the last one (ticket) stores the status
+// words and leaves the counters zeroed for the next call.
+//
+// The bound is the host link.  The reads of many CUs fill it (1638 rows of
+// 1152 bytes alone: 72 us from 16 workgroups, 46 from 32, 40 from 128 and
+// more), so the spans are short, up to 256 workgroups; past that they take
+// several spans in turn, which keeps the rows in flight near each other
+// (64 requests of 2048 positions: 64 workgroups 674 us, 128 639, 256 633, 512
+// 651, 1024 662; spans of 128: 654 from 256).  Against a launch that marked
+// the winners in memory and one that listed and moved the rows: 8192 positions
+// 56 -> 47 us, 1665 positions in the earlier one-launch form, where every
+// workgroup counted all positions, 29 -> 19; 131072 positions 639 -> 633 (the
+// link).
+constexpr uint32_t kOneMinSpan = 16, kOneMaxSpan = 64;
+constexpr uint32_t kOneMaxGroup = 8192;  // positions of a group (each workgroup reads the later ones)
+constexpr uint32_t kOneMaxBlocks = 256;  // workgroups; more spans are taken in turn
+constexpr int kOneThreads = 256;
 
-__global__ __launch_bounds__(256) void kvx_gather_small(GatherParams P)
+__global__ __launch_bounds__(kOneThreads) void kvx_gather_one(GatherParams P)
 {
+    __shared__ uint32_t sLater[65536 / 32];
     __shared__ uint32_t sCnt[64 * 8], sErr[64 * 8];
-    __shared__ uint64_t sSrc[kSmallSpan], sDst[kSmallSpan];
-    __shared__ int32_t sKey[kSmallMaxPositions];  // slot of each position of the requests met, or -1
-    __shared__ uint32_t sN, sEpoch, sLose;         // sLose bit i: own position lo + i is not a winner
+    __shared__ uint64_t sSrc[kOneMaxSpan], sDst[kOneMaxSpan];
+    __shared__ int32_t sKey[kOneMaxSpan];   // slot of an own position in the winner rule, else -1
+    __shared__ uint32_t sLose[kOneMaxSpan / 32];
+    __shared__ uint32_t sN;
     __shared__ int sLast;
     const KvcGatherArgs &a = P.l.a;
     const GatherExtra &x = P.x;
-    const uint32_t tid = threadIdx.x;
-    const int32_t numReal = clamp_num_real(a.numReal, a.maxNumReqs);
-    const int64_t total = static_cast<int64_t>(numReal) * a.topK;  // <= kSmallMaxPositions (host)
+    const uint32_t tid = threadIdx.x, lane = static_cast<uint32_t>(lane_id());
     const uint32_t n0 = x.fused ? 0u : a.myNode;
     const uint32_t n1 = x.fused ? a.nodeNum : a.myNode + 1u;
-    const uint64_t ppc = a.positionsPerCore == 0 ? 1ull : a.positionsPerCore;
+    const uint32_t ppc = a.positionsPerCore == 0 ? 1u : a.positionsPerCore;
     const KVX_G int32_t *topk = reinterpret_cast<const KVX_G int32_t *>(a.topkIndices);
     const KVX_G int32_t *slots = reinterpret_cast<const KVX_G int32_t *>(a.topKDeviceSlots);
     const KVX_G int8_t *miss = reinterpret_cast<const KVX_G int8_t *>(a.isMiss);
     const KVX_G int64_t *pool = reinterpret_cast<const KVX_G int64_t *>(a.reqPoolIndices);
     const KVX_G int64_t *hostBase = reinterpret_cast<const KVX_G int64_t *>(a.reqHostBase);
+    const int32_t numReal = clamp_num_real(a.numReal, a.maxNumReqs);
+    const uint32_t total = static_cast<uint32_t>(numReal) * a.topK;  // (host: below 2^31)
     if (blockIdx.x == 0 && a.status != 0) {  // the call's status words read 0 until its rows have landed
-        for (uint32_t i = tid; i < (n1 - n0) * x.statusWords; i += blockDim.x) {
-            const uint32_t node = n0 + i / x.statusWords, b = i % x.statusWords;
-            store_status(a.status + node * 64ull + b * 8ull, 0ull);
+        for (uint32_t i = tid; i < (n1 - n0) * x.statusWords; i += kOneThreads) {
+            store_status(a.status + (n0 + i / x.statusWords) * 64ull + (i % x.statusWords) * 8ull, 0ull);
         }
     }
-    for (uint32_t i = tid; i < 64u * 8u; i += blockDim.x) {
+    for (uint32_t i = n0 * 8u + tid; i < n1 * 8u; i += kOneThreads) {
         sCnt[i] = 0u;
-        sErr[i] = 0xFFFFFFFFu;  // lowest failing position, min-reduced
+        sErr[i] = 0u;
     }
-    if (tid == 0) {
-        sN = 0u;
-        sEpoch = *x.epoch;
-    }
-    __syncthreads();
-    const unsigned long long tagHi = static_cast<unsigned long long>(sEpoch) << 32;
-    const int64_t lo = static_cast<int64_t>(blockIdx.x) * kSmallSpan, hi = lo + kSmallSpan;
-    // the slot of position p when p takes part in the winner rule, else -1
-    // (the four reads issued together)
-    auto tagged_slot = [&](int64_t p) -> int32_t {
-        const int64_t bid = p / a.topK;
-        const int8_t m = miss[p];
-        const int32_t t = topk[p], s = slots[p];
-        const int64_t pl = pool[bid];
-        if (m == 0 || t < 0 || s < 0 || s >= 65536 || pl < 0) return -1;
-        return win_index(bid, s, x.spanRows) < x.winEntries ? s : -1;
-    };
-    // the positions of the requests that [lo, hi) meets (at most the call's)
-    const int64_t tagLo = lo < total ? (lo / a.topK) * a.topK : total;
-    const int64_t tagHiPos = hi < total ? ((hi - 1) / a.topK + 1) * a.topK : total;
-    int shared = 0;
-    for (int64_t p = tagLo + tid; p < tagHiPos; p += blockDim.x) {
-        const int32_t s = tagged_slot(p);
-        sKey[p - tagLo] = s;
-        shared |= (p >= lo && p < hi && s >= 0 && static_cast<uint32_t>(s) >= x.spanRows) ? 1 : 0;
-    }
-    if (tid == 0) sLose = 0u;
-    const bool global = __syncthreads_or(shared) != 0;
-    if (global) {
-        for (int64_t p = tid; p < total; p += blockDim.x) {
-            const int32_t s = tagged_slot(p);
-            if (s >= 0) win_max(x.win + win_index(p / a.topK, s, x.spanRows), tagHi | static_cast<unsigned long long>(p));
+    for (uint32_t blk = blockIdx.x; blk < x.blocks; blk += gridDim.x) {
+        const uint32_t group = blk / x.parts, part = blk - group * x.parts;
+        const uint32_t g0 = group * x.groupSize, lo = g0 + part * x.span, p = lo + tid, bid = p / a.topK;
+        for (uint32_t i = tid; i < 65536u / 32u / 4u; i += kOneThreads) reinterpret_cast<uint4 *>(sLater)[i] = make_uint4(0, 0, 0, 0);
+        if (tid < kOneMaxSpan / 32u) sLose[tid] = 0u;
+        if (tid == 0) sN = 0u;
+        const uint32_t gEnd = min(g0 + x.groupSize, total);
+        const uint32_t hi = min(lo + x.span, gEnd);
+        int8_t m = 0;
+        int32_t t = -1, s = -1;
+        int64_t pl = -1, hb = 0;
+        if (tid < x.span && p < gEnd) {  // the own position's five reads, issued together
+            m = miss[p];
+            t = topk[p];
+            s = slots[p];
+            pl = pool[bid];
+            hb = hostBase[bid];
         }
-        __threadfence();
-    } else {
-        // lanes 8i .. 8i+7: own position lo + i against the later positions of its request
-        const int64_t p = lo + static_cast<int64_t>(tid >> 3);
-        int32_t s = -1;
-        int64_t end = 0;
-        if (p < hi && p < total) {
-            s = sKey[p - tagLo];
-            end = (p / a.topK + 1) * a.topK;
-        }
-        bool later = false;
-        if (s >= 0) {
-            for (int64_t q = p + 1 + static_cast<int64_t>(tid & 7u); q < end; q += 8) later |= sKey[q - tagLo] == s;
-        }
-        const uint64_t m = __ballot(later);
-        const uint32_t lane = static_cast<uint32_t>(lane_id());
-        if ((tid & 7u) == 0u && ((m >> lane) & 0xFFull) != 0ull) atomicOr(&sLose, 1u << (tid >> 3));
-    }
-    __syncthreads();
-    for (int64_t p = tid; p < total; p += blockDim.x) {
-        const int64_t bid = p / a.topK;
-        const int8_t m = miss[p];  // the five reads issued together
-        const int32_t t = topk[p], s = slots[p];
-        const int64_t pl = pool[bid], hb = hostBase[bid];
-        if (m == 0 || t < 0 || s < 0 || pl < 0) continue;
-        const uint32_t row = static_cast<uint32_t>(hb + t);  // kvc_gather_rows.cpp:69-73
-        const uint32_t node = kvx_node_of(row, a.stripeRows, a.nodeNum);
-        const bool owned = x.fused ? (node < a.nodeNum) : (node == a.myNode);
-        if (!owned) continue;
-        const uint32_t key = node * 8u + static_cast<uint32_t>(static_cast<uint64_t>(p) / ppc);
-        atomicAdd(&sCnt[key], 1u);
-        const uint64_t segRow = kvx_seg_row_of(row, a.stripeRows, a.nodeNum);
-        if (segRow >= a.perLayerSegRows) {  // row outside the segment: report, do not read
-            atomicMin(&sErr[key], static_cast<uint32_t>(p));
-            continue;
-        }
-        if (p < lo || p >= hi) continue;
-        if (s < 65536) {
-            const uint64_t d = win_index(bid, s, x.spanRows);
-            if (d < x.winEntries && (global ? win_load(x.win + d) != (tagHi | static_cast<unsigned long long>(p))
-                                            : ((sLose >> (p - lo)) & 1u) != 0u)) {
-                continue;
+        // a position in the winner rule: a miss with a token and a slot (16 bits)
+        const bool valid = m != 0 && t >= 0 && s >= 0 && pl >= 0;
+        const bool rule = valid && s < 65536;
+        if (tid < x.span) sKey[tid] = rule ? s : -1;
+        __syncthreads();
+        for (uint32_t q0 = hi + tid; q0 < gEnd; q0 += 4u * kOneThreads) {
+            int8_t mq[4];
+            int32_t tq[4], sq[4];
+            int64_t pq[4];
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; ++j) {  // issued together
+                const uint32_t q = q0 + j * kOneThreads, c = q < gEnd ? q : gEnd - 1u;
+                mq[j] = q < gEnd ? miss[c] : static_cast<int8_t>(0);
+                tq[j] = topk[c];
+                sq[j] = slots[c];
+                pq[j] = pool[c / a.topK];
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; ++j) {
+                if (mq[j] != 0 && tq[j] >= 0 && sq[j] >= 0 && sq[j] < 65536 && pq[j] >= 0) {
+                    atomicOr(&sLater[sq[j] >> 5], 1u << (sq[j] & 31));
+                }
             }
         }
-        const uint64_t segBase = x.fused ? x.segBases[node] : a.segBase;
-        const uint32_t at = atomicAdd(&sN, 1u);
-        sSrc[at] = segBase + (static_cast<uint64_t>(a.layerOffsetRows) + segRow) * a.rowBytes;
-        sDst[at] = a.hotRowBase + (static_cast<uint64_t>(s) + static_cast<uint64_t>(bid) * a.hotReqStrideRows) *
-                                      a.rowBytes;
+        // own positions against the later own ones, kOneThreads / span lanes each
+        {
+            const uint32_t per = kOneThreads / x.span, i = tid / per;  // span: a power of two
+            const int32_t k = sKey[i];
+            bool later = false;
+            if (k >= 0) {
+                for (uint32_t j = i + 1u + (tid & (per - 1u)); j < x.span; j += per) later |= sKey[j] == k;
+            }
+            if (later) atomicOr(&sLose[i >> 5], 1u << (i & 31u));
+        }
+        const bool far = rule && x.spanRows != 0u && static_cast<uint32_t>(s) >= x.spanRows;
+        if (__syncthreads_or(far ? 1 : 0)) {
+            for (uint32_t i = 0; i < x.span; ++i) {
+                const int32_t k = sKey[i];
+                if (k < 0 || static_cast<uint32_t>(k) < x.spanRows) continue;
+                const uint32_t b0 = (lo + i) / a.topK;
+                const uint32_t b1 = min(static_cast<uint32_t>(numReal) - 1u, b0 + static_cast<uint32_t>(k) / x.spanRows);
+                bool later = false;
+                for (uint32_t q = (b0 + 1u) * a.topK + tid; q < (b1 + 1u) * a.topK; q += kOneThreads) {
+                    const uint32_t bq = q / a.topK;
+                    later |= miss[q] != 0 && topk[q] >= 0 && pool[bq] >= 0 &&
+                             slots[q] == k - static_cast<int32_t>((bq - b0) * x.spanRows);
+                }
+                if (later) atomicOr(&sLose[i >> 5], 1u << (i & 31u));
+            }
+            __syncthreads();
+        }
+        bool copy = false;
+        uint64_t src = 0, dst = 0;
+        if (valid) {
+            const uint32_t row = static_cast<uint32_t>(hb + t);  // kvc_gather_rows.cpp:69-73
+            const uint32_t node = kvx_node_of(row, a.stripeRows, a.nodeNum);
+            if (x.fused ? (node < a.nodeNum) : (node == a.myNode)) {
+                const uint32_t key = node * 8u + p / ppc;
+                atomicAdd(&sCnt[key], 1u);
+                const uint64_t segRow = kvx_seg_row_of(row, a.stripeRows, a.nodeNum);
+                if (segRow >= a.perLayerSegRows) {  // row outside the segment: report the lowest, do not read
+                    atomicMax(&sErr[key], ~p);
+                } else {
+                    copy = !rule || (((sLater[s >> 5] >> (s & 31)) | (sLose[tid >> 5] >> (tid & 31u))) & 1u) == 0u;
+                    src = (x.fused ? x.segBases[node] : a.segBase) +
+                          (static_cast<uint64_t>(a.layerOffsetRows) + segRow) * a.rowBytes;
+                    dst = a.hotRowBase + (static_cast<uint64_t>(s) + static_cast<uint64_t>(bid) * a.hotReqStrideRows) * a.rowBytes;
+                }
+            }
+        }
+        const uint64_t cm = __ballot(copy);
+        uint32_t at = 0;
+        if (lane == 0 && cm != 0ull) at = atomicAdd(&sN, static_cast<uint32_t>(__popcll(cm)));
+        at = static_cast<uint32_t>(__shfl(static_cast<int>(at), 0));
+        if (copy) {
+            at += static_cast<uint32_t>(__popcll(cm & ((1ull << lane) - 1ull)));
+            sSrc[at] = src;
+            sDst[at] = dst;
+        }
+        __syncthreads();
+        // the rows' chunks over all lanes
+        const uint32_t cpr = a.rowBytes / 16u, chunks = sN * cpr;
+        for (uint32_t c0 = tid; c0 < chunks; c0 += kOneThreads * kUnroll) {
+            u32x4 v[kUnroll];
+            uint64_t d[kUnroll];
+#pragma unroll
+            for (int j = 0; j < kUnroll; ++j) {
+                const uint32_t c = c0 + static_cast<uint32_t>(j) * kOneThreads;
+                d[j] = 0;
+                if (c < chunks) {
+                    const uint32_t r = c / cpr, o = (c - r * cpr) * 16u;
+                    v[j] = __builtin_nontemporal_load(reinterpret_cast<const GVec *>(sSrc[r] + o));
+                    d[j] = sDst[r] + o;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < kUnroll; ++j) {
+                if (d[j] != 0) store_through(d[j], v[j]);
+            }
+        }
+        __syncthreads();  // the lists are rewritten by the next span
     }
-    __syncthreads();
-    {
-        // the rows, shared among the waves
-        const uint32_t n = sN, cpr = a.rowBytes / 16u, waves = blockDim.x / 64u, w = tid / 64u;
-        const uint32_t share = (n + waves - 1u) / waves, r0 = w * share;
-        if (r0 < n) wave_copy_rows(sSrc + r0, sDst + r0, (n - r0 < share) ? n - r0 : share, cpr);
+    // the call's counts
+    for (uint32_t i = n0 * 8u + tid; i < n1 * 8u; i += kOneThreads) {
+        if (sCnt[i] != 0u) atomicAdd(&x.counters[i], sCnt[i]);
+        if (sErr[i] != 0u) atomicMax(&x.errs[i], sErr[i]);
     }
-    __threadfence();
+    wait_stores();
     __syncthreads();
     if (tid == 0) {
         const unsigned int ticket = atomicInc(&x.tickets[3], gridDim.x - 1u);
@@ -446,20 +508,16 @@ __global__ __launch_bounds__(256) void kvx_gather_small(GatherParams P)
     }
     __syncthreads();
     if (!sLast) return;
-    // the next call's epoch (at the wrap to 0, once in 2^32 calls, the table is cleared)
-    if (sEpoch + 1u == 0u) {
-        for (uint64_t i = tid; i < x.winEntries; i += blockDim.x) x.win[i] = 0ull;
-    }
-    if (tid == 0) *x.epoch = sEpoch + 1u;
-    if (a.status == 0) return;
     __threadfence();
-    for (uint32_t i = tid; i < (n1 - n0) * x.statusWords; i += blockDim.x) {
-        const uint32_t node = n0 + i / x.statusWords, b = i % x.statusWords;
+    for (uint32_t i = tid; i < (n1 - n0) * 8u; i += kOneThreads) {
+        const uint32_t node = n0 + i / 8u, b = i % 8u;
+        const uint32_t q = __hip_atomic_load(&x.counters[node * 8u + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t e = __hip_atomic_load(&x.errs[node * 8u + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (q != 0u) __hip_atomic_store(&x.counters[node * 8u + b], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (e != 0u) __hip_atomic_store(&x.errs[node * 8u + b], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (a.status == 0 || b >= x.statusWords) continue;
         uint64_t word = 1ull << 32;  // kvc_gather_rows.cpp:29-33, :93
-        if (static_cast<int64_t>(b * ppc) < total) {
-            const uint32_t e = sErr[node * 8u + b];
-            word |= (static_cast<uint64_t>(sCnt[node * 8u + b]) << 40) | (e == 0xFFFFFFFFu ? 0u : row_error_code(e));
-        }
+        if (static_cast<uint64_t>(b) * ppc < total) word |= (static_cast<uint64_t>(q) << 40) | (e == 0u ? 0u : row_error_code(~e));
         store_status(a.status + node * 64ull + b * 8ull, word);
     }
 }
@@ -644,15 +702,17 @@ __global__ __launch_bounds__(256) void kvx_export_rows_copy(ExportRowsParams P)
         for (uint64_t k = threadIdx.x; k < P.winEntries; k += blockDim.x) P.win[k] = 0ull;
     }
     if (threadIdx.x == 0) *P.epoch = sEpoch;
-    if (a.status == 0) return;
     __threadfence_system();
     const uint32_t n0 = a.fused ? 0u : a.myNode, n1 = a.fused ? a.nodeNum : a.myNode + 1u;
     for (uint32_t k = threadIdx.x; k < (n1 - n0) * words; k += blockDim.x) {
         const uint32_t node = n0 + k / words, b = k % words;
+        const uint32_t q = __hip_atomic_load(&P.counters[node * 8u + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t e = __hip_atomic_load(&P.errs[node * 8u + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        P.counters[node * 8u + b] = 0u;  // the one-launch import finds them zeroed
+        P.errs[node * 8u + b] = 0u;
+        if (a.status == 0) continue;
         uint64_t word = 1ull << 32;
         if (static_cast<int64_t>(b) * ppc < n) {
-            const uint32_t q = __hip_atomic_load(&P.counters[node * 8u + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const uint32_t e = __hip_atomic_load(&P.errs[node * 8u + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             word |= (static_cast<uint64_t>(q) << 40) | (e == 0xFFFFFFFFu ? 0u : row_error_code(e));
         }
         store_status(a.status + node * 64ull + b * 8ull, word);
@@ -837,10 +897,21 @@ hipError_t launch_gather(const GatherPlan &plan, const RowScratch &scr, uint64_t
     P.x.spanRows = plan.spanRows;
     P.x.statusWords = plan.statusWords;
     const uint64_t positions = static_cast<uint64_t>(plan.a.maxNumReqs) * plan.a.topK;
-    if (positions <= kSmallMaxPositions) {
-        const uint32_t blocks = static_cast<uint32_t>((positions + kSmallSpan - 1u) / kSmallSpan);
-        hipLaunchKernelGGL(kvx_gather_small, dim3(blocks), dim3(256), 0, stream, P);
-        return hipGetLastError();
+    // the positions that can share a destination row
+    const uint64_t group = plan.spanRows == 0 ? positions : plan.a.topK;
+    if (positions != 0 && group <= kOneMaxGroup && positions < (1ull << 31)) {
+        uint32_t span = kOneMinSpan;
+        while (span < kOneMaxSpan && positions / span > kOneMaxBlocks) span *= 2u;
+        P.x.span = span;
+        P.x.groupSize = static_cast<uint32_t>(group);
+        P.x.parts = (P.x.groupSize + span - 1u) / span;
+        const uint64_t blocks = positions / group * P.x.parts;
+        if (blocks < (1ull << 31)) {
+            P.x.blocks = static_cast<uint32_t>(blocks);
+            hipLaunchKernelGGL(kvx_gather_one, dim3(static_cast<uint32_t>(blocks < kOneMaxBlocks ? blocks : kOneMaxBlocks)),
+                               dim3(kOneThreads), 0, stream, P);
+            return hipGetLastError();
+        }
     }
     uint64_t prepBlocks = (positions + 255ull) / 256ull;
     if (prepBlocks < 1) prepBlocks = 1;

@@ -232,6 +232,21 @@ def test_gather_small_batch_winners(kvops, req, top_k, dbs, stride_mode, fused, 
         pool.destroy(close_ext=False)
 
 
+@pytest.mark.parametrize("req,top_k,dbs,stride_mode,fused,block_dim", [
+    (3, 1, 16, "padded", True, 1),           # spans longer than a request
+    (9, 17, 16, "half", True, 8),            # a span of 16 and one of 1 per request
+    (40, 513, 96, "padded", True, 3),        # 20520 positions: workgroups take several spans
+    (40, 513, 96, "half", False, 2),         # ... with rows shared between neighbouring requests
+    (2, 8192, 4096, "padded", True, 2),      # the longest request of the one-launch form
+    (2, 8193, 4096, "padded", True, 2),      # one past it: two launches
+    (8, 1024, 64, "zero", True, 1),          # the longest call with one set of rows
+    (9, 1000, 64, "zero", False, 1),         # one past it: two launches
+])
+def test_gather_spans(kvops, req, top_k, dbs, stride_mode, fused, block_dim):
+    """The same at the edges of the spans, of their number and of the forms."""
+    test_gather_small_batch_winners(kvops, req, top_k, dbs, stride_mode, fused, block_dim)
+
+
 @pytest.mark.parametrize("top_k", [1000, 3000])   # 3 x 1000 positions: one-launch form; 3 x 3000: two launches
 @pytest.mark.parametrize("fused", [False, True])    # import_seg per segment, or import_all
 def test_gather_rows_past_layer_region(kvops, top_k, fused):
