@@ -105,9 +105,17 @@ __device__ __forceinline__ void store_through(uint64_t addr, u32x4 v)
 }
 __device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" : : : "memory"); }
 
+// A status word cleared at the start of a launch: the last workgroup's word
+// follows it (its ticket comes after the clearing workgroup's wait).
+__device__ __forceinline__ void clear_status(uint64_t addr)
+{
+    __hip_atomic_store(reinterpret_cast<uint64_t *>(addr), 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Copy `n` rows whose byte addresses sit in src[0..n), dst[0..n) (LDS or
 // global) with the whole wave: chunk c covers bytes [16*(c%cpr), +16) of row
 // c/cpr.  kUnroll loads are issued before their stores.
+template <bool kThrough = false>
 __device__ __forceinline__ void wave_copy_rows(const uint64_t *src, const uint64_t *dst, uint32_t n, uint32_t cpr)
 {
     const uint32_t total = n * cpr;
@@ -128,7 +136,9 @@ __device__ __forceinline__ void wave_copy_rows(const uint64_t *src, const uint64
         }
 #pragma unroll
         for (int j = 0; j < kUnroll; ++j) {
-            if (d[j] != 0) __builtin_nontemporal_store(v[j], reinterpret_cast<GVec *>(d[j]));
+            if (d[j] == 0) continue;
+            if constexpr (kThrough) store_through(d[j], v[j]);
+            else __builtin_nontemporal_store(v[j], reinterpret_cast<GVec *>(d[j]));
         }
     }
 }
@@ -368,7 +378,7 @@ __global__ __launch_bounds__(kOneThreads) void kvx_gather_one(GatherParams P)
     const uint32_t total = static_cast<uint32_t>(numReal) * a.topK;  // (host: below 2^31)
     if (blockIdx.x == 0 && a.status != 0) {  // the call's status words read 0 until its rows have landed
         for (uint32_t i = tid; i < (n1 - n0) * x.statusWords; i += kOneThreads) {
-            store_status(a.status + (n0 + i / x.statusWords) * 64ull + (i % x.statusWords) * 8ull, 0ull);
+            clear_status(a.status + (n0 + i / x.statusWords) * 64ull + (i % x.statusWords) * 8ull);
         }
     }
     for (uint32_t i = n0 * 8u + tid; i < n1 * 8u; i += kOneThreads) {
@@ -523,7 +533,10 @@ __global__ __launch_bounds__(kOneThreads) void kvx_gather_one(GatherParams P)
 }
 
 // Prefill export: item (layer l, owned stripe i) copies the stripe's winning
-// row (its highest row inside the range) to segment row q/N of layer l.
+// row (its highest row inside the range) to segment row q/N of layer l.  Rows
+// are stored through the caches: with a system-scope fence per workgroup, each
+// a write-back of an XCD's L2, 144 MB took 2751 us, now 2534 (56.9 GB/s of the
+// link's 57.0); 32 workgroups take 2592.
 __global__ __launch_bounds__(256) void kvx_export_alllayer(ExportParams P)
 {
     __shared__ uint64_t sSrc[kWaves][64];
@@ -551,11 +564,11 @@ __global__ __launch_bounds__(256) void kvx_export_alllayer(ExportParams P)
         }
         wave_sync_lds();
         const uint64_t left = items - base;
-        wave_copy_rows(sSrc[wave], sDst[wave], static_cast<uint32_t>(left < 64ull ? left : 64ull), cpr);
+        wave_copy_rows<true>(sSrc[wave], sDst[wave], static_cast<uint32_t>(left < 64ull ? left : 64ull), cpr);
         wave_sync_lds();
     }
 
-    __threadfence_system();
+    wait_stores();
     __syncthreads();
     if (threadIdx.x == 0) {
         const unsigned int ticket = atomicInc(&x.tickets[1], gridDim.x - 1u);
@@ -563,7 +576,6 @@ __global__ __launch_bounds__(256) void kvx_export_alllayer(ExportParams P)
     }
     __syncthreads();
     if (!sLast || a.status == 0) return;
-    __threadfence_system();
     const uint32_t words = a.blockDim == 0 ? 1u : a.blockDim;
     for (uint32_t b = threadIdx.x; b < words; b += blockDim.x) {
         uint64_t word = 1ull << 32;  // kvc_scatter_rows_alllayer.cpp:59-61
@@ -684,11 +696,11 @@ __global__ __launch_bounds__(256) void kvx_export_rows_copy(ExportRowsParams P)
             sDst[wave][at] = dst;
         }
         wave_sync_lds();
-        wave_copy_rows(sSrc[wave], sDst[wave], static_cast<uint32_t>(__popcll(cm)), cpr);
+        wave_copy_rows<true>(sSrc[wave], sDst[wave], static_cast<uint32_t>(__popcll(cm)), cpr);
         wave_sync_lds();
     }
 
-    __threadfence_system();
+    wait_stores();
     __syncthreads();
     if (threadIdx.x == 0) {
         const unsigned int ticket = atomicInc(&P.tickets[2], gridDim.x - 1u);
@@ -720,133 +732,120 @@ __global__ __launch_bounds__(256) void kvx_export_rows_copy(ExportRowsParams P)
 }
 
 // Short exports (max_rows <= kExportSmallMax, the rows a decode step
-// appends): both passes in one launch.  A winner is the last entry on its
-// destination row.  Up to kExportSmallLds entries, every workgroup loads the
-// destinations of all entries into LDS and eight lanes per own entry look for
-// a later entry with the same destination (no device-scope atomics, no
-// fence); above that, every workgroup tags the winners of all entries (the
-// same atomicMax values, so the repeats are harmless) and reads its own
-// entries' tags.  Each workgroup counts the owned entries and the lowest
-// out-of-region entry per status word in its own LDS, then copies the
-// winners among its own 32 entries (8 per wave); the last workgroup (ticket)
-// advances the epoch and stores the status words from its counts.
+// appends): both passes in one launch.  Rows share a destination iff they lie
+// in one stripe, and the last entry wins: each workgroup takes a few entries
+// and looks for a later entry in the same stripe among all of them, counts its
+// own owned and out-of-region entries, and copies its winners with all lanes;
+// the last workgroup (ticket) stores the status words and leaves the call's
+// counters zeroed.  The bound is latency: three dependent reads, a row's way
+// over the link and back.  Entries go to many workgroups (4 each up to 1024:
+// 64 rows, one
+// layer: 9.7 us from 2 workgroups ending in system-scope fences, 7.2 now).
 constexpr uint32_t kExportSmallMax = 4096;
-constexpr uint32_t kExportSmallLds = 1024;
+constexpr uint32_t kExportSpanRows = 1024;  // up to here 4 entries a workgroup, else 16
+constexpr uint32_t kExportMaxSpan = 16;
 
 __global__ __launch_bounds__(256) void kvx_export_rows_small(ExportRowsParams P)
 {
-    __shared__ uint64_t sSrc[kWaves][64];
-    __shared__ uint64_t sDst[kWaves][64];
-    __shared__ uint32_t sCnt[64 * 8], sErr[64 * 8];
-    __shared__ uint64_t sDest[kExportSmallLds];  // destination of each entry (~0: none), for n <= kExportSmallLds
+    __shared__ uint64_t sSrc[kExportMaxSpan], sDst[kExportMaxSpan];
+    __shared__ uint64_t sKey[kExportMaxSpan];  // stripe of an own entry in the winner rule, else ~0
+    __shared__ uint32_t sLose, sN;             // sLose bit e: own entry e is not a winner
     __shared__ int sLast;
-    __shared__ uint32_t sEpoch, sLose;  // sLose bit e: own entry e is not a winner
     const ExportRowsArgs &a = P.a;
-    const int wave = threadIdx.x / 64;
-    const uint32_t lane = static_cast<uint32_t>(lane_id());
+    const uint32_t tid = threadIdx.x;
     const int32_t n = clamp_num_real(a.numReal, a.maxRows);  // <= kExportSmallMax (host)
     const KVX_G int64_t *idx = reinterpret_cast<const KVX_G int64_t *>(a.indicesHost);
     const uint32_t cpr = a.rowBytes / 16u;
     const uint32_t words = a.statusWords;
     const uint32_t ppc = (a.maxRows + words - 1u) / words;  // entries per status word
     const uint32_t n0 = a.fused ? 0u : a.myNode, n1 = a.fused ? a.nodeNum : a.myNode + 1u;
+    const int32_t span = a.maxRows <= kExportSpanRows ? 4 : static_cast<int32_t>(kExportMaxSpan);
+    const int32_t lo = static_cast<int32_t>(blockIdx.x) * span;
+    auto stripe = [&](int64_t row) {  // (the mapping is u32 math; a stripe of 0 rows is the identity)
+        const uint32_t r = static_cast<uint32_t>(row);
+        return static_cast<uint64_t>(a.stripeRows == 0u ? r : r / a.stripeRows);
+    };
     if (blockIdx.x == 0 && a.status != 0) {  // the call's status words read 0 until its rows have landed
-        for (uint32_t k = threadIdx.x; k < (n1 - n0) * words; k += blockDim.x) {
-            store_status(a.status + (n0 + k / words) * 64ull + (k % words) * 8ull, 0ull);
+        for (uint32_t k = tid; k < (n1 - n0) * words; k += blockDim.x) {
+            clear_status(a.status + (n0 + k / words) * 64ull + (k % words) * 8ull);
         }
     }
-    for (uint32_t k = threadIdx.x; k < 64u * 8u; k += blockDim.x) {
-        sCnt[k] = 0u;
-        sErr[k] = 0xFFFFFFFFu;  // lowest failing entry, min-reduced
+    if (tid == 0) sLose = sN = 0u;
+    uint32_t node = 0, segRow = 0;
+    bool owned = false, rule = false;
+    if (static_cast<int32_t>(tid) < span) {
+        const int32_t i = lo + static_cast<int32_t>(tid);
+        const int64_t row = i < n ? idx[i] : -1;
+        owned = export_row_target(a, row, node, segRow);
+        rule = owned && segRow < a.perLayerSegRows;
+        sKey[tid] = rule ? stripe(row) : ~0ull;
     }
-    if (threadIdx.x == 0) sEpoch = *P.epoch;
     __syncthreads();
-    const unsigned long long tagHi = static_cast<unsigned long long>(sEpoch) << 32;
-    // the destination of entry i when the winner rule applies to it, else ~0
-    auto entry_dest = [&](int32_t i) -> uint64_t {
-        uint32_t node, segRow;
-        if (!export_row_target(a, idx[i], node, segRow) || segRow >= a.perLayerSegRows) return ~0ull;
-        const uint64_t w = (a.fused ? static_cast<uint64_t>(node) * a.perLayerSegRows : 0ull) + segRow;
-        return w < P.winEntries ? w : ~0ull;
-    };
-    const int32_t first = static_cast<int32_t>(blockIdx.x) * kWaves * kExportRowsPerWave;  // own entries: 32 from here
-    const bool inLds = n <= static_cast<int32_t>(kExportSmallLds);
-    if (inLds) {
-        for (int32_t i = threadIdx.x; i < n; i += blockDim.x) sDest[i] = entry_dest(i);
-        if (threadIdx.x == 0) sLose = 0u;
-        __syncthreads();
-        // lanes 8e .. 8e+7: own entry first + e against the later entries
-        const int32_t e = static_cast<int32_t>(threadIdx.x >> 3), i = first + e;
-        bool later = false;
-        if (i < n) {
-            const uint64_t w = sDest[i];
-            if (w != ~0ull) {
-                for (int32_t j = i + 1 + static_cast<int32_t>(threadIdx.x & 7u); j < n; j += 8) later |= sDest[j] == w;
+    uint32_t lose = 0u;
+    for (int32_t i0 = lo + static_cast<int32_t>(tid); i0 < n; i0 += 4 * 256) {
+        int64_t row[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) row[j] = idx[min(i0 + j * 256, n - 1)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int32_t i = i0 + j * 256;
+            if (i >= n || row[j] < 0) continue;
+            const uint64_t q = stripe(row[j]);
+            for (int32_t e = 0; e < span && lo + e < i; ++e) lose |= sKey[e] == q ? 1u << e : 0u;
+        }
+    }
+    if (lose != 0u) atomicOr(&sLose, lose);
+    __syncthreads();
+    if (owned) {
+        const uint32_t i = static_cast<uint32_t>(lo) + tid, key = node * 8u + i / ppc;
+        atomicAdd(&P.counters[key], 1u);
+        if (!rule) {
+            atomicMax(&P.errs[key], ~i);  // the lowest failing entry
+        } else if (((sLose >> tid) & 1u) == 0u) {
+            const uint32_t at = atomicAdd(&sN, 1u);
+            sSrc[at] = a.srcLayerBase + static_cast<uint64_t>(i) * a.rowBytes;
+            sDst[at] = (a.fused ? export_seg_base(node) : a.segBase) +
+                       (static_cast<uint64_t>(a.layerId) * a.perLayerSegRows + segRow) * a.rowBytes;
+        }
+    }
+    __syncthreads();
+    const uint32_t chunks = sN * cpr;
+    for (uint32_t c0 = tid; c0 < chunks; c0 += 256u * 4u) {
+        u32x4 v[4];
+        uint64_t d[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t c = c0 + static_cast<uint32_t>(j) * 256u;
+            d[j] = 0;
+            if (c < chunks) {
+                const uint32_t r = c / cpr, o = (c - r * cpr) * 16u;
+                v[j] = __builtin_nontemporal_load(reinterpret_cast<const GVec *>(sSrc[r] + o));
+                d[j] = sDst[r] + o;
             }
         }
-        const uint64_t m = __ballot(later);
-        if ((threadIdx.x & 7u) == 0u && ((m >> lane) & 0xFFull) != 0ull) atomicOr(&sLose, 1u << e);
-    } else {
-        for (int32_t i = threadIdx.x; i < n; i += blockDim.x) {
-            const uint64_t w = entry_dest(i);
-            if (w != ~0ull) win_max(P.win + w, tagHi | static_cast<unsigned long long>(i));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (d[j] != 0) store_through(d[j], v[j]);
         }
-        __threadfence();
     }
+    wait_stores();
     __syncthreads();
-    for (int32_t i = threadIdx.x; i < n; i += blockDim.x) {
-        uint32_t node, segRow;
-        if (!export_row_target(a, idx[i], node, segRow)) continue;
-        const uint32_t key = node * 8u + static_cast<uint32_t>(i) / ppc;
-        atomicAdd(&sCnt[key], 1u);
-        if (segRow >= a.perLayerSegRows) atomicMin(&sErr[key], static_cast<uint32_t>(i));
-    }
-    constexpr int32_t R = kExportRowsPerWave;
-    {
-        const int32_t i = (static_cast<int32_t>(blockIdx.x) * kWaves + wave) * R + static_cast<int32_t>(lane);
-        bool copy = false;
-        uint64_t src = 0, dst = 0;
-        uint32_t node, segRow;
-        if (static_cast<int32_t>(lane) < R && i < n && export_row_target(a, idx[i], node, segRow) &&
-            segRow < a.perLayerSegRows) {
-            const uint64_t w = (a.fused ? static_cast<uint64_t>(node) * a.perLayerSegRows : 0ull) + segRow;
-            copy = w >= P.winEntries || (inLds ? ((sLose >> (i - first)) & 1u) == 0u
-                                               : win_load(P.win + w) == (tagHi | static_cast<unsigned long long>(i)));
-            src = a.srcLayerBase + static_cast<uint64_t>(i) * a.rowBytes;
-            dst = (a.fused ? export_seg_base(node) : a.segBase) +
-                  (static_cast<uint64_t>(a.layerId) * a.perLayerSegRows + segRow) * a.rowBytes;
-        }
-        const uint64_t cm = __ballot(copy);
-        if (copy) {
-            const uint32_t at = static_cast<uint32_t>(__popcll(cm & ((1ull << lane) - 1ull)));
-            sSrc[wave][at] = src;
-            sDst[wave][at] = dst;
-        }
-        wave_sync_lds();
-        wave_copy_rows(sSrc[wave], sDst[wave], static_cast<uint32_t>(__popcll(cm)), cpr);
-    }
-    __threadfence_system();
-    __syncthreads();
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
         const unsigned int ticket = atomicInc(&P.tickets[4], gridDim.x - 1u);
         sLast = (ticket == gridDim.x - 1u) ? 1 : 0;
     }
     __syncthreads();
     if (!sLast) return;
-    if (sEpoch + 1u == 0u) {  // at the wrap (once in 2^32 calls) the tag table is cleared
-        for (uint64_t k = threadIdx.x; k < P.winEntries; k += blockDim.x) P.win[k] = 0ull;
-    }
-    if (threadIdx.x == 0) *P.epoch = sEpoch + 1u;
-    if (a.status == 0) return;
-    __threadfence_system();
-    for (uint32_t k = threadIdx.x; k < (n1 - n0) * words; k += blockDim.x) {
-        const uint32_t node = n0 + k / words, b = k % words;
+    for (uint32_t k = tid; k < (n1 - n0) * 8u; k += blockDim.x) {
+        const uint32_t nd = n0 + k / 8u, b = k % 8u;
+        const uint32_t q = __hip_atomic_load(&P.counters[nd * 8u + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t e = __hip_atomic_load(&P.errs[nd * 8u + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (q != 0u) __hip_atomic_store(&P.counters[nd * 8u + b], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (e != 0u) __hip_atomic_store(&P.errs[nd * 8u + b], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (a.status == 0 || b >= words) continue;
         uint64_t word = 1ull << 32;
-        if (static_cast<int64_t>(b) * ppc < n) {
-            const uint32_t e = sErr[node * 8u + b];
-            word |= (static_cast<uint64_t>(sCnt[node * 8u + b]) << 40) | (e == 0xFFFFFFFFu ? 0u : row_error_code(e));
-        }
-        store_status(a.status + node * 64ull + b * 8ull, word);
+        if (static_cast<int64_t>(b) * ppc < n) word |= (static_cast<uint64_t>(q) << 40) | (e == 0u ? 0u : row_error_code(~e));
+        store_status(a.status + nd * 64ull + b * 8ull, word);
     }
 }
 
@@ -961,7 +960,8 @@ hipError_t launch_export_rows(const ExportRowsArgs &a, const uint64_t *segBases,
     P.tickets = scr.tickets;
     P.epoch = scr.epoch;
     if (a.maxRows <= kExportSmallMax) {
-        const uint32_t blocks = (a.maxRows + kExportRowsPerWave * kWaves - 1u) / (kExportRowsPerWave * kWaves);
+        const uint32_t span = a.maxRows <= kExportSpanRows ? 4u : kExportMaxSpan;
+        const uint32_t blocks = (a.maxRows + span - 1u) / span;
         hipLaunchKernelGGL(kvx_export_rows_small, dim3(blocks), dim3(256), 0, stream, P);
         return hipGetLastError();
     }

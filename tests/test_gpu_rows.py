@@ -338,8 +338,8 @@ def test_export_rows_parity(kvops, S, N, block_dim, max_rows, num_real, fused):
     outside the layer region (reported, not written), num_real below the
     capacity; all segment bytes and every node's status words.  Up to 4096
     entries the export is one launch, above it two (the 5000-entry case); the
-    one launch decides winners in LDS up to 1024 entries and by device-scope
-    tags above (the 2900-entry case)."""
+    one launch takes 4 entries a workgroup up to 1024 entries and 16 above
+    (the 2900-entry case)."""
     print("export_rows case", S, N, block_dim, max_rows, num_real, fused, flush=True)
     L, layer_rows = 3, 4096
     pool = HostSegPool(0, L, layer_rows, ROW, stripe_rows=S, node_num=N)
