@@ -105,7 +105,7 @@ __host__ __device__ __forceinline__ uint64_t export_rows_win_entries(uint32_t pe
 constexpr int kFastThreads = KVX_FAST_THREADS;
 
 struct FastLayout {
-    uint32_t tok, ht, vis, ptok, pinf, vt, evslot, smKp, eseq, tb, smA, smB, vset, ber, occ, fin, nkb, cmask, emask,
+    uint32_t tok, ht, vis, ptok, pinf, vt, evslot, smKp, eseq, tb, smA, smB, vset, ber, occ, fin, rnk, cmask, emask,
         smask, rsn, rsm, total;
 };
 
@@ -119,9 +119,10 @@ __host__ __device__ __forceinline__ uint32_t align16(uint32_t x) { return (x + 1
 // replaced by the Knuth hash of each slot's token (full tokens stay in HBM),
 // and the per-slot first-hit codes (vt) take 16 bits instead of 32.
 // cmask/emask/smask/rsn/rsm hold one 64-bit ballot per (wave, block of one
-// entry per lane).  ber, occ, fin and nkb are one bit per table cell: cells
-// of evicted tokens, the pre-step occupancy, the occupancy as the erase and
-// insert phases change it, and the cells new keys claim.
+// entry per lane).  ber, occ and fin are one bit per table cell: cells of
+// evicted tokens, the pre-step occupancy, the occupancy as the erase changes
+// it.  rnk: the event order of up to 64 slots (rows decided in registers).
+constexpr uint32_t kRankBytes = 64u * 2u;
 __host__ __device__ __forceinline__ FastLayout fast_layout(uint32_t padded, uint32_t htSize, uint32_t topK,
                                                            uint32_t visStrideB, bool compact = false)
 {
@@ -152,7 +153,7 @@ __host__ __device__ __forceinline__ FastLayout fast_layout(uint32_t padded, uint
     l.rsn = o;     o += ringMaskBytes;
     l.rsm = o;     o += ringMaskBytes;
     l.fin = o;     o += align16(bmBytes);
-    l.nkb = o;     o += align16(bmBytes);
+    l.rnk = o;     o += kRankBytes;
     l.total = o;
     return l;
 }
@@ -200,14 +201,13 @@ __host__ __device__ __forceinline__ FastLayout fast_layout_fixed(uint32_t padded
     l.vis = o;     o += align16(visStrideB);
     l.ber = o;     o += align16(htSize / 8u);
     l.occ = o;     o += align16(htSize / 8u);
-    // the two table bitmaps of the insert phases take the per-position
-    // classes' region, which the fixed kernels keep in registers instead
-    if (2u * align16(htSize / 8u) <= Kx * 4u) {
+    // the bitmap that the erase changes takes the per-position classes'
+    // region, which the fixed kernels keep in registers instead
+    l.rnk = o;     o += kRankBytes;
+    if (align16(htSize / 8u) <= Kx * 4u) {
         l.fin = l.pinf;
-        l.nkb = l.pinf + align16(htSize / 8u);
     } else {
         l.fin = o;  o += align16(htSize / 8u);
-        l.nkb = o;  o += align16(htSize / 8u);
     }
     l.total = o;
     return l;

@@ -43,13 +43,13 @@
 //   outputs  slots, is_miss, visited bits; erase the evicted tokens
 //            (Algorithm R deletions commute when each pre-step cluster is
 //            done right to left by its rightmost marked cell)
-//   insert   tentative parallel placement of the new tokens (the occupied
-//            cells do not depend on order), entries naming the event; a key
-//            alone in its final cluster takes its cell, and every other
-//            cluster is redone in event order by one wave (a lane per cell).  Linear probing
-//            with Algorithm R leaves the table equal to inserting the live
-//            keys in insertion order, so the result is the sequential table
-//            byte for byte.
+//   insert   the new tokens' keys propose to the cells the survivors leave
+//            free, from their home on, all at once; a cell keeps the earliest
+//            event's key and the other goes on.  First-come-first-served
+//            linear probing is the stable matching that finds, whatever the
+//            order of the proposals, and Algorithm R leaves the table equal to
+//            inserting the live keys in insertion order, so the result is the
+//            sequential table byte for byte.
 //
 // Shape preconditions, checked by the launcher: padded + 1 + topK <= 65535,
 // topK < 16383, dbs <= 32 * 1024, htSize <= 32768.  State preconditions,
@@ -123,7 +123,7 @@ __device__ unsigned long long kvx_dbg_sub[1024][16];
 struct Misc {
     unsigned long long evMask;  // in-order path: the events that placed a slot's final token
     int32_t nEv, handOut;
-    int32_t bad, ovf, late, nSM, nUnd, uEnd, nTakes, nLead, nDone, snNext;
+    int32_t bad, ovf, late, nSM, nUnd, uEnd, nTakes, nDone, snNext;
     int32_t diff;  // live tokens minus table entries
     uint32_t fp0, fpd;  // the staged tokens' fingerprint; its change by the step's new tokens
     uint32_t M;    // candidates (first occurrences of missing tokens)
@@ -245,23 +245,6 @@ __device__ __forceinline__ void lds_min16(uint32_t *w32, uint32_t i, uint16_t v)
         if (prev == old) return;
         old = prev;
     }
-}
-
-// Claim the first free cell at or after `idx` in an occupancy bitmap (one
-// bit per cell) with an atomic OR per try; a failed try moves to the next
-// free cell the returned word shows.  Bits are only set while claims run, so
-// every cell from idx to the one returned was occupied when passed.  Returns
-// the cell, or -1 after a whole-table probe.
-__device__ __forceinline__ int32_t lds_claim_bit(uint32_t *bm, int32_t idx, int32_t mask)
-{
-    for (int32_t n = 0; n <= mask; ++n) {
-        const uint32_t b = static_cast<uint32_t>(idx) & 31u, bit = 1u << b;
-        const uint32_t old = atomicOr(bm + (idx >> 5), bit);
-        if (!(old & bit)) return idx;
-        const uint32_t fr = ~old & (0xFFFFFFFEu << b);  // free cells above b in the word
-        idx = fr ? ((idx & ~31) | __builtin_ctz(fr)) : (((idx | 31) + 1) & mask);
-    }
-    return -1;
 }
 
 // Algorithm R deletion of the entry at cell c (homes from the tokens row, or
@@ -408,7 +391,7 @@ __global__ __launch_bounds__(NT) void kvx_sieve_update_fast(KvxLaunch<HispSieveU
     }
     if (tid == 0) {  // ordered before every update by the barrier in the staging pass
         ms.bad = ms.ovf = ms.late = 0;
-        ms.nSM = ms.nUnd = ms.uEnd = ms.nTakes = ms.nLead = ms.nDone = ms.snNext = 0;
+        ms.nSM = ms.nUnd = ms.uEnd = ms.nTakes = ms.nDone = ms.snNext = 0;
         ms.diff = 0;
         ms.fp0 = ms.fpd = 0u;
         ms.M = 0;
@@ -442,9 +425,9 @@ __global__ __launch_bounds__(NT) void kvx_sieve_update_fast(KvxLaunch<HispSieveU
     uint32_t *ber = reinterpret_cast<uint32_t *>(smem + lay.ber);   // cells of evicted tokens
     uint32_t *occ = reinterpret_cast<uint32_t *>(smem + lay.occ);   // occupied cells of the pre-step table
     uint8_t *occ8 = smem + lay.occ;
-    uint32_t *fin = reinterpret_cast<uint32_t *>(smem + lay.fin);   // occupied cells as erase and claims change them
+    uint32_t *fin = reinterpret_cast<uint32_t *>(smem + lay.fin);   // occupied cells as the erase changes them
     uint8_t *fin8 = smem + lay.fin;
-    uint32_t *nkb = reinterpret_cast<uint32_t *>(smem + lay.nkb);   // cells claimed by new keys
+    uint16_t *evRank = reinterpret_cast<uint16_t *>(smem + lay.rnk);  // rows decided in registers: the slots' event order
     uint64_t *cmask = reinterpret_cast<uint64_t *>(smem + lay.cmask);  // first occurrences of candidates
     uint64_t *emask = reinterpret_cast<uint64_t *>(smem + lay.emask);  // conversion positions
     uint64_t *smask = reinterpret_cast<uint64_t *>(smem + lay.smask);  // evicted SM slots
@@ -456,7 +439,6 @@ __global__ __launch_bounds__(NT) void kvx_sieve_update_fast(KvxLaunch<HispSieveU
     uint32_t *pcell = smA;                                   // classify: provisional cell per position
     uint16_t *undl = eseq;                                   // decide: undecided SM indices
     uint32_t *ecell = smA;                                   // per event: table cell | slot << 16
-    uint16_t *lead = eseq;                                   // redo: start cell of each multi-key cluster
     int32_t *ntokv = reinterpret_cast<int32_t *>(smB);       // per event: the token inserted
     uint16_t *snList = evslot;                               // scan -> decide: the evicted SN slots in ring order
     uint16_t *smCell = smKp;                                 // events -> marks: table cell of each evicted SM slot
@@ -585,7 +567,7 @@ __global__ __launch_bounds__(NT) void kvx_sieve_update_fast(KvxLaunch<HispSieveU
     // event's slot loses, NOCELL for none, | slot << 16; ntokv[r]: the token
     // it gains, in event order): erase the lost tokens -- the rightmost
     // marked cell (ber) of each pre-step cluster (occ) leads it and deletes
-    // right to left -- then place the gained ones (claims, clusters, redo).
+    // right to left -- then place the gained ones.
     // setVset: also mark the events' slots visited in vset.  Sets ms.late on
     // a bound violation.  Every thread calls it.
     auto table_update = [&](int32_t Nev, bool setVset) {
@@ -648,206 +630,78 @@ __global__ __launch_bounds__(NT) void kvx_sieve_update_fast(KvxLaunch<HispSieveU
         }
         __syncthreads();
         STAMP(7);
-        // ---- new tokens; tentative placement (the final occupied cells do
-        // not depend on order), entries padded+1+r name the event; the
-        // fingerprint's change (each event's slot loses one token, gains one)
+        // ---- new tokens: each event's key proposes to the cells from its
+        // home that the survivors leave free (fin); a cell keeps the earliest
+        // event's key and the one it gives up goes on to the next such cell
+        // (the stable matching of sequential inserts, found in any order of
+        // the proposals).  The entries are final at once: the slot says the
+        // event's order, its ring offset or (rows decided in registers, whose
+        // hand may turn) its entry of evRank.  Also the fingerprint's change
+        // (each event's slot loses one token, gains one)
         uint32_t fpd = 0;
+        auto order = [&](uint32_t s) -> uint32_t {
+            if (!setVset) return evRank[s & 63u];
+            const int32_t x = static_cast<int32_t>(s) - hand0;
+            return static_cast<uint32_t>(x < 0 ? x + dbs : x);
+        };
+        uint32_t *ht32 = reinterpret_cast<uint32_t *>(ht);
         for (int32_t q = 0; q < Pn; ++q) {
             const int32_t r = tid + q * NT;
             if (r >= Nev) break;
             const uint32_t s = ((q == 0) ? ecR : ecell[r]) >> 16;
             const int32_t t = ntokv[r];
-            int32_t old;
+            int32_t c = static_cast<int32_t>(ht_hash(t)) & mask;
+            // the home's word of the bitmap and of the table, read together
+            uint32_t fw = fin[c >> 5], old = ht32[c >> 1];
+            int32_t was;
             if constexpr (kC) {
-                old = (q == 0) ? oldR : gTok[s];
+                was = (q == 0) ? oldR : gTok[s];
                 hv[s] = static_cast<uint16_t>(ht_hash(t) & static_cast<uint32_t>(mask));
                 gTok[s] = t;
             } else {
-                old = tok[s];
+                was = tok[s];
                 tok[s] = t;
             }
-            fpd += slot_token_mix(s, t) - slot_token_mix(s, old);
-            const int32_t c = lds_claim_bit(fin, static_cast<int32_t>(ht_hash(t)) & mask, mask);
-            if (c < 0) {
-                g.code = kOverflowProbe;
-                continue;
+            fpd += slot_token_mix(s, t) - slot_token_mix(s, was);
+            uint32_t mine = s + 1u, myOrder = order(s);
+            bool read = true;  // old is the word of cell c
+            for (int32_t n = 0;; ++n) {
+                if (n > 4 * H) {  // a full table: only a corrupted one
+                    g.code = kOverflowProbe;
+                    break;
+                }
+                const uint32_t fr = ~fw & (0xFFFFFFFFu << (c & 31));  // free cells of the word from c on
+                if (fr == 0u) {
+                    c = ((c | 31) + 1) & mask;
+                    fw = fin[c >> 5];
+                    read = false;
+                    continue;
+                }
+                const int32_t y = (c & ~31) | __builtin_ctz(fr);
+                if (y != c || !read) old = ht32[y >> 1];
+                c = y;
+                read = true;
+                const uint32_t sh = (static_cast<uint32_t>(c) & 1u) * 16u, cur = (old >> sh) & 0xFFFFu;
+                uint32_t curOrder = 0xFFFFFFFFu;
+                if (cur != 0u) curOrder = order(cur - 1u);
+                if (curOrder > myOrder) {
+                    const uint32_t prev = atomicCAS(ht32 + (c >> 1), old, (old & ~(0xFFFFu << sh)) | (mine << sh));
+                    if (prev != old) {  // the word changed: look again
+                        old = prev;
+                        continue;
+                    }
+                    if (cur == 0u) break;
+                    mine = cur;
+                    myOrder = curOrder;
+                }
+                c = (c + 1) & mask;
+                if ((c & 31) == 0) fw = fin[c >> 5];
+                read = false;
             }
-            ht[c] = static_cast<uint16_t>(padded + 1 + r);
-            atomicOr(nkb + (c >> 5), 1u << (c & 31));
-            ecell[r] = static_cast<uint32_t>(c) | (s << 16);
-            if (q == 0) ecR = static_cast<uint32_t>(c) | (s << 16);
         }
         {
             const uint32_t fw = wave_sum(fpd);
             if (lane == 0 && fw != 0u) atomicAdd(&ms.fpd, fw);
-        }
-        __syncthreads();
-        STAMP(8);
-        // ---- final cluster of each new key, from the bitmaps: the leftmost
-        // new key of a cluster leads it; alone, the key takes its cell, with
-        // others the leader queues the cluster's start for the redo
-        const int32_t wmask = (H >> 5) - 1;
-        for (int32_t q = 0; q < Pn; ++q) {
-            const int32_t r = tid + q * NT;
-            if (r >= Nev) break;
-            const uint32_t ec = (q == 0) ? ecR : ecell[r];
-            const int32_t c = static_cast<int32_t>(ec & 0xFFFFu) & mask;  // in range even after a failed claim
-            // the bitmap words either side of c, read together
-            const int32_t wl = ((c - 1) & mask) >> 5, wr = ((c + 1) & mask) >> 5;
-            const uint32_t fL = fin[wl], nL = nkb[wl], fR = fin[wr], nR = nkb[wr];
-            asm volatile("" : : "v"(fL), "v"(nL), "v"(fR), "v"(nR));
-            // leftwards from c - 1 to the cluster's start: a new key on the
-            // way leads instead
-            int32_t st = -1;
-            bool leads = true;
-            {
-                int32_t w = wl;
-                uint32_t keep = (2u << ((c - 1) & 31)) - 1u, fw = fL, nw0 = nL;  // bits 0..(c-1)&31
-                for (int32_t n = 0; n <= wmask; ++n) {
-                    if (n > 0) {
-                        fw = fin[w];
-                        nw0 = nkb[w];
-                    }
-                    const uint32_t empt = ~fw & keep, nw = nw0 & keep;
-                    const int32_t hiE = empt ? 31 - __builtin_clz(empt) : -1;
-                    const uint32_t after = (hiE >= 0) ? (nw & ~((2u << hiE) - 1u)) : nw;
-                    if (after) {
-                        leads = false;
-                        break;
-                    }
-                    if (hiE >= 0) {
-                        st = ((w << 5) + hiE + 1) & mask;
-                        break;
-                    }
-                    w = (w - 1) & wmask;
-                    keep = 0xFFFFFFFFu;
-                }
-            }
-            if (!leads) continue;
-            if (st < 0) {
-                g.code = kOverflowProbe;
-                continue;
-            }
-            // rightwards from c + 1 to the cluster's end: another new key
-            bool alone = true;
-            {
-                int32_t w = wr;
-                uint32_t sel = 0xFFFFFFFFu << ((c + 1) & 31), fw = fR, nw = nR;
-                for (int32_t n = 0; n <= wmask; ++n) {
-                    if (n > 0) {
-                        fw = fin[w];
-                        nw = nkb[w];
-                    }
-                    const uint32_t empt = ~fw & sel;
-                    const uint32_t before = empt ? ((1u << __builtin_ctz(empt)) - 1u) : 0xFFFFFFFFu;
-                    if (nw & sel & before) {
-                        alone = false;
-                        break;
-                    }
-                    if (empt) break;
-                    w = (w + 1) & wmask;
-                    sel = 0xFFFFFFFFu;
-                }
-            }
-            if (alone) ht[c] = static_cast<uint16_t>((ec >> 16) + 1u);
-            else lead[atomicAdd(&ms.nLead, 1)] = static_cast<uint16_t>(st);
-        }
-        if (g.code) atomicOr(&ms.late, 1);
-        __syncthreads();
-        STAMP(9);
-        // ---- redo: insert the cluster's new keys in event order.  The cells
-        // still holding padded+1+r' are exactly the ones empty when the next
-        // key is inserted, so key r probes from its home to the first of them
-        // and swaps in; the key it displaces keeps its event number.  One
-        // wave per cluster, a lane per cell (longer clusters: one lane).
-        const int32_t nLead = ms.nLead;
-        const int32_t st0 = lead[wave];  // read with nLead; used only when wave < nLead
-        if (nLead == 0) return;
-        for (int32_t li = wave; li < nLead; li += NWAVES) {
-            const int32_t st = (li == wave) ? st0 : lead[li];
-            const int32_t x = (st + static_cast<int32_t>(lane)) & mask;
-            uint32_t e = ht[x];
-            const uint64_t empt = __ballot(e == 0u);
-            if (empt != 0ull) {
-                const int32_t Lc = __builtin_ctzll(empt);  // cluster length
-                bool un = static_cast<int32_t>(lane) < Lc && e > static_cast<uint32_t>(padded);
-                // each unprocessed key's home (offset from st) and final
-                // entry, read once; they move with the key when it is displaced
-                int32_t hoff = 0;
-                uint32_t fe = 0;
-                if (un) {
-                    const uint32_t rr = e - static_cast<uint32_t>(padded) - 1u;
-                    hoff = ((static_cast<int32_t>(ht_hash(ntokv[rr])) & mask) - st) & mask;
-                    fe = (ecell[rr] >> 16) + 1u;
-                }
-                const uint64_t um0 = __ballot(un);
-                if (__popcll(um0) == 2) {
-                    // two keys at a < b: the earlier event's key takes the
-                    // first of them at or after its home, the other the rest
-                    const int32_t a = __builtin_ctzll(um0), b = 63 - __builtin_clzll(um0);
-                    const uint32_t ea = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(e), a));
-                    const uint32_t eb = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(e), b));
-                    const uint32_t fa = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(fe), a));
-                    const uint32_t fb = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(fe), b));
-                    const int32_t x0 = (ea < eb) ? a : b;
-                    const int32_t hX = __builtin_amdgcn_readlane(hoff, x0);
-                    const int32_t f = (hX <= a) ? a : (hX <= b) ? b : x0;
-                    const uint32_t fX = (x0 == a) ? fa : fb, fY = (x0 == a) ? fb : fa;
-                    if (static_cast<int32_t>(lane) == a) e = (f == a) ? fX : fY;
-                    if (static_cast<int32_t>(lane) == b) e = (f == b) ? fX : fY;
-                    un = false;
-                }
-                for (int32_t it = 0; it < 64; ++it) {
-                    uint64_t um = __ballot(un);
-                    if (um == 0ull) break;
-                    uint32_t best = 0xFFFFFFFFu;
-                    int32_t cm = 0;
-                    for (; um != 0ull; um &= um - 1ull) {
-                        const int32_t l = __builtin_ctzll(um);
-                        const uint32_t v = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(e), l));
-                        if (v < best) {
-                            best = v;
-                            cm = l;
-                        }
-                    }
-                    const int32_t hl = __builtin_amdgcn_readlane(hoff, cm);
-                    const uint32_t fv = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(fe), cm));
-                    const uint64_t fm = __ballot(un && static_cast<int32_t>(lane) >= hl);
-                    const int32_t f = fm ? __builtin_ctzll(fm) : cm;  // the home lies in the cluster
-                    const uint32_t ef = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(e), f));
-                    const int32_t hf = __builtin_amdgcn_readlane(hoff, f);
-                    const uint32_t ff = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(fe), f));
-                    if (static_cast<int32_t>(lane) == cm) {
-                        e = ef;
-                        hoff = hf;
-                        fe = ff;
-                    }
-                    if (static_cast<int32_t>(lane) == f) {
-                        e = fv;
-                        un = false;
-                    }
-                }
-                if (static_cast<int32_t>(lane) < Lc) ht[x] = static_cast<uint16_t>(e);
-            } else if (lane == 0) {
-                for (int32_t it = 0; it < H; ++it) {
-                    uint32_t mn = 0xFFFFFFFFu;
-                    int32_t cm = -1;
-                    int32_t y = st;
-                    for (int32_t n = 0; n < H && ht[y] != 0; ++n, y = (y + 1) & mask) {
-                        const uint32_t ey = ht[y];
-                        if (ey > static_cast<uint32_t>(padded) && ey < mn) {
-                            mn = ey;
-                            cm = y;
-                        }
-                    }
-                    if (cm < 0) break;
-                    const uint32_t rr = mn - static_cast<uint32_t>(padded) - 1u;
-                    int32_t f = static_cast<int32_t>(ht_hash(ntokv[rr])) & mask;
-                    for (int32_t n = 0; n < H && ht[f] <= static_cast<uint32_t>(padded); ++n) f = (f + 1) & mask;
-                    ht[cm] = ht[f];
-                    ht[f] = static_cast<uint16_t>((ecell[rr] >> 16) + 1u);
-                }
-            }
         }
         if (g.code) atomicOr(&ms.late, 1);
         __syncthreads();
@@ -967,7 +821,6 @@ __global__ __launch_bounds__(NT) void kvx_sieve_update_fast(KvxLaunch<HispSieveU
         for (int32_t i = tid; i < vsetWords; i += NT) vset[i] = 0u;
         for (int32_t i = tid; i < (H >> 5); i += NT) {
             ber[i] = 0u;
-            nkb[i] = 0u;
         }
         for (int32_t i = tid; i < 2 * P * NWAVES; i += NT) emask[i] = 0ull;  // emask, smask (adjacent)
         const int32_t dw = static_cast<int32_t>(wave_sum(nTok)) - static_cast<int32_t>(wave_sum(nEnt));
@@ -1048,6 +901,7 @@ __global__ __launch_bounds__(NT) void kvx_sieve_update_fast(KvxLaunch<HispSieveU
             if (alive) {
                 ecell[rank] = cell_of(static_cast<int32_t>(lane)) | (lane << 16);  // the pre-step token's cell
                 ntokv[rank] = tokFin;
+                evRank[lane] = static_cast<uint16_t>(rank);
             }
             if (static_cast<int32_t>(lane) < (dbs + 7) / 8) {  // visited bytes of slots [0, dbs)
                 const int32_t b0 = static_cast<int32_t>(lane) * 8;
