@@ -274,8 +274,12 @@ __host__ __device__ __forceinline__ BatchLayout batch_layout(uint32_t dbs, uint3
 //   newk [H/2]         new keys in event order: (home << 16) | (slot + 1)
 //   evict [H/32]       the step's evicted slots (bitmap)
 //   chunkA [H/kTblChunkCells]  per cell chunk: start of its cluster, or -1
-constexpr uint32_t kTblChunkCells = 256;     // survivors' cells per chunk
-constexpr uint32_t kTblChunkKeys = 256;      // new keys per chunk
+//   (cellw and chunkA hold min(H, kTblCells) cells)
+constexpr uint32_t kTblChunkCells = 1024;    // survivors' cells per chunk
+constexpr uint32_t kTblChunkKeys = 1024;     // new keys per chunk
+// A hash has 16 bits, so homes lie in the first 2^16 cells, and fewer than
+// 2^16 keys run past them: cells from 2^17 on are never taken.
+constexpr uint32_t kTblCells = 1u << 17;
 constexpr uint32_t kTblWinBits = 3u << 16;   // free-cell window of a chunk (bits)
 constexpr uint32_t kTblMaxHt = 1u << 18;     // largest table the rebuild takes
 

@@ -377,7 +377,7 @@ __global__ __launch_bounds__(kCellThreads) void kvx_sieve_table_cells(TblParams 
     KVX_GM uint32_t *hist = tb + P.t.hist;
     const KVX_GM uint32_t *evict = tb + P.t.evict;
     const uint32_t c8 = blockIdx.x * kCellThreads + threadIdx.x;  // 8 cells
-    if (c8 * 8u < H) {
+    if (c8 * 8u < (H < kTblCells ? H : kTblCells)) {
         const u32x4 v = reinterpret_cast<const KVX_GM u32x4 *>(ht)[c8];
         const uint32_t w[4] = {v.x, v.y, v.z, v.w};
         uint32_t out[8];
@@ -436,15 +436,65 @@ __device__ __forceinline__ int32_t block_scan_max(int32_t v, int32_t *sPart)
     return inc > before ? inc : before;
 }
 
-constexpr uint32_t kTblChunks = kTblMaxHt / kTblChunkCells;  // chunks of the largest table
+constexpr uint32_t kTblChunks = kTblCells / kTblChunkCells;
+
+// The per-home counts in LDS: 16 bits a home, eight homes a 16-byte chunk.  A
+// thread scans 64 or more homes in a row, so lanes read chunks 8 or more
+// apart: the chunk's low bits are exchanged with those of the thread, which
+// spreads a wave's reads over the banks (in plain order they meet on two
+// chunk columns in sixteen).
+__device__ __forceinline__ uint32_t swz8(uint32_t chunk) { return chunk ^ ((chunk >> 4) & 7u); }
+__device__ __forceinline__ uint32_t swz_word(uint32_t i) { return (swz8(i >> 3) << 2) + ((i >> 1) & 3u); }  // word of count i
+__device__ __forceinline__ void counts8(const uint32_t *hist, uint32_t i, int32_t *c)  // counts i .. i+7, i a multiple of 8
+{
+    const uint4 v = reinterpret_cast<const uint4 *>(hist)[swz8(i >> 3)];
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+        c[2 * h] = static_cast<int32_t>(w[h] & 0xFFFFu);
+        c[2 * h + 1] = static_cast<int32_t>(w[h] >> 16);
+    }
+}
+__device__ __forceinline__ int32_t count1(const uint32_t *hist, uint32_t i)
+{
+    return static_cast<int32_t>((hist[swz_word(i)] >> (16u * (i & 1u))) & 0xFFFFu);
+}
+
+// The counts of homes [0, HH) from HBM (32 bits each) into LDS, eight a lane
+// at a time, four of those in flight.  HH a multiple of 8.
+__device__ __forceinline__ void load_counts(uint32_t *hist, const KVX_GM uint32_t *src, uint32_t HH)
+{
+    constexpr uint32_t U = 4;
+    const KVX_GM u32x4 *s4 = reinterpret_cast<const KVX_GM u32x4 *>(src);
+    for (uint32_t i0 = threadIdx.x; i0 < HH / 8u; i0 += U * kTT) {
+        u32x4 a[U], b[U];
+#pragma unroll
+        for (uint32_t q = 0; q < U; ++q) {
+            const uint32_t i = i0 + q * kTT < HH / 8u ? i0 + q * kTT : i0;
+            a[q] = s4[2u * i];
+            b[q] = s4[2u * i + 1u];
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < U; ++q) {
+            const uint32_t i = i0 + q * kTT;
+            if (i >= HH / 8u) break;
+            reinterpret_cast<uint4 *>(hist)[swz8(i)] =
+                make_uint4((a[q].x & 0xFFFFu) | (a[q].y << 16), (a[q].z & 0xFFFFu) | (a[q].w << 16),
+                           (b[q].x & 0xFFFFu) | (b[q].y << 16), (b[q].z & 0xFFFFu) | (b[q].w << 16));
+        }
+    }
+}
+
+constexpr uint32_t kFinalLdsBytes = 65536u * 2u + kTblCells / 8u;  // counts, cells taken before the step
 
 __global__ __launch_bounds__(kTT) void kvx_sieve_table_final(TblParams P)
 {
+    extern __shared__ __align__(16) unsigned char lds[];
     __shared__ MP sPart[kTW + 1];
     __shared__ int32_t sMax[kTW];
     __shared__ int32_t sE, sEAligned;
-    // per chunk of 256 cells (table order): the last empty cell, the last
-    // deleted cell (offsets in the chunk, -1 = none), and whether a survivor is there
+    // per chunk of cells (table order): the last empty cell, the last deleted
+    // cell (offsets in the chunk, -1 = none), and whether a survivor is there
     __shared__ int32_t sLastEmpty[kTblChunks], sLastDel[kTblChunks];
     __shared__ uint32_t sSurv[kTblChunks];
     const HispSieveUpdateArgs &a = P.L.a;
@@ -452,103 +502,120 @@ __global__ __launch_bounds__(kTT) void kvx_sieve_table_final(TblParams P)
     if (bid >= static_cast<int32_t>(a.maxNumReqs)) return;
     KVX_GM uint32_t *tb = row_tbl(P, bid);
     if (tb[P.t.meta] != 1u) return;
-    const uint32_t H = a.htSize, mask = H - 1u, HH = H < 65536u ? H : 65536u;
+    const uint32_t H = a.htSize, mask = H - 1u, HH = H < 65536u ? H : 65536u, C = H < kTblCells ? H : kTblCells;
     const int64_t reqIdx = reinterpret_cast<const KVX_GM int64_t *>(a.reqPoolIndices)[bid];
     KVX_GM uint16_t *ht = reinterpret_cast<KVX_GM uint16_t *>(a.deviceBufferHt) + reqIdx * H;
     const KVX_GM uint32_t *cellw = tb + P.t.cellw;
-    const KVX_GM uint32_t *hist = tb + P.t.hist;
-    const uint32_t tid = threadIdx.x;
-    const uint32_t S = H / kTT;  // cells per thread (H >= 1024, a power of two: S a power of two)
-    const uint32_t c0 = tid * S;
-    const uint32_t nC = H / kTblChunkCells;
-    // cells go four at a time (16-byte loads) when a thread has at least four
-    const uint32_t step = S >= 4u ? 4u : S;
-    auto load = [&](const KVX_GM uint32_t *a4, uint32_t x, uint32_t *out) {
-        if (step == 4u) {
-            const u32x4 v = reinterpret_cast<const KVX_GM u32x4 *>(a4)[x >> 2];
-            out[0] = v.x;
-            out[1] = v.y;
-            out[2] = v.z;
-            out[3] = v.w;
-        } else {
-            for (uint32_t h = 0; h < step; ++h) out[h] = a4[x + h];
-        }
-    };
-    auto cnts = [&](uint32_t x, uint32_t *out) {  // counts of cells x .. x + step - 1
-        if (x < HH) {
-            load(hist, x, out);
-        } else {
-            for (uint32_t h = 0; h < 4u; ++h) out[h] = 0u;
-        }
-    };
-
-    // the cells occupied after the step, cyclic: the backlog entering cell 0
-    // is the fixed point of the whole ring's map, max(p, b + q) with q < 0
-    // (fewer keys than cells), i.e. p
-    MP m{kNegInf, 0};
-    if (c0 >= HH) {
-        m = MP{0, -static_cast<int32_t>(S)};  // no keys homed here
-    } else {
-        for (uint32_t x = c0; x < c0 + S; x += step) {
-            uint32_t n[4];
-            cnts(x, n);
-            for (uint32_t h = 0; h < step; ++h) m = mp_then(m, mp_cell(static_cast<int32_t>(n[h])));
-        }
-    }
-    MP total;
-    const MP ex = block_scan_mp(m, total, sPart);
-    if (tid == 0) {
-        sE = 0x7FFFFFFF;
-        sEAligned = 0x7FFFFFFF;
-    }
+    const uint32_t tid = threadIdx.x, lane = static_cast<uint32_t>(__lane_id());
+    const uint32_t nC = C / kTblChunkCells;
+    uint32_t *hist = reinterpret_cast<uint32_t *>(lds);
+    uint8_t *taken8 = lds + 65536u * 2u;  // cells taken before the step, 8 a byte
     for (uint32_t i = tid; i < nC; i += kTT) {
         sLastEmpty[i] = -1;
         sLastDel[i] = -1;
         sSurv[i] = 0u;
     }
+    if (tid == 0) {
+        sE = 0x7FFFFFFF;
+        sEAligned = 0x7FFFFFFF;
+    }
+    load_counts(hist, tb + P.t.hist, HH);
     __syncthreads();
-    int32_t b = mp_apply(ex, total.p > 0 ? total.p : 0);
-    int32_t eMin = 0x7FFFFFFF, eAl = 0x7FFFFFFF;
-    // this thread's chunk statistics (one chunk at a time; S and 256 are powers of two)
-    int32_t le = -1, ld = -1;
-    uint32_t sv = 0u, g = c0 / kTblChunkCells;
-    for (uint32_t x = c0; x < c0 + S; x += step) {
-        uint32_t nn[4], ww[4];
-        cnts(x, nn);
-        load(cellw, x, ww);
-        for (uint32_t h = 0; h < step; ++h) {
-            const uint32_t c = x + h;
-            const int32_t n = static_cast<int32_t>(nn[h]);
-            const bool occ = b + n >= 1;
-            b = b + n - 1 > 0 ? b + n - 1 : 0;
-            const uint32_t cw = ww[h];
-            if (cw != 0u && !occ) ht[c] = 0;  // occupied before the step, empty after
-            if (cw == 0u && !occ && (H <= 65536u || c >= 65535u)) {
-                if (static_cast<int32_t>(c) < eMin) eMin = static_cast<int32_t>(c);
-                if ((c & (kTblChunkCells - 1u)) == kTblChunkCells - 1u && static_cast<int32_t>(c) < eAl)
-                    eAl = static_cast<int32_t>(c);
-            }
-            const int32_t off = static_cast<int32_t>(c & (kTblChunkCells - 1u));
-            if (cw == 0u) le = off;
-            else if (cw == kDeleted) ld = off;
-            else sv = 1u;
+    // the statistics of eight cells (positions or cells i*8 .. i*8+7), merged
+    // per chunk (whole waves lie in one chunk or the chunk is a whole table)
+    auto stats = [&](uint32_t i, uint32_t empt, uint32_t del, uint32_t surv, bool on) {
+        int32_t le = on && empt ? static_cast<int32_t>((i * 8u) % kTblChunkCells) + 31 - __builtin_clz(empt) : -1;
+        int32_t ld = on && del ? static_cast<int32_t>((i * 8u) % kTblChunkCells) + 31 - __builtin_clz(del) : -1;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int32_t x = __shfl_xor(le, d), y = __shfl_xor(ld, d);
+            le = x > le ? x : le;
+            ld = y > ld ? y : ld;
         }
-        if (((x + step) & (kTblChunkCells - 1u)) == 0u || x + step == c0 + S) {
-            // the chunk ends (or this thread's part of it): publish
+        const uint64_t sm = __ballot(on && surv != 0u);
+        if (lane == 0u && on) {
+            const uint32_t g = i * 8u / kTblChunkCells;
             if (le >= 0) atomicMax(&sLastEmpty[g], le);
             if (ld >= 0) atomicMax(&sLastDel[g], ld);
-            if (sv) sSurv[g] = 1u;
-            le = -1;
-            ld = -1;
-            sv = 0u;
-            g = (x + step) / kTblChunkCells;
+            if (sm != 0ull) sSurv[g] = 1u;
         }
+    };
+    {
+        constexpr uint32_t U = 4;  // eights of cells in flight per lane
+        const KVX_GM u32x4 *c4 = reinterpret_cast<const KVX_GM u32x4 *>(cellw);
+        for (uint32_t i0 = tid; i0 - lane < C / 8u; i0 += U * kTT) {
+            u32x4 x[U], y[U];
+#pragma unroll
+            for (uint32_t q = 0; q < U; ++q) {
+                const uint32_t i = i0 + q * kTT < C / 8u ? i0 + q * kTT : 0u;
+                x[q] = c4[2u * i];
+                y[q] = c4[2u * i + 1u];
+            }
+#pragma unroll
+            for (uint32_t q = 0; q < U; ++q) {
+                const uint32_t i = i0 + q * kTT;
+                if (i - lane >= C / 8u) break;
+                const uint32_t w[8] = {x[q].x, x[q].y, x[q].z, x[q].w, y[q].x, y[q].y, y[q].z, y[q].w};
+                uint32_t taken = 0, del = 0;
+#pragma unroll
+                for (int h = 0; h < 8; ++h) {
+                    taken |= (w[h] != 0u ? 1u : 0u) << h;
+                    del |= (w[h] == kDeleted ? 1u : 0u) << h;
+                }
+                const bool on = i < C / 8u;
+                if (on) taken8[i] = static_cast<uint8_t>(taken);
+                stats(i, ~taken & 0xFFu, del, taken & ~del, on);
+            }
+        }
+    }
+    __syncthreads();
+    // The cells taken after the step.  A table of up to 65536 cells is cyclic:
+    // the backlog entering cell 0 is the fixed point of the whole ring's map,
+    // max(p, b + q) with q < 0 (fewer keys than cells), i.e. p.  In a larger
+    // one nothing wraps: the backlog leaving cell 65535 takes the cells after
+    // it, one each.
+    const uint32_t S = HH / kTT, c0 = tid * S;  // homes per thread: 1 to 64
+    auto each = [&](auto f) {
+        if (S >= 8u) {
+            for (uint32_t x = c0; x < c0 + S; x += 8u) {
+                int32_t n[8];
+                counts8(hist, x, n);
+#pragma unroll
+                for (int h = 0; h < 8; ++h) f(x + static_cast<uint32_t>(h), n[h]);
+            }
+        } else {
+            for (uint32_t x = c0; x < c0 + S; ++x) f(x, count1(hist, x));
+        }
+    };
+    MP m{kNegInf, 0};
+    each([&](uint32_t, int32_t n) { m = mp_then(m, mp_cell(n)); });
+    MP total;
+    const MP ex = block_scan_mp(m, total, sPart);
+    const bool wraps = H <= 65536u;
+    int32_t b = mp_apply(ex, wraps && total.p > 0 ? total.p : 0);
+    int32_t eMin = 0x7FFFFFFF, eAl = 0x7FFFFFFF;
+    each([&](uint32_t c, int32_t n) {
+        const bool occ = b + n >= 1;
+        b = b + n - 1 > 0 ? b + n - 1 : 0;
+        if (occ) return;
+        if ((taken8[c >> 3] >> (c & 7u)) & 1u) {
+            ht[c] = 0;  // taken before the step, empty after
+        } else if (wraps) {
+            if (static_cast<int32_t>(c) < eMin) eMin = static_cast<int32_t>(c);
+            if ((c & (kTblChunkCells - 1u)) == kTblChunkCells - 1u && static_cast<int32_t>(c) < eAl) eAl = static_cast<int32_t>(c);
+        }
+    });
+    if (!wraps) {
+        const uint32_t out = static_cast<uint32_t>(mp_apply(total, 0));  // keys past cell 65535
+        for (uint32_t c = HH + out + tid; c < C && ((taken8[c >> 3] >> (c & 7u)) & 1u); c += kTT) ht[c] = 0;
     }
     if (eMin != 0x7FFFFFFF) atomicMin(&sE, eMin);
     if (eAl != 0x7FFFFFFF) atomicMin(&sEAligned, eAl);
     __syncthreads();
-    // the order starts after e; one that ends a chunk keeps the chunks whole
-    const int32_t e = sEAligned != 0x7FFFFFFF ? sEAligned : sE;
+    // the order starts after e, a cell empty before and after; one that ends a
+    // chunk keeps the chunks whole (in a larger table the last cell does)
+    const bool aligned = !wraps || sEAligned != 0x7FFFFFFF;
+    const int32_t e = !wraps ? static_cast<int32_t>(H - 1u) : (aligned ? sEAligned : sE);
     if (e == 0x7FFFFFFF) {  // not reachable: fewer keys than cells leave one
         if (tid == 0) {
             report_overflow(P.L.overflowSlot, kOverflowProbe);
@@ -556,41 +623,29 @@ __global__ __launch_bounds__(kTT) void kvx_sieve_table_final(TblParams P)
         }
         return;
     }
-    if (sEAligned == 0x7FFFFFFF) {
+    if (!aligned) {
         // chunks of the cell order straddle the table's: count them again in
         // positions (position x is cell (x + e + 1) mod H)
-        __syncthreads();
         for (uint32_t i = tid; i < nC; i += kTT) {
             sLastEmpty[i] = -1;
             sLastDel[i] = -1;
             sSurv[i] = 0u;
         }
         __syncthreads();
-        le = -1;
-        ld = -1;
-        sv = 0u;
-        g = c0 / kTblChunkCells;
-        for (uint32_t x = c0; x < c0 + S; ++x) {
-            const uint32_t cw = cellw[(x + static_cast<uint32_t>(e) + 1u) & mask];
-            const int32_t off = static_cast<int32_t>(x & (kTblChunkCells - 1u));
-            if (cw == 0u) le = off;
-            else if (cw == kDeleted) ld = off;
-            else sv = 1u;
-            if (((x + 1u) & (kTblChunkCells - 1u)) == 0u || x + 1u == c0 + S) {
-                if (le >= 0) atomicMax(&sLastEmpty[g], le);
-                if (ld >= 0) atomicMax(&sLastDel[g], ld);
-                if (sv) sSurv[g] = 1u;
-                le = -1;
-                ld = -1;
-                sv = 0u;
-                g = (x + 1u) / kTblChunkCells;
+        for (uint32_t i = tid; i - lane < C / 8u; i += kTT) {
+            uint32_t taken = 0, del = 0;
+            for (uint32_t h = 0; h < 8u; ++h) {
+                const uint32_t cw = cellw[(i * 8u + h + static_cast<uint32_t>(e) + 1u) & mask];
+                taken |= (cw != 0u ? 1u : 0u) << h;
+                del |= (cw == kDeleted ? 1u : 0u) << h;
             }
+            stats(i, ~taken & 0xFFu, del, taken & ~del, i < C / 8u);
         }
         __syncthreads();
     }
     // position chunk q is table chunk (q + shift) mod nC (shift 0 when the
     // order does not start at a chunk boundary: the statistics were counted in positions)
-    const uint32_t shift = sEAligned != 0x7FFFFFFF ? ((static_cast<uint32_t>(e) + 1u) / kTblChunkCells) % nC : 0u;
+    const uint32_t shift = aligned ? ((static_cast<uint32_t>(e) + 1u) & mask) / kTblChunkCells : 0u;
     // a chunk's cluster starts after the last empty cell before it; its
     // survivors can move only if a deleted cell lies between that start and
     // the chunk's end
@@ -609,9 +664,9 @@ __global__ __launch_bounds__(kTT) void kvx_sieve_table_final(TblParams P)
     // the last empty cell strictly before chunk q: the inclusive max of chunk q - 1
     const int32_t lePrev = __shfl_up(leInc, 1);
     __shared__ int32_t sWaveLast[kTW];
-    if ((tid & 63u) == 63u) sWaveLast[tid >> 6] = leInc;
+    if (lane == 63u) sWaveLast[tid >> 6] = leInc;
     __syncthreads();
-    const int32_t leBefore = (tid & 63u) ? lePrev : (tid >= 64u ? sWaveLast[(tid >> 6) - 1u] : -1);
+    const int32_t leBefore = lane ? lePrev : (tid >= 64u ? sWaveLast[(tid >> 6) - 1u] : -1);
     if (q < nC) {
         const int32_t start = leBefore + 1;
         KVX_GM int32_t *chunkA = reinterpret_cast<KVX_GM int32_t *>(tb + P.t.chunkA);
@@ -791,6 +846,36 @@ __device__ __forceinline__ void match_cells(const PlaceLds &L, uint32_t n)
     __syncthreads();
 }
 
+// L.home[0, n) in increasing order to L.sortedH, one key per thread, all ones
+// past n: a bitonic sort, the exchanges between lanes of a wave by shuffles.
+__device__ __forceinline__ void sort_homes(const PlaceLds &L, uint32_t n)
+{
+    const uint32_t tid = threadIdx.x;
+    uint32_t v = tid < n ? L.home[tid] : 0xFFFFFFFFu;
+    uint32_t *buf = L.sortedH, *alt = L.z;  // exchanged by turns, one barrier each
+    for (uint32_t k = 2; k <= kTblChunkCells; k <<= 1) {
+        for (uint32_t j = k >> 1; j != 0u; j >>= 1) {
+            uint32_t o;
+            if (j >= 64u) {
+                buf[tid] = v;
+                __syncthreads();
+                o = buf[tid ^ j];
+                uint32_t *x = buf;
+                buf = alt;
+                alt = x;
+            } else {
+                o = static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), static_cast<int>(j)));
+            }
+            const bool up = (tid & k) == 0u, low = (tid & j) == 0u;
+            v = (low == up) == (v > o) ? o : v;
+        }
+    }
+    __syncthreads();
+    L.sortedH[tid] = v;
+    __syncthreads();
+}
+static_assert(kTblChunkCells == kTT && kTblChunkKeys == kTT, "one key of a chunk per thread");
+
 // All threads; the items are in L.home/ent/own [0, n).  Returns through L.res
 // the window cell of each item.  False: a key found no cell (not reachable).
 __device__ bool place_chunk(const PlaceLds &L, const uint64_t *win, uint32_t n, MP *sPart, int32_t *sMax)
@@ -830,17 +915,8 @@ __device__ bool place_chunk(const PlaceLds &L, const uint64_t *win, uint32_t n, 
     }
     __syncthreads();
     const uint32_t totalFree = L.rank[kTblWinWords];
-    // homes in order (ties by insertion order)
-    if (tid < n) {
-        const uint32_t h = L.home[tid];
-        uint32_t rk = 0;
-        for (uint32_t j = 0; j < n; ++j) {
-            const uint32_t hj = L.home[j];
-            rk += (hj < h || (hj == h && j < tid)) ? 1u : 0u;
-        }
-        L.sortedH[rk] = h;
-    }
-    __syncthreads();
+    // homes in order
+    sort_homes(L, n);
     // r_j = j + max_{i<=j} (p_i - i)
     int32_t v = -0x3FFFFFFF;
     if (tid < n) {
@@ -912,43 +988,40 @@ __global__ __launch_bounds__(kTT) void kvx_sieve_table_chunks(TblParams P)
     KVX_GM uint16_t *ht = reinterpret_cast<KVX_GM uint16_t *>(a.deviceBufferHt) + reqIdx * H;
     const KVX_GM uint32_t *cellw = tb + P.t.cellw;
     const uint32_t tid = threadIdx.x, lane = __lane_id();
-    const uint32_t nS = H / kTblChunkCells;
+    // the last chunks first: they count the most keys before them
+    const uint32_t blk = gridDim.x - 1u - blockIdx.x;
+    const uint32_t nS = (H < kTblCells ? H : kTblCells) / kTblChunkCells;
     auto tab = [&](uint32_t x) { return (x + e + 1u) & mask; };  // position -> cell
     auto pos = [&](uint32_t c) { return (c - e - 1u) & mask; };  // cell -> position
-    auto count16 = [&](uint32_t i) { return static_cast<int32_t>((hist[i >> 1] >> (16u * (i & 1u))) & 0xFFFFu); };
-    auto count8from = [&](uint32_t i, int32_t *c) {  // counts i .. i+7, i a multiple of 8
-        const uint4 v = *reinterpret_cast<const uint4 *>(hist + (i >> 1));
-        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-            c[2 * h] = static_cast<int32_t>(w[h] & 0xFFFFu);
-            c[2 * h + 1] = static_cast<int32_t>(w[h] >> 16);
-        }
-    };
 #ifdef KVX_BATCH_STAMPS
     uint64_t t0 = __builtin_amdgcn_s_memtime(), t1 = 0, t2 = 0;
 #endif
     uint32_t wb = 0, n = 0;
-    bool survivors = blockIdx.x < nS;
+    bool survivors = blk < nS;
     uint32_t s0 = 0;
     if (survivors) {
         // survivors of positions [s0, s0 + 256), after those of [A, s0) in the same cluster
-        const int32_t a0 = reinterpret_cast<const KVX_GM int32_t *>(tb + P.t.chunkA)[blockIdx.x];
+        const int32_t a0 = reinterpret_cast<const KVX_GM int32_t *>(tb + P.t.chunkA)[blk];
         if (a0 < 0) return;
-        s0 = blockIdx.x * kTblChunkCells;
+        s0 = blk * kTblChunkCells;
         const uint32_t s1 = s0 + kTblChunkCells;
         const uint32_t A = static_cast<uint32_t>(a0);
         wb = A & ~63u;
         const uint32_t nh = s0 - wb;  // counted positions [wb, s0), by position - wb
         uint32_t cw = 0u;
         if (tid < kTblChunkCells) cw = cellw[tab(s0 + tid)];
-        for (uint32_t i = tid; i < (nh + 1u) / 2u + 4u; i += kTT) hist[i] = 0u;
+        for (uint32_t i = tid; i < nh / 8u; i += kTT) reinterpret_cast<uint4 *>(hist)[i] = make_uint4(0, 0, 0, 0);
         __syncthreads();
-        for (uint32_t x = A + tid; x < s0; x += kTT) {
-            const uint32_t c = cellw[tab(x)];
-            if ((c & 0xFFFFu) == 0u) continue;  // empty or deleted
-            const uint32_t i = pos(c >> 16) - wb;
-            if (i < nh) atomicAdd(&hist[i >> 1], 1u << (16u * (i & 1u)));
+        for (uint32_t x = A + tid; x < s0; x += 8u * kTT) {
+            uint32_t c[8];
+#pragma unroll
+            for (uint32_t q = 0; q < 8u; ++q) c[q] = x + q * kTT < s0 ? cellw[tab(x + q * kTT)] : 0u;
+#pragma unroll
+            for (uint32_t q = 0; q < 8u; ++q) {
+                if ((c[q] & 0xFFFFu) == 0u) continue;  // empty or deleted
+                const uint32_t i = pos(c[q] >> 16) - wb;
+                if (i < nh) atomicAdd(&hist[swz_word(i)], 1u << (16u * (i & 1u)));
+            }
         }
         __syncthreads();
 #ifdef KVX_BATCH_STAMPS
@@ -957,7 +1030,7 @@ __global__ __launch_bounds__(kTT) void kvx_sieve_table_chunks(TblParams P)
         chunk_free_cells(wb, s1, wb, win,
                          [&](uint32_t x, int32_t *c) {
                              if (x < s0) {
-                                 count8from(x - wb, c);
+                                 counts8(hist, x - wb, c);
                              } else {
 #pragma unroll
                                  for (int h = 0; h < 8; ++h) c[h] = 0;
@@ -986,34 +1059,32 @@ __global__ __launch_bounds__(kTT) void kvx_sieve_table_chunks(TblParams P)
         __syncthreads();
     } else {
         // new keys [j0, j1), after every survivor and the new keys before j0
-        const uint32_t j0 = (blockIdx.x - nS) * kTblChunkKeys;
+        const uint32_t j0 = (blk - nS) * kTblChunkKeys;
         if (j0 >= N) return;
         const uint32_t j1 = j0 + kTblChunkKeys < N ? j0 + kTblChunkKeys : N;
         const KVX_GM uint32_t *newk = tb + P.t.newk;
         const KVX_GM uint32_t *histAll = tb + P.t.hist;
         if (tid == 0) sLo = 0x7FFFFFFF;
-        for (uint32_t i = tid; i < HH / 2u; i += kTT) hist[i] = (histAll[2u * i] & 0xFFFFu) | (histAll[2u * i + 1u] << 16);
+        load_counts(hist, histAll, HH);
         __syncthreads();
         for (uint32_t j = j0 + tid; j < N; j += kTT) {
             const uint32_t h = newk[j] >> 16;
-            atomicSub(&hist[h >> 1], 1u << (16u * (h & 1u)));
+            atomicSub(&hist[swz_word(h)], 1u << (16u * (h & 1u)));
             if (j < j1) atomicMin(&sLo, static_cast<int32_t>(pos(h)));
         }
         __syncthreads();
         wb = static_cast<uint32_t>(sLo) & ~63u;
-        // homes lie in cells [0, HH): positions [pos(0), pos(0) + HH) (the order
-        // starts past 65535 when the table is larger)
-        const uint32_t x0 = H > 65536u ? (pos(0) & ~63u) : 0u;
+        const uint32_t x0 = 0u;  // (a larger table's order starts at its first cell)
         const bool aligned = ((e + 1u) & 7u) == 0u;  // positions of 8 cells then read 8 counts at once
 #ifdef KVX_BATCH_STAMPS
         t1 = __builtin_amdgcn_s_memtime();
 #endif
-        chunk_free_cells(x0, H, wb, win,
+        chunk_free_cells(x0, H < kTblCells ? H : kTblCells, wb, win,
                          [&](uint32_t x, int32_t *c) {
                              const uint32_t c0 = tab(x);
                              if (aligned) {
                                  if (c0 < HH) {
-                                     count8from(c0, c);
+                                     counts8(hist, c0, c);
                                  } else {
 #pragma unroll
                                      for (int h = 0; h < 8; ++h) c[h] = 0;
@@ -1022,7 +1093,7 @@ __global__ __launch_bounds__(kTT) void kvx_sieve_table_chunks(TblParams P)
 #pragma unroll
                                  for (int h = 0; h < 8; ++h) {
                                      const uint32_t ch = tab(x + static_cast<uint32_t>(h));
-                                     c[h] = ch < HH ? count16(ch) : 0;
+                                     c[h] = ch < HH ? count1(hist, ch) : 0;
                                  }
                              }
                          },
@@ -1053,8 +1124,8 @@ __global__ __launch_bounds__(kTT) void kvx_sieve_table_chunks(TblParams P)
         }
     }
 #ifdef KVX_BATCH_STAMPS
-    if (tid == 0 && bid == 0 && (blockIdx.x & 31u) == 0u)
-        printf("chunk %u n %u: hist %llu scan %llu place %llu\n", blockIdx.x, n, (unsigned long long)(t1 - t0),
+    if (tid == 0 && bid == 0 && (blk & 7u) == 0u)
+        printf("chunk %u n %u: hist %llu scan %llu place %llu\n", blk, n, (unsigned long long)(t1 - t0),
                (unsigned long long)(t2 - t1), (unsigned long long)(__builtin_amdgcn_s_memtime() - t2));
 #endif
 }
@@ -1065,8 +1136,11 @@ constexpr uint32_t kLocalLds(uint32_t cells) { return cells * 2u + cells / 4u + 
 
 hipError_t sieve_table_set_lds_limit(size_t bytes)
 {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&kvx_sieve_table_local),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&kvx_sieve_table_local),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kLocalLds(kLocalCells)));
+    if (e != hipSuccess) return e;
+    e = hipFuncSetAttribute(reinterpret_cast<const void *>(&kvx_sieve_table_final),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kFinalLdsBytes));
     if (e != hipSuccess) return e;
     return hipFuncSetAttribute(reinterpret_cast<const void *>(&kvx_sieve_table_chunks),
                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes));
@@ -1079,12 +1153,13 @@ hipError_t launch_sieve_table_rebuild(const HispSieveUpdateArgs &a, uint64_t ove
     P.L = KvxLaunch<HispSieveUpdateArgs>{a, overflowSlot};
     P.tbl = tbl;
     P.t = table_layout(a.htSize);
-    const uint32_t cellBlocks = (a.htSize + kCellsPerBlock - 1u) / kCellsPerBlock;
+    const uint32_t cells = a.htSize < kTblCells ? a.htSize : kTblCells;
+    const uint32_t cellBlocks = (cells + kCellsPerBlock - 1u) / kCellsPerBlock;
     const uint32_t localCells = a.htSize < kLocalCells ? a.htSize : kLocalCells;
     hipLaunchKernelGGL(kvx_sieve_table_local, dim3(a.maxNumReqs), dim3(kTT), kLocalLds(localCells), stream, P);
     hipLaunchKernelGGL(kvx_sieve_table_cells, dim3(cellBlocks, a.maxNumReqs), dim3(kCellThreads), 0, stream, P);
-    hipLaunchKernelGGL(kvx_sieve_table_final, dim3(a.maxNumReqs), dim3(kTT), 0, stream, P);
-    const uint32_t chunks = a.htSize / kTblChunkCells + (a.topK + kTblChunkKeys - 1u) / kTblChunkKeys;
+    hipLaunchKernelGGL(kvx_sieve_table_final, dim3(a.maxNumReqs), dim3(kTT), kFinalLdsBytes, stream, P);
+    const uint32_t chunks = cells / kTblChunkCells + (a.topK + kTblChunkKeys - 1u) / kTblChunkKeys;
     hipLaunchKernelGGL(kvx_sieve_table_chunks, dim3(chunks, a.maxNumReqs), dim3(kTT), kTblLdsBytes, stream, P);
     return hipGetLastError();
 }
