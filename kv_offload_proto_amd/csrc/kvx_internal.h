@@ -236,10 +236,11 @@ __host__ __device__ __forceinline__ FastLayout fast_layout_for(uint32_t padded, 
 constexpr int kBatchThreads = 1024;
 constexpr int kBatchWaves = kBatchThreads / 64;
 constexpr uint32_t kBatchStage = 4096;       // table cells staged per step of the deletion walk
+constexpr uint32_t kBatchLds = 154u * 1024u;  // dynamic LDS of the batch kernel (it keeps ~4.7 KiB of static LDS)
 constexpr uint32_t kBatchMapCap = 1u << 18;  // tokens the map holds (rows with larger tokens run in order)
 
 struct BatchLayout {
-    uint32_t vis, ev, del, slot, uni, uniL1, uniL2, stage, total;
+    uint32_t vis, ev, del, slot, uni, uniL1, uniL2, stage, evl, total;
 };
 
 __host__ __device__ __forceinline__ BatchLayout batch_layout(uint32_t dbs, uint32_t htSize, uint32_t topK)
@@ -259,6 +260,10 @@ __host__ __device__ __forceinline__ BatchLayout batch_layout(uint32_t dbs, uint3
     const uint32_t uniBytes = topK * 4u > bitBytes ? topK * 4u : bitBytes;
     o += align16(uniBytes);
     l.stage = o;  o += kBatchStage * 4u;
+    // the evicted slots in event order, where that still fits (0: searched for)
+    const uint32_t evl = align16(topK * 2u);
+    l.evl = o + evl <= kBatchLds ? o : 0u;
+    if (l.evl != 0u) o += evl;
     l.total = o;
     return l;
 }

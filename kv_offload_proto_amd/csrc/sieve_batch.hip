@@ -371,6 +371,7 @@ struct PdLds {
     uint32_t regABytes;
     unsigned char *regB;      // scratch (the walk's stage)
     uint32_t regBBytes;
+    uint16_t *evList;         // [topK] the evicted slots in event order, or null
 };
 
 __device__ __forceinline__ uint64_t low_bits(uint32_t n) { return n >= 64u ? ~0ull : ((1ull << n) - 1ull); }
@@ -399,30 +400,21 @@ __device__ __forceinline__ uint64_t ring_word(const uint64_t *bm, uint32_t j, ui
 }
 
 // Exclusive prefix sum of one value per thread of the block; total in *tot.
+// The waves' sums are scanned by every wave for itself (DPP: no LDS round
+// trips, one barrier before it and one that frees sPart; a serial pass of one
+// thread over the 16 sums and shuffles took ~3.5k cycles a call).
 __device__ __forceinline__ uint32_t block_exscan(uint32_t v, uint32_t *tot, uint32_t *sPart)
 {
-    const uint32_t lane = static_cast<uint32_t>(__lane_id()), wave = threadIdx.x >> 6;
-    uint32_t inc = v;
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t o = static_cast<uint32_t>(__shfl_up(static_cast<int>(inc), d));
-        if (lane >= static_cast<uint32_t>(d)) inc += o;
-    }
+    const uint32_t lane = static_cast<uint32_t>(__lane_id());
+    const int32_t wave = uniform32(static_cast<int32_t>(threadIdx.x >> 6));
+    const uint32_t inc = sieve::wave_incl_scan(v);
     if (lane == 63u) sPart[wave] = inc;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t run = 0;
-        for (int w = 0; w < kBatchWaves; ++w) {
-            const uint32_t x = sPart[w];
-            sPart[w] = run;
-            run += x;
-        }
-        sPart[kBatchWaves] = run;
-    }
+    const uint32_t w = sieve::wave_incl_scan(lane < static_cast<uint32_t>(kBatchWaves) ? sPart[lane] : 0u);
+    const uint32_t before = wave ? static_cast<uint32_t>(lane_value(static_cast<int32_t>(w), wave - 1)) : 0u;
+    *tot = static_cast<uint32_t>(lane_value(static_cast<int32_t>(w), kBatchWaves - 1));
     __syncthreads();
-    const uint32_t r = sPart[wave] + inc - v;
-    *tot = sPart[kBatchWaves];
-    __syncthreads();
-    return r;
+    return before + inc - v;
 }
 
 // Offset of the r-th set bit (r < popcount) of x.
@@ -635,7 +627,17 @@ __device__ __forceinline__ bool decide_parallel(const PdLds L, int32_t K, int32_
     if (tid < nP) ePre[tid] = eEx;
     __syncthreads();
     // 6. outputs: misses take the evicted slot of their rank; hits keep theirs
-    auto evictedSlot = [&](uint32_t r) {  // the r-th eviction in ring order
+    if (L.evList != nullptr) {
+        // the first E evictions, listed a ring word per thread (a search over
+        // the words per miss was ten dependent reads each)
+        uint64_t x = tid < nR ? snR[tid] : 0ull;
+        for (uint32_t r = evEx; x != 0ull && r < E; x &= x - 1ull, ++r) {
+            L.evList[r] = static_cast<uint16_t>(slotOf((tid << 6) + static_cast<uint32_t>(__builtin_ctzll(x))));
+        }
+        __syncthreads();
+    }
+    auto evictedSlot = [&](uint32_t r) -> uint32_t {  // the r-th eviction in ring order
+        if (L.evList != nullptr) return L.evList[r];
         uint32_t lo = 0, hi = nR;  // the last word whose prefix is <= r
         while (hi - lo > 1u) {
             const uint32_t mid = (lo + hi) >> 1;
@@ -729,7 +731,8 @@ __device__ __forceinline__ bool decide_parallel(const PdLds L, int32_t K, int32_
 __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
 {
     extern __shared__ __align__(16) unsigned char lds[];
-    __shared__ int32_t sScan[BT];
+    __shared__ int32_t sScan[128];  // the waves' counts: of a check's segments, of eight blocks of positions
+    static_assert(kBatchWaves * 8 == 128, "two counts per lane");
     __shared__ int32_t sBits;  // the pre-passes' bitmap form holds for the row
     __shared__ int32_t sRing;  // the hand made no full turn: the misses took their slots in ring order
     __shared__ int32_t sBad, sWrap, sLive, sOcc, sNamed, sNdel, sHand, sE0, sTableBad, sFirstMiss, sMisses;
@@ -1062,22 +1065,37 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
             }
         }
         __syncthreads();
-        for (int32_t k = tid; k < K; k += BT) {
-            if (code[k] != kNotRes) continue;
-            const int32_t t = rt[k];
-            if (t >= mapLim) {
-                sBad = 1;  // a token the map cannot hold: decided in order instead
-                continue;
+        for (int32_t k0 = tid; k0 < K; k0 += BT * kMapUnroll) {
+            // the tokens' first occurrences (and map entries), loads in flight together
+            int32_t tv[kMapUnroll];
+            uint32_t fv[kMapUnroll], mv[kMapUnroll];
+#pragma unroll
+            for (int q = 0; q < kMapUnroll; ++q) {
+                const int32_t k = k0 + q * BT;
+                const bool need = k < K && code[k] == kNotRes;
+                tv[q] = !need ? -1 : (k0 == tid ? tv0[q] : rt[k]);
             }
-            const int32_t f = K - static_cast<int32_t>(first[t]);
-            if (f < k) {
-                code[k] = kDup | static_cast<uint32_t>(f);
-            } else {
+#pragma unroll
+            for (int q = 0; q < kMapUnroll; ++q) {
+                const bool in = tv[q] >= 0 && tv[q] < mapLim;
+                fv[q] = in ? first[tv[q]] : 0u;
                 // a first occurrence still unresolved: with the bitmap, not
                 // resident; otherwise the map says
-                const uint32_t s0 = useBits ? 0u : map[t];
-                if (s0 != 0u) {
-                    code[k] = s0 - 1u;
+                mv[q] = in && !useBits ? map[tv[q]] : 0u;
+            }
+#pragma unroll
+            for (int q = 0; q < kMapUnroll; ++q) {
+                const int32_t k = k0 + q * BT;
+                if (tv[q] < 0) continue;
+                if (tv[q] >= mapLim) {
+                    sBad = 1;  // a token the map cannot hold: decided in order instead
+                    continue;
+                }
+                const int32_t f = K - static_cast<int32_t>(fv[q]);
+                if (f < k) {
+                    code[k] = kDup | static_cast<uint32_t>(f);
+                } else if (mv[q] != 0u) {
+                    code[k] = mv[q] - 1u;
                 } else {
                     atomicMin(&sFirstMiss, k);  // a first occurrence not resident: a miss
                 }
@@ -1100,7 +1118,8 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
     bool decided = false;
     if (canonical && sBad == 0 && sFirstMiss < K) {
         const PdLds pl{code, slotOut, visB, evB, reinterpret_cast<unsigned char *>(delB), nCellW * 8u,
-                       reinterpret_cast<unsigned char *>(stage), kBatchStage * 4u};
+                       reinterpret_cast<unsigned char *>(stage), kBatchStage * 4u,
+                       y.evl != 0u ? reinterpret_cast<uint16_t *>(lds + y.evl) : nullptr};
         int32_t ph = 0, pm = 0;
         decided = decide_parallel(pl, K, dbs, hand0, sFirstMiss, &ph, &pm);
         if (decided && tid == 0) {
@@ -1321,50 +1340,45 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
         // then the new tokens.
         KVX_GM uint64_t *ev64 = (KVX_GM uint64_t *)(tbl + P.t.evict);
         for (uint32_t w = tid; w < nVisW; w += BT) ev64[w] = evB[w];
-        // the misses' ranks in position order: a contiguous run of positions per thread
-        const int32_t per = (K + BT - 1) / BT;
-        const int32_t k0 = tid * per, k1 = k0 + per < K ? k0 + per : K;
-        int32_t cnt = 0;
-        for (int32_t k = k0; k < k1; ++k) cnt += (slotOut[k] & kMissBit) ? 1 : 0;
-        int32_t inc = cnt;
-        for (int d = 1; d < 64; d <<= 1) {
-            const int32_t o = __shfl_up(inc, d);
-            if (static_cast<int>(lane) >= d) inc += o;
-        }
-        if (lane == 63) sScan[tid >> 6] = inc;
-        __syncthreads();
-        if (tid == 0) {
-            int32_t run = 0;
-            for (int w = 0; w < kBatchWaves; ++w) {
-                const int32_t v = sScan[w];
-                sScan[w] = run;
-                run += v;
-            }
-        }
-        __syncthreads();
-        int32_t rank = sScan[tid >> 6] + inc - cnt;
+        // The misses' ranks in position order, up to kHandoff positions a
+        // thread at a time (a block of BT positions each): the waves' counts
+        // per block in LDS, then their tokens and their slots' old tokens
+        // loaded together before any store (each evicted slot is named once).
         KVX_GM uint32_t *newk = tbl + P.t.newk;
-        // 8 positions at a time: their tokens and their slots' old tokens
-        // are loaded before any store (each evicted slot is named once)
-        uint32_t fpd = 0;
-        for (int32_t kb = k0; kb < k1; kb += 8) {
-            uint32_t so[8];
-            int32_t tk[8], old[8];
+        constexpr int kHandoff = 8;
+        const int32_t wave = uniform32(tid >> 6);
+        uint32_t fpd = 0, ranked = 0;
+        for (int32_t kb = tid; kb - tid < K; kb += kHandoff * BT) {
+            uint32_t so[kHandoff], rank[kHandoff];
+            int32_t tk[kHandoff], old[kHandoff];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int32_t k = kb + q;
-                so[q] = k < k1 ? slotOut[k] : 0u;
+            for (int q = 0; q < kHandoff; ++q) {
+                const int32_t k = kb + q * BT;
+                so[q] = k < K ? slotOut[k] : 0u;
+                const uint64_t mm = __ballot((so[q] & kMissBit) != 0u);
+                rank[q] = static_cast<uint32_t>(__builtin_popcountll(mm & ((1ull << lane) - 1ull)));
+                if (lane == 0) sScan[q * kBatchWaves + wave] = __builtin_popcountll(mm);
                 tk[q] = (so[q] & kMissBit) ? rt[k] : 0;
                 old[q] = (so[q] & kMissBit) ? r.tok[so[q] & 0xFFFFu] : 0;
             }
+            __syncthreads();
+            const uint32_t c0 = sScan[2 * lane], c1 = sScan[2 * lane + 1];  // (kHandoff * kBatchWaves = 128 counts)
+            const uint32_t inc = sieve::wave_incl_scan(c0 + c1);
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
+            for (int q = 0; q < kHandoff; ++q) {
+                const int32_t e = q * kBatchWaves + wave;  // counts before entry e
+                const uint32_t half = static_cast<uint32_t>(lane_value(static_cast<int32_t>(inc), e >> 1));
+                const uint32_t hc1 = static_cast<uint32_t>(lane_value(static_cast<int32_t>(c1), e >> 1));
+                const uint32_t hc0 = static_cast<uint32_t>(lane_value(static_cast<int32_t>(c0), e >> 1));
+                rank[q] += ranked + half - hc1 - ((e & 1) ? 0u : hc0);
                 if (!(so[q] & kMissBit)) continue;
                 const uint32_t sl = so[q] & 0xFFFFu;
-                newk[rank++] = ((ht_hash(tk[q]) & mask) << 16) | (sl + 1u);
+                newk[rank[q]] = ((ht_hash(tk[q]) & mask) << 16) | (sl + 1u);
                 r.tok[sl] = tk[q];
                 fpd += slot_token_mix(sl, tk[q]) - slot_token_mix(sl, old[q]);
             }
+            ranked += static_cast<uint32_t>(lane_value(static_cast<int32_t>(inc), 63));
+            __syncthreads();
         }
         for (int d = 32; d > 0; d >>= 1) fpd += __shfl_xor(fpd, d);
         if (lane == 0 && fpd) atomicAdd(&sFpD, fpd);

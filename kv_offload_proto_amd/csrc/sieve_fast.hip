@@ -133,20 +133,6 @@ struct Misc {
 
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 
-// Inclusive prefix sum over the 64 lanes of a wave from DPP row shifts and
-// row broadcasts (no LDS round trips).  Call with the whole wave active.
-__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x)
-{
-    int v = static_cast<int>(x);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);   // row_shr:1
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);   // row_shr:2
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);   // row_shr:4
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);   // row_shr:8
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1, 3
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2, 3
-    return static_cast<uint32_t>(v);
-}
-
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v)
 {
     return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(wave_incl_scan(v)), 63));
