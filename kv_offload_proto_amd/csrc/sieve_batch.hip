@@ -471,19 +471,20 @@ __device__ __forceinline__ bool decide_parallel(const PdLds L, int32_t K, int32_
     // 1. positions from the first miss: non-resident first occurrences; the
     // slots hit by resident first occurrences (evB, zero until now)
     for (uint32_t w = tid; w < nP; w += BT) {
-        cB[w] = 0ull;
+        if (w < (k0 >> 6)) cB[w] = 0ull;
         eB[w] = 0ull;
     }
     if (tid == 0) {
         sRel = 0u;
         sNev = 0u;
     }
-    __syncthreads();
-    for (uint32_t k = k0 + tid; k < static_cast<uint32_t>(K); k += BT) {
-        const uint32_t c = L.code[k];
-        if (c == kNotRes) {
-            atomicOr(reinterpret_cast<unsigned long long *>(cB + (k >> 6)), 1ull << (k & 63u));
-        } else if (c != kInvalid && c != kExt && !(c & kDup)) {
+    // (a wave takes the 64 positions of a word, whose bits are its ballot)
+    for (uint32_t kw = (k0 & ~63u) + (tid & ~63u); kw < static_cast<uint32_t>(K); kw += BT) {
+        const uint32_t k = kw + lane;
+        const uint32_t c = k >= k0 && k < static_cast<uint32_t>(K) ? L.code[k] : kInvalid;
+        const uint64_t m = __ballot(c == kNotRes);
+        if (lane == 0u) cB[kw >> 6] = m;
+        if (c != kNotRes && c != kInvalid && c != kExt && !(c & kDup)) {
             atomicOr(reinterpret_cast<unsigned long long *>(L.evB + (c >> 6)), 1ull << (c & 63u));
         }
     }
@@ -1065,6 +1066,7 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
             }
         }
         __syncthreads();
+        int32_t miss0 = K;  // the lane's first miss
         for (int32_t k0 = tid; k0 < K; k0 += BT * kMapUnroll) {
             // the tokens' first occurrences (and map entries), loads in flight together
             int32_t tv[kMapUnroll];
@@ -1097,10 +1099,15 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
                 } else if (mv[q] != 0u) {
                     code[k] = mv[q] - 1u;
                 } else {
-                    atomicMin(&sFirstMiss, k);  // a first occurrence not resident: a miss
+                    miss0 = k < miss0 ? k : miss0;  // a first occurrence not resident: a miss
                 }
             }
         }
+        // one LDS atomic a wave: lanes on one address take turns (an atomic per
+        // miss: the kernel 68 us at 8192 positions, most of them misses; 49 so, 44
+        // with the bits of decide_parallel's position words from ballots)
+        for (int d = 32; d > 0; d >>= 1) miss0 = min(miss0, __shfl_xor(miss0, d));
+        if (lane == 0) atomicMin(&sFirstMiss, miss0);
         __syncthreads();
         // Up to the first miss every position is a hit (no slot has been
         // evicted yet): applied in parallel, a later occurrence taking its
