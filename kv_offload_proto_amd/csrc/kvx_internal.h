@@ -271,8 +271,7 @@ __host__ __device__ __forceinline__ BatchLayout batch_layout(uint32_t dbs, uint3
 // The table rebuild of a step with misses (sieve_table.hip): per batch row,
 // HBM scratch of its own (table_layout(H).words uint32 words a row; nothing in
 // it needs to start zeroed, every launch writes what it reads):
-//   meta [16]          0: rebuild pending, 1: new keys, 2: linearization cell,
-//                      3: the events took their slots in ring order, 4: from this hand
+//   meta [16]          0: rebuild pending, 1: new keys, 2: linearization cell
 //   cellw [H]          per cell of the pre-step table: 0 empty, 0xFFFF0000 a
 //                      deleted key, else (home << 16) | entry of a survivor
 //   hist [min(H,2^16)] keys per home cell after the step (survivors + new keys)

@@ -54,6 +54,7 @@
 //     row's consistency flag is then set (cleared on the in-order path).
 #include "kvx_internal.h"
 #include "sieve_hbm.h"
+#include "sieve_local.h"
 
 namespace kvx {
 namespace {
@@ -1392,8 +1393,6 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
         __syncthreads();
         if (tid == 0) {
             tbl[P.t.meta + 1] = static_cast<uint32_t>(sMisses);
-            tbl[P.t.meta + 3] = sRing ? 1u : 0u;
-            tbl[P.t.meta + 4] = static_cast<uint32_t>(hand0 < 0 || hand0 >= dbs ? 0 : hand0);
             tbl[P.t.meta] = 1u;
             gHand[1] = kCanonFlag;  // the rebuild leaves the table consistent
             gHand[kFingerprintWord] = static_cast<int32_t>(sFp + sFpD);
@@ -1405,6 +1404,10 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
                    (unsigned long long)(stamp[1] - stamp[0]), (unsigned long long)(stamp[2] - stamp[1]),
                    (unsigned long long)(stamp[3] - stamp[2]), (unsigned long long)(stamp[4] - stamp[3]));
 #endif
+        __threadfence_block();
+        __syncthreads();
+        table_local::apply(a, tbl, P.t, reqIdx, static_cast<uint32_t>(sMisses),
+                           static_cast<uint32_t>(hand0 < 0 || hand0 >= dbs ? 0 : hand0), sRing != 0, lds);
         return;
     }
     if (sMisses > 0) {
@@ -1890,7 +1893,10 @@ hipError_t launch_sieve_update_batch(const HispSieveUpdateArgs &a, uint64_t over
     P.t = table_layout(a.htSize);
     hipLaunchKernelGGL(kvx_sieve_batch_pre, dim3(kPreSplit, a.maxNumReqs), dim3(kPreThreads), 0, stream, P);
     hipLaunchKernelGGL(kvx_sieve_batch_slots, dim3(kPreSplit, a.maxNumReqs), dim3(kPreThreads), 0, stream, P);
-    hipLaunchKernelGGL(kvx_sieve_update_batch, dim3(a.maxNumReqs), dim3(BT), P.lay.total, stream, P);
+    // the table update at the kernel's end takes the decisions' LDS again
+    const uint32_t local = tbl == nullptr ? 0u : table_local::lds_bytes(a.htSize < table_local::kLocalCells ? a.htSize : table_local::kLocalCells);
+    const uint32_t ldsBytes = local > P.lay.total ? local : P.lay.total;
+    hipLaunchKernelGGL(kvx_sieve_update_batch, dim3(a.maxNumReqs), dim3(BT), ldsBytes, stream, P);
     if (tbl != nullptr) {
         const hipError_t err = hipGetLastError();
         if (err != hipSuccess) return err;
