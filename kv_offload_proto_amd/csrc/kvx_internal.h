@@ -105,7 +105,7 @@ __host__ __device__ __forceinline__ uint64_t export_rows_win_entries(uint32_t pe
 constexpr int kFastThreads = KVX_FAST_THREADS;
 
 struct FastLayout {
-    uint32_t tok, ht, vis, ptok, pinf, vt, evslot, smKp, eseq, tb, smA, smB, vset, ber, occ, fin, rnk, cmask, emask,
+    uint32_t tok, ht, vis, ptok, pinf, vt, evslot, smKp, eseq, tb, smA, smB, vset, ber, occ, fin, nkb, cmask, emask,
         smask, rsn, rsm, total;
 };
 
@@ -121,8 +121,8 @@ __host__ __device__ __forceinline__ uint32_t align16(uint32_t x) { return (x + 1
 // cmask/emask/smask/rsn/rsm hold one 64-bit ballot per (wave, block of one
 // entry per lane).  ber, occ and fin are one bit per table cell: cells of
 // evicted tokens, the pre-step occupancy, the occupancy as the erase changes
-// it.  rnk: the event order of up to 64 slots (rows decided in registers).
-constexpr uint32_t kRankBytes = 64u * 2u;
+// it.  nkb (htSize / 8 bytes, at least 128): the event order of up to 64 slots
+// (rows decided in registers).
 __host__ __device__ __forceinline__ FastLayout fast_layout(uint32_t padded, uint32_t htSize, uint32_t topK,
                                                            uint32_t visStrideB, bool compact = false)
 {
@@ -153,7 +153,7 @@ __host__ __device__ __forceinline__ FastLayout fast_layout(uint32_t padded, uint
     l.rsn = o;     o += ringMaskBytes;
     l.rsm = o;     o += ringMaskBytes;
     l.fin = o;     o += align16(bmBytes);
-    l.rnk = o;     o += kRankBytes;
+    l.nkb = o;     o += align16(bmBytes);
     l.total = o;
     return l;
 }
@@ -201,13 +201,15 @@ __host__ __device__ __forceinline__ FastLayout fast_layout_fixed(uint32_t padded
     l.vis = o;     o += align16(visStrideB);
     l.ber = o;     o += align16(htSize / 8u);
     l.occ = o;     o += align16(htSize / 8u);
-    // the bitmap that the erase changes takes the per-position classes'
-    // region, which the fixed kernels keep in registers instead
-    l.rnk = o;     o += kRankBytes;
-    if (align16(htSize / 8u) <= Kx * 4u) {
+    // the bitmap that the erase changes and the event orders take the
+    // per-position classes' region, which the fixed kernels keep in registers
+    // instead
+    if (2u * align16(htSize / 8u) <= Kx * 4u) {
         l.fin = l.pinf;
+        l.nkb = l.pinf + align16(htSize / 8u);
     } else {
         l.fin = o;  o += align16(htSize / 8u);
+        l.nkb = o;  o += align16(htSize / 8u);
     }
     l.total = o;
     return l;
@@ -253,17 +255,18 @@ __host__ __device__ __forceinline__ BatchLayout batch_layout(uint32_t dbs, uint3
     l.ev = o;     o += nVisW * 8u;
     l.del = o;    o += nCellW * 8u;
     l.slot = o;   o += align16(topK * 4u);
+    const uint32_t bitBytes = (nCellW + nL1 + nL2) * 8u;
+    const uint32_t uniBytes = topK * 4u > bitBytes ? topK * 4u : bitBytes;
+    // the evicted slots in event order, where that still fits (0: searched for)
+    const uint64_t rest = static_cast<uint64_t>(align16(uniBytes)) + kBatchStage * 4u;
+    const uint32_t evl = align16(topK * 2u);
+    l.evl = o + evl + rest <= kBatchLds ? o : 0u;
+    if (l.evl != 0u) o += evl;
     l.uni = o;
     l.uniL1 = o + nCellW * 8u;
     l.uniL2 = l.uniL1 + nL1 * 8u;
-    const uint32_t bitBytes = (nCellW + nL1 + nL2) * 8u;
-    const uint32_t uniBytes = topK * 4u > bitBytes ? topK * 4u : bitBytes;
     o += align16(uniBytes);
     l.stage = o;  o += kBatchStage * 4u;
-    // the evicted slots in event order, where that still fits (0: searched for)
-    const uint32_t evl = align16(topK * 2u);
-    l.evl = o + evl <= kBatchLds ? o : 0u;
-    if (l.evl != 0u) o += evl;
     l.total = o;
     return l;
 }

@@ -1298,9 +1298,9 @@ def test_sieve_table_rebuild_cluster_edges(kvops, case):
     assert kvops.read_overflow() == 0
 
 
-@pytest.mark.parametrize("dbs,top_k,want", [(9370, 1655, 4), (10000, 2000, 5), (12000, 1200, 4), (15000, 1000, 5), (700, 16383, 0)])
+@pytest.mark.parametrize("dbs,top_k,want", [(9370, 1655, 5), (10000, 2000, 5), (12000, 1200, 5), (15000, 1000, 5), (700, 16383, 0)])
 def test_sieve_rows_between_the_layouts(kvops, dbs, top_k, want):
-    """Rows about and past the end of the parallel kernel's layouts: the batch
+    """Rows that fit LDS but neither layout of the parallel kernel: the batch
     kernel, or the sequential one with as many positions as slots; full state
     against the oracle after every step."""
     rng = np.random.default_rng(dbs)
