@@ -9,9 +9,9 @@
 // finds the winners (the last miss position per destination row) among its own
 // positions, lists their rows in LDS with the reference's queued counts, and
 // moves them as 16-byte chunks, 8 chunks in flight per lane.  Calls whose
-// requests share rows over more than 8192 positions take two launches: winners
-// in memory, then the listing and the copy, where 64 workgroups claim 256
-// positions at a time.
+// requests share rows over more than 8192 positions, and larger ones on
+// striped segments, take two launches: winners in memory, then the listing and
+// the copy, where 64 workgroups claim 256 positions at a time.
 //
 // Completion: the last workgroup to finish (atomicInc ticket) stores the
 // status words with a system-scope release, after every workgroup fenced its
@@ -352,6 +352,11 @@ __global__ __launch_bounds__(256) void kvx_gather_span(GatherParams P)
 constexpr uint32_t kOneMinSpan = 16, kOneMaxSpan = 64;
 constexpr uint32_t kOneMaxGroup = 8192;  // positions of a group (each workgroup reads the later ones)
 constexpr uint32_t kOneMaxBlocks = 256;  // workgroups; more spans are taken in turn
+// Rows of a stripe share one segment row, whose repeats an XCD's L2 serves
+// when neighbouring positions meet there: larger calls of that kind keep the
+// two launches, whose 64 workgroups take 256 positions each (32768 positions,
+// stripes of 16: 178 us, 238 in short spans; 3600 positions: 64 and 37).
+constexpr uint32_t kOneMaxStriped = 4096;
 constexpr int kOneThreads = 256;
 
 __global__ __launch_bounds__(kOneThreads) void kvx_gather_one(GatherParams P)
@@ -898,7 +903,8 @@ hipError_t launch_gather(const GatherPlan &plan, const RowScratch &scr, uint64_t
     const uint64_t positions = static_cast<uint64_t>(plan.a.maxNumReqs) * plan.a.topK;
     // the positions that can share a destination row
     const uint64_t group = plan.spanRows == 0 ? positions : plan.a.topK;
-    if (positions != 0 && group <= kOneMaxGroup && positions < (1ull << 31)) {
+    const bool striped = plan.a.stripeRows > 1u && positions > kOneMaxStriped;
+    if (positions != 0 && group <= kOneMaxGroup && positions < (1ull << 31) && !striped) {
         uint32_t span = kOneMinSpan;
         while (span < kOneMaxSpan && positions / span > kOneMaxBlocks) span *= 2u;
         P.x.span = span;
