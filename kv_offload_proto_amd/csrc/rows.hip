@@ -341,8 +341,10 @@ __global__ __launch_bounds__(256) void kvx_gather_span(GatherParams P)
 //
 // The bound is the host link.  The reads of many CUs fill it (1638 rows of
 // 1152 bytes alone: 72 us from 16 workgroups, 46 from 32, 40 from 128 and
-// more), so the spans are short, up to 256 workgroups; past that they take
-// several spans in turn, which keeps the rows in flight near each other
+// more), so the spans are short: 16 positions up to 1024 spans, so that a
+// workgroup's next span is listed while others copy (50 requests of 300
+// positions: 182 us in spans of 64, 172 of 32, 159 of 16), then up to 64, taken
+// in turn by 256 workgroups, which keeps the rows in flight near each other
 // (64 requests of 2048 positions: 64 workgroups 674 us, 128 639, 256 633, 512
 // 651, 1024 662; spans of 128: 654 from 256).  Against a launch that marked
 // the winners in memory and one that listed and moved the rows: 8192 positions
@@ -906,7 +908,7 @@ hipError_t launch_gather(const GatherPlan &plan, const RowScratch &scr, uint64_t
     const bool striped = plan.a.stripeRows > 1u && positions > kOneMaxStriped;
     if (positions != 0 && group <= kOneMaxGroup && positions < (1ull << 31) && !striped) {
         uint32_t span = kOneMinSpan;
-        while (span < kOneMaxSpan && positions / span > kOneMaxBlocks) span *= 2u;
+        while (span < kOneMaxSpan && positions / span > 4u * kOneMaxBlocks) span *= 2u;
         P.x.span = span;
         P.x.groupSize = static_cast<uint32_t>(group);
         P.x.parts = (P.x.groupSize + span - 1u) / span;
