@@ -67,7 +67,17 @@ __device__ __forceinline__ void apply(const HispSieveUpdateArgs &a, KVX_GM uint3
     uint32_t *changed = del + C / 32u;       // cells to write back
     uint32_t *evict = changed + C / 32u;     // evicted slots, 65536 bits
     uint8_t *del8 = reinterpret_cast<uint8_t *>(del), *changed8 = reinterpret_cast<uint8_t *>(changed);
+    // Whether the row is left to the rebuild is decided at a barrier, from
+    // every thread's own flag; sStop only lets other waves' loops end early.
+    // (Read behind a barrier, it could already hold the next phase's value in
+    // a late wave, which would then leave alone.)
+    bool stop = false;
+    auto stop_now = [&]() {
+        stop = true;
+        *const_cast<volatile int32_t *>(&sStop) = 1;
+    };
     auto stopped = [&]() { return *const_cast<volatile int32_t *>(&sStop) != 0; };
+    auto refused = [&]() { return __syncthreads_or(stop ? 1 : 0) != 0; };
     auto evicted = [&](uint32_t s) { return (evict[s >> 5] >> (s & 31u)) & 1u; };
     Cells8 v[kLocalLoads];
 #pragma unroll
@@ -101,12 +111,11 @@ __device__ __forceinline__ void apply(const HispSieveUpdateArgs &a, KVX_GM uint3
         runs &= runs >> 1;
         runs &= runs >> 2;
         runs &= runs >> 4;
-        if (runs != 0ull) sStop = 1;
+        if (runs != 0ull) stop_now();
         // a key in a cell past 65535 has a home below it: cell 65535 is taken
-        if (H > kLocalCells && i == kLocalCells / 8u - 1u && (v[q].w >> 16) != 0u) sStop = 1;
+        if (H > kLocalCells && i == kLocalCells / 8u - 1u && (v[q].w >> 16) != 0u) stop_now();
     }
-    __syncthreads();
-    if (sStop) {
+    if (refused()) {
         leave();
         return;
     }
@@ -131,15 +140,14 @@ __device__ __forceinline__ void apply(const HispSieveUpdateArgs &a, KVX_GM uint3
                     break;
                 }
                 if (n >= kLocalWalk) {
-                    sStop = 1;
+                    stop_now();
                     break;
                 }
             }
             if (first) lead[q] |= 1u << (c & 31u);
         }
     }
-    __syncthreads();
-    if (sStop) {
+    if (refused()) {
         leave();
         return;
     }
@@ -152,7 +160,7 @@ __device__ __forceinline__ void apply(const HispSieveUpdateArgs &a, KVX_GM uint3
             bool done = false;
             for (uint32_t o0 = 1; !done; o0 += 4u) {
                 if (o0 + 4u > kLocalWalk) {
-                    sStop = 1;
+                    stop_now();
                     break;
                 }
                 uint32_t x[4], e[4];
@@ -167,7 +175,7 @@ __device__ __forceinline__ void apply(const HispSieveUpdateArgs &a, KVX_GM uint3
                     run = run && e[h] != 0u;
                     dl[h] = run && ((del[x[h] >> 5] >> (x[h] & 31u)) & 1u);
                     if (run && e[h] > padded) {  // only in a corrupted table: the rebuild takes the row
-                        sStop = 1;
+                        stop_now();
                         run = false;
                         e[h] = 0u;
                     }
@@ -200,8 +208,7 @@ __device__ __forceinline__ void apply(const HispSieveUpdateArgs &a, KVX_GM uint3
             }
         }
     }
-    __syncthreads();
-    if (sStop) {
+    if (refused()) {
         leave();
         return;
     }
@@ -212,7 +219,7 @@ __device__ __forceinline__ void apply(const HispSieveUpdateArgs &a, KVX_GM uint3
         for (uint32_t hops = 0;; ++hops) {
             if (c >= C && wraps) c = 0u;
             if (c >= C || hops >= kLocalHops) {
-                sStop = 1;
+                stop_now();
                 break;
             }
             uint32_t *w = cells32 + (c >> 1);
@@ -237,8 +244,7 @@ __device__ __forceinline__ void apply(const HispSieveUpdateArgs &a, KVX_GM uint3
             ++c;
         }
     }
-    __syncthreads();
-    if (sStop) {
+    if (refused()) {
         leave();
         return;
     }

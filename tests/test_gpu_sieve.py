@@ -1251,6 +1251,62 @@ def test_sieve_table_short_clusters(kvops, dbs, top_k, last):
     assert kvops.read_overflow() == 0
 
 
+@pytest.mark.parametrize("kinds", [["lead"], ["walk"], ["chain"], ["short", "lead", "walk", "chain"] * 3])
+def test_sieve_table_update_refused_late(kvops, kinds):
+    """Rows that the one-workgroup table update leaves to the rebuild only in
+    its later phases: a lost key too far into its cluster to find the cluster's
+    start ("lead"), a cluster too long to close up ("walk"; both 120 cells in a
+    row around a multiple of 512 cells, so that the staging sees no run of 64 in
+    a wave's cells), a chain of proposals past its limit ("chain"); full state
+    against the oracle after every step."""
+    dbs, top_k, prefill = 16384, 2048, 1 << 18
+    req = len(kinds)
+    st = orc.SieveState(1, req, dbs, top_k)
+    assert st.ht_size == 65536
+    order = np.argsort(_home(np.arange(prefill, dtype=np.int64), 65536), kind="stable")
+    homes = _home(order, 65536)
+    by_home = [order[np.searchsorted(homes, h):np.searchsorted(homes, h, "right")] for h in range(65536)]
+    steps = 4
+    batch = np.full((steps, req, top_k), -1, dtype=np.int32)
+    for r, kind in enumerate(kinds):
+        st.admit(r, prefill)
+        st.tokens[0, r, :] = -1
+        for i in range(steps):
+            middle = 512 * (8 * i + 4 + r)
+            run = [by_home[h][0] for h in range(middle - 60, middle + 60) if len(by_home[h])]
+            at = {"lead": 110, "walk": 0, "chain": 60, "short": 60}[kind]
+            if kind == "short":
+                run = run[at - 5:at + 5]
+                at = 5
+            misses = [by_home[(middle + 2048) & 65535][0]]
+            if kind == "chain":
+                misses = [t for h in range(middle + 200, middle + 500) for t in by_home[h]]
+            # slots in ring order: the step evicts the run's key at `at` first
+            lo = 4096 * i
+            st.tokens[0, r, lo] = run[at]
+            rest = run[:at] + run[at + 1:]
+            st.tokens[0, r, lo + 2048:lo + 2048 + len(rest)] = rest
+            assert len(misses) <= top_k
+            batch[i, r, :len(misses)] = misses
+    orc.sieve_ht_init(st.tokens, st.ht, 0, req, 1, req, dbs, st.padded, st.ht_size)
+    dev = DevSieve(st)
+    kvops.sieve_force_variant(5)
+    try:
+        for i in range(steps):
+            st.hand[0, :, 0] = 4096 * i
+            dev.hand[0, :, 0] = 4096 * i
+            seq = np.full(req, prefill)
+            e_slots, e_miss = st.update(0, batch[i], np.arange(req), seq, req)
+            g_slots, g_miss, _ = dev.update(kvops, 0, batch[i], np.arange(req), seq, req, req, top_k)
+            assert kvops.last_sieve_variant() == 5
+            np.testing.assert_array_equal(g_miss, e_miss, err_msg="step {}".format(i))
+            np.testing.assert_array_equal(g_slots, e_slots, err_msg="step {}".format(i))
+            dev.assert_state_equal()
+    finally:
+        kvops.sieve_force_variant(-1)
+    assert kvops.read_overflow() == 0
+
+
 @pytest.mark.parametrize("case", ["wrap", "past-2^16"])
 def test_sieve_table_rebuild_cluster_edges(kvops, case):
     """The parallel table rebuild where the cell order matters most: "wrap"
