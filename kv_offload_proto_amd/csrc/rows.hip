@@ -98,10 +98,13 @@ __device__ __forceinline__ void store_status(uint64_t addr, uint64_t word)
 // and it can report them without a fence: a device-scope release writes back
 // the whole L2 of its XCD, and one per workgroup, while others still copy,
 // took a fifth of the import (131072 positions from 1024 workgroups 859 -> 671
-// us without it, 1665 positions from 105 27 -> 19).
+// us without it, 1665 positions from 105 27 -> 19).  The data registers of a
+// store of more than 8 bytes may not be rewritten for two wait states, and the
+// compiler, which does not see the store, does not keep them: they are part
+// of the asm.
 __device__ __forceinline__ void store_through(uint64_t addr, u32x4 v)
 {
-    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt" : : "v"(addr), "v"(v) : "memory");
+    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt\n\ts_nop 1" : : "v"(addr), "v"(v) : "memory");
 }
 __device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" : : : "memory"); }
 
