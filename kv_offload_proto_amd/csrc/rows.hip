@@ -108,6 +108,19 @@ __device__ __forceinline__ void store_through(uint64_t addr, u32x4 v)
 }
 __device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" : : : "memory"); }
 
+// Waits for N predicated loads at one point: each value passes through the
+// asm, so the compiler waits for all of them before it and for none after it.
+// Without it, every use under a condition of its own waits for everything in
+// flight (vmcnt(0)), stores included: a copy's stores then go one round trip
+// after another, and where a load's registers are reused for its address, its
+// loads too (an export of 4000 rows 203 us, 98 so; 64 rows' append 7.3, 6.8).
+template <int N>
+__device__ __forceinline__ void wait_loads(u32x4 *v)
+{
+#pragma unroll
+    for (int j = 0; j < N; ++j) asm volatile("" : "+v"(v[j]));
+}
+
 // A status word cleared at the start of a launch: the last workgroup's word
 // follows it (its ticket comes after the clearing workgroup's wait).
 __device__ __forceinline__ void clear_status(uint64_t addr)
@@ -117,7 +130,9 @@ __device__ __forceinline__ void clear_status(uint64_t addr)
 
 // Copy `n` rows whose byte addresses sit in src[0..n), dst[0..n) (LDS or
 // global) with the whole wave: chunk c covers bytes [16*(c%cpr), +16) of row
-// c/cpr.  kUnroll loads are issued before their stores.
+// c/cpr.  kUnroll loads are issued before their stores.  (kThrough false, the
+// two-launch import: its stores wait for one another; in flight together they
+// make it slower by 1 % at 32768 positions.)
 template <bool kThrough = false>
 __device__ __forceinline__ void wave_copy_rows(const uint64_t *src, const uint64_t *dst, uint32_t n, uint32_t cpr)
 {
@@ -137,6 +152,7 @@ __device__ __forceinline__ void wave_copy_rows(const uint64_t *src, const uint64
                 d[j] = dst[r] + o;
             }
         }
+        if constexpr (kThrough) wait_loads<kUnroll>(v);
 #pragma unroll
         for (int j = 0; j < kUnroll; ++j) {
             if (d[j] == 0) continue;
@@ -508,6 +524,7 @@ __global__ __launch_bounds__(kOneThreads) void kvx_gather_one(GatherParams P)
                     d[j] = sDst[r] + o;
                 }
             }
+            wait_loads<kUnroll>(v);
 #pragma unroll
             for (int j = 0; j < kUnroll; ++j) {
                 if (d[j] != 0) store_through(d[j], v[j]);
@@ -546,7 +563,11 @@ __global__ __launch_bounds__(kOneThreads) void kvx_gather_one(GatherParams P)
 // row (its highest row inside the range) to segment row q/N of layer l.  Rows
 // are stored through the caches: with a system-scope fence per workgroup, each
 // a write-back of an XCD's L2, 144 MB took 2751 us, now 2534 (56.9 GB/s of the
-// link's 57.0); 32 workgroups take 2592.
+// link's 57.0).  Up to 64 workgroups: with their chunks in flight they fill
+// the link, and 128 or more get less from it (131072 rows, 2671 us from 48 or
+// 64, 2681 from 96, 2690 from 128 to 512).
+constexpr uint32_t kExportBlocks = 64;
+
 __global__ __launch_bounds__(256) void kvx_export_alllayer(ExportParams P)
 {
     __shared__ uint64_t sSrc[kWaves][64];
@@ -833,6 +854,7 @@ __global__ __launch_bounds__(256) void kvx_export_rows_small(ExportRowsParams P)
                 d[j] = sDst[r] + o;
             }
         }
+        wait_loads<4>(v);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             if (d[j] != 0) store_through(d[j], v[j]);
@@ -951,7 +973,7 @@ hipError_t launch_export(const KvcScatterAllArgs &a, const RowScratch &scr, uint
     const uint64_t items = P.x.nStripes * a.layerNum;
     uint64_t blocks = (items + 64ull * kWaves - 1ull) / (64ull * kWaves);
     if (blocks < 1) blocks = 1;
-    if (blocks > 2048) blocks = 2048;
+    if (blocks > kExportBlocks) blocks = kExportBlocks;
     hipLaunchKernelGGL(kvx_export_alllayer, dim3(static_cast<uint32_t>(blocks)), dim3(256), 0, stream, P);
     return hipGetLastError();
 }

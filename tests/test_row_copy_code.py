@@ -55,3 +55,16 @@ def test_stores_through_the_caches_keep_their_wait_states(kernels, name):
     assert stores
     for i in stores:
         assert code[i + 1] == "s_nop 1", code[i:i + 3]
+
+
+@pytest.mark.parametrize("name", THROUGH)
+def test_copy_loops_keep_their_chunks_in_flight(kernels, name):
+    """A copy loop that stores through the caches issues its loads, waits once, and issues its stores: no wait
+    for memory from a loop's first load to its last, nor from its first store
+    to its last."""
+    code = _kernel(kernels, name)
+    unroll = 4 if name == "kvx_export_rows_small" else 8
+    for kind in ("load", "store"):
+        at = [i for i, op in enumerate(code) if op.startswith("global_{}_dwordx4".format(kind))]
+        assert len(at) == unroll
+        assert not [op for op in code[at[0]:at[-1]] if "vmcnt" in op]
