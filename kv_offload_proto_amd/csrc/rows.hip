@@ -57,7 +57,6 @@ struct GatherExtra {
     uint32_t fused;
     uint32_t spanRows;
     uint32_t statusWords;
-    uint32_t groupSize, span, parts, blocks;  // one launch: positions of a group and of a span, spans of a group and in all
 };
 
 struct GatherParams {
@@ -369,7 +368,10 @@ __global__ __launch_bounds__(256) void kvx_gather_span(GatherParams P)
 // the winners in memory and one that listed and moved the rows: 8192 positions
 // 56 -> 47 us, 1665 positions in the earlier one-launch form, where every
 // workgroup counted all positions, 29 -> 19; 131072 positions 639 -> 633 (the
-// link).
+// link).  The spans are those of the positions in use: a call, or a captured
+// graph's replay, with fewer requests than it was made for does nothing for
+// the others (256 requests of 1024 positions with 16 in use 102 us when every
+// span of the largest batch was walked, 77 so; with none 20 and 7).
 constexpr uint32_t kOneMinSpan = 16, kOneMaxSpan = 64;
 constexpr uint32_t kOneMaxGroup = 8192;  // positions of a group (each workgroup reads the later ones)
 constexpr uint32_t kOneMaxBlocks = 256;  // workgroups; more spans are taken in turn
@@ -379,6 +381,21 @@ constexpr uint32_t kOneMaxBlocks = 256;  // workgroups; more spans are taken in 
 // stripes of 16: 178 us, 238 in short spans; 3600 positions: 64 and 37).
 constexpr uint32_t kOneMaxStriped = 4096;
 constexpr int kOneThreads = 256;
+
+struct GatherSpans {
+    uint32_t span, parts, count;  // positions of a span, spans of a group and in all
+};
+
+// The spans of `positions` positions in groups of `group` (a divisor).
+__host__ __device__ __forceinline__ GatherSpans gather_spans(uint32_t positions, uint32_t group)
+{
+    GatherSpans g{kOneMinSpan, 0u, 0u};
+    if (positions == 0u) return g;
+    while (g.span < kOneMaxSpan && positions / g.span > 4u * kOneMaxBlocks) g.span *= 2u;
+    g.parts = (group + g.span - 1u) / g.span;
+    g.count = positions / group * g.parts;
+    return g;
+}
 
 __global__ __launch_bounds__(kOneThreads) void kvx_gather_one(GatherParams P)
 {
@@ -400,8 +417,11 @@ __global__ __launch_bounds__(kOneThreads) void kvx_gather_one(GatherParams P)
     const KVX_G int8_t *miss = reinterpret_cast<const KVX_G int8_t *>(a.isMiss);
     const KVX_G int64_t *pool = reinterpret_cast<const KVX_G int64_t *>(a.reqPoolIndices);
     const KVX_G int64_t *hostBase = reinterpret_cast<const KVX_G int64_t *>(a.reqHostBase);
-    const int32_t numReal = clamp_num_real(a.numReal, a.maxNumReqs);
+    const int32_t numReal = __builtin_amdgcn_readfirstlane(clamp_num_real(a.numReal, a.maxNumReqs));
     const uint32_t total = static_cast<uint32_t>(numReal) * a.topK;  // (host: below 2^31)
+    const uint32_t groupSize = x.spanRows == 0u ? total : a.topK;
+    const GatherSpans sp = gather_spans(total, groupSize);
+    const uint32_t span = sp.span;
     if (blockIdx.x == 0 && a.status != 0) {  // the call's status words read 0 until its rows have landed
         for (uint32_t i = tid; i < (n1 - n0) * x.statusWords; i += kOneThreads) {
             clear_status(a.status + (n0 + i / x.statusWords) * 64ull + (i % x.statusWords) * 8ull);
@@ -411,18 +431,18 @@ __global__ __launch_bounds__(kOneThreads) void kvx_gather_one(GatherParams P)
         sCnt[i] = 0u;
         sErr[i] = 0u;
     }
-    for (uint32_t blk = blockIdx.x; blk < x.blocks; blk += gridDim.x) {
-        const uint32_t group = blk / x.parts, part = blk - group * x.parts;
-        const uint32_t g0 = group * x.groupSize, lo = g0 + part * x.span, p = lo + tid, bid = p / a.topK;
+    for (uint32_t blk = blockIdx.x; blk < sp.count; blk += gridDim.x) {
+        const uint32_t group = blk / sp.parts, part = blk - group * sp.parts;
+        const uint32_t g0 = group * groupSize, lo = g0 + part * span, p = lo + tid, bid = p / a.topK;
         for (uint32_t i = tid; i < 65536u / 32u / 4u; i += kOneThreads) reinterpret_cast<uint4 *>(sLater)[i] = make_uint4(0, 0, 0, 0);
         if (tid < kOneMaxSpan / 32u) sLose[tid] = 0u;
         if (tid == 0) sN = 0u;
-        const uint32_t gEnd = min(g0 + x.groupSize, total);
-        const uint32_t hi = min(lo + x.span, gEnd);
+        const uint32_t gEnd = min(g0 + groupSize, total);
+        const uint32_t hi = min(lo + span, gEnd);
         int8_t m = 0;
         int32_t t = -1, s = -1;
         int64_t pl = -1, hb = 0;
-        if (tid < x.span && p < gEnd) {  // the own position's five reads, issued together
+        if (tid < span && p < gEnd) {  // the own position's five reads, issued together
             m = miss[p];
             t = topk[p];
             s = slots[p];
@@ -432,7 +452,7 @@ __global__ __launch_bounds__(kOneThreads) void kvx_gather_one(GatherParams P)
         // a position in the winner rule: a miss with a token and a slot (16 bits)
         const bool valid = m != 0 && t >= 0 && s >= 0 && pl >= 0;
         const bool rule = valid && s < 65536;
-        if (tid < x.span) sKey[tid] = rule ? s : -1;
+        if (tid < span) sKey[tid] = rule ? s : -1;
         __syncthreads();
         for (uint32_t q0 = hi + tid; q0 < gEnd; q0 += 4u * kOneThreads) {
             int8_t mq[4];
@@ -455,17 +475,17 @@ __global__ __launch_bounds__(kOneThreads) void kvx_gather_one(GatherParams P)
         }
         // own positions against the later own ones, kOneThreads / span lanes each
         {
-            const uint32_t per = kOneThreads / x.span, i = tid / per;  // span: a power of two
+            const uint32_t per = kOneThreads / span, i = tid / per;  // span: a power of two
             const int32_t k = sKey[i];
             bool later = false;
             if (k >= 0) {
-                for (uint32_t j = i + 1u + (tid & (per - 1u)); j < x.span; j += per) later |= sKey[j] == k;
+                for (uint32_t j = i + 1u + (tid & (per - 1u)); j < span; j += per) later |= sKey[j] == k;
             }
             if (later) atomicOr(&sLose[i >> 5], 1u << (i & 31u));
         }
         const bool far = rule && x.spanRows != 0u && static_cast<uint32_t>(s) >= x.spanRows;
         if (__syncthreads_or(far ? 1 : 0)) {
-            for (uint32_t i = 0; i < x.span; ++i) {
+            for (uint32_t i = 0; i < span; ++i) {
                 const int32_t k = sKey[i];
                 if (k < 0 || static_cast<uint32_t>(k) < x.spanRows) continue;
                 const uint32_t b0 = (lo + i) / a.topK;
@@ -932,18 +952,10 @@ hipError_t launch_gather(const GatherPlan &plan, const RowScratch &scr, uint64_t
     const uint64_t group = plan.spanRows == 0 ? positions : plan.a.topK;
     const bool striped = plan.a.stripeRows > 1u && positions > kOneMaxStriped;
     if (positions != 0 && group <= kOneMaxGroup && positions < (1ull << 31) && !striped) {
-        uint32_t span = kOneMinSpan;
-        while (span < kOneMaxSpan && positions / span > 4u * kOneMaxBlocks) span *= 2u;
-        P.x.span = span;
-        P.x.groupSize = static_cast<uint32_t>(group);
-        P.x.parts = (P.x.groupSize + span - 1u) / span;
-        const uint64_t blocks = positions / group * P.x.parts;
-        if (blocks < (1ull << 31)) {
-            P.x.blocks = static_cast<uint32_t>(blocks);
-            hipLaunchKernelGGL(kvx_gather_one, dim3(static_cast<uint32_t>(blocks < kOneMaxBlocks ? blocks : kOneMaxBlocks)),
-                               dim3(kOneThreads), 0, stream, P);
-            return hipGetLastError();
-        }
+        // (spans of the largest batch; the kernel takes those of the real one)
+        const uint32_t count = gather_spans(static_cast<uint32_t>(positions), static_cast<uint32_t>(group)).count;
+        hipLaunchKernelGGL(kvx_gather_one, dim3(count < kOneMaxBlocks ? count : kOneMaxBlocks), dim3(kOneThreads), 0, stream, P);
+        return hipGetLastError();
     }
     uint64_t prepBlocks = (positions + 255ull) / 256ull;
     if (prepBlocks < 1) prepBlocks = 1;

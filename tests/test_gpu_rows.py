@@ -247,6 +247,51 @@ def test_gather_spans(kvops, req, top_k, dbs, stride_mode, fused, block_dim):
     test_gather_small_batch_winners(kvops, req, top_k, dbs, stride_mode, fused, block_dim)
 
 
+@pytest.mark.parametrize("req,top_k,num_real,S,N,stride_mode,fused,block_dim", [
+    (40, 513, 0, 1, 2, "padded", True, 3),    # an empty step
+    (40, 513, 1, 1, 2, "padded", True, 8),    # spans of 32 for the whole batch, of 16 for its one request
+    (70, 1000, 17, 1, 3, "padded", False, 2),  # of 64 and of 32
+    (9, 800, 2, 1, 2, "zero", True, 1),       # one group of every position in use
+    (9, 800, 0, 1, 2, "zero", False, 4),
+])
+def test_gather_spans_of_the_real_batch(kvops, req, top_k, num_real, S, N, stride_mode, fused, block_dim):
+    """The one-launch import of fewer requests than the call was made for:
+    its spans are those of the requests in use."""
+    test_gather_large_batch_parity(kvops, req, top_k, num_real, S, N, stride_mode, fused, block_dim)
+
+
+def test_gather_empty_step_costs_no_more_for_a_larger_batch(kvops):
+    """With num_real 0 an import does nothing for the requests it was made for,
+    however many (4,194,304 positions: 203 us a call when every span of the
+    largest batch was walked, 8 for one request of 16)."""
+    import time
+
+    pool = HostSegPool(0, 1, 64, ROW, stripe_rows=1, node_num=1)
+    pool.create_pool()
+    try:
+        def best(req, top_k):
+            z = torch.zeros((req, top_k), dtype=torch.int32, device="cuda")
+            args = (0, z, torch.zeros(req, dtype=torch.int64, device="cuda"),
+                    torch.zeros(req, dtype=torch.int64, device="cuda"), z,
+                    torch.zeros((req, top_k), dtype=torch.int8, device="cuda"),
+                    torch.zeros(1, dtype=torch.int32, device="cuda"), torch.zeros((16, ROW), dtype=torch.uint8, device="cuda"),
+                    req, top_k)
+            us = []
+            for _ in range(8):
+                torch.cuda.synchronize()
+                t0 = time.perf_counter()
+                for _ in range(20):
+                    pool.batch_read_fused(*args, hot_req_stride_rows=16)
+                torch.cuda.synchronize()
+                us.append((time.perf_counter() - t0) / 20 * 1e6)
+            return min(us)
+
+        small, large = best(1, 16), best(1024, 4096)
+        assert large < 4 * small + 20, (small, large)
+    finally:
+        pool.destroy(close_ext=False)
+
+
 @pytest.mark.parametrize("top_k", [1000, 3000])   # 3 x 1000 positions: one-launch form; 3 x 3000: two launches
 @pytest.mark.parametrize("fused", [False, True])    # import_seg per segment, or import_all
 def test_gather_rows_past_layer_region(kvops, top_k, fused):
