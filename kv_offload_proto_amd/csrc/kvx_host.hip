@@ -55,10 +55,11 @@ struct StreamScratch {
 // object, so each GPU the library is loaded on holds its own copy from load
 // to process exit, and the entry point allocates nothing.  Layout: the
 // control words (counters, error words, tickets, chunk counter, epoch), then
-// the winner table.  It starts zeroed; the kernels clear the counters, error
-// words and chunk counter at the start of every call, and the winner table is
-// tagged with the epoch that every call advances, so it is never cleared
-// (except at the epoch's 2^32 wrap, by the last copy workgroup).
+// the winner table.  It starts zeroed; the last workgroup of a call leaves the
+// counters and error words zero for the next, a two-launch call's first pass
+// clears the chunk counter, and the winner table is tagged with the epoch that
+// every two-launch call advances, so it is never cleared (except at the
+// epoch's 2^32 wrap, by the last copy workgroup).
 constexpr uint64_t kNoAllocMaxWinEntries = 34ull << 16;     // (max_num_reqs-1)*min(stride,65536) + 65536
 constexpr uint64_t kNoAllocControlBytes = (kvx::kControlWords * 4 + 255) / 256 * 256;
 constexpr uint64_t kNoAllocBytes = kNoAllocControlBytes + kNoAllocMaxWinEntries * 8;

@@ -67,10 +67,10 @@ __host__ __device__ __forceinline__ uint32_t slot_token_mix(uint32_t slot, int32
 struct RowScratch {
     unsigned long long *win;   // winner tags, (epoch << 32) | position
     uint64_t winEntries;       // capacity of win[]
-    uint32_t *counters;        // [64 nodes][8 status words] queued counts
-    uint32_t *errs;            // [64 nodes][8 status words] first error code
-    uint32_t *tickets;         // [8] last-block tickets (gather, export, export_rows, small gather, small export_rows)
-    uint32_t *epoch;           // gather winner-tag epoch, advanced on the device by each call
+    uint32_t *counters;        // [64 nodes][8 status words] queued counts, zero between calls
+    uint32_t *errs;            // [64 nodes][8 status words] ~(lowest failing position), zero between calls
+    uint32_t *tickets;         // [8] last-block tickets (gather, export, export_rows, one-launch gather, small export_rows)
+    uint32_t *epoch;           // gather winner-tag epoch, advanced on the device by each two-launch call
     uint32_t *chunkNext;       // next position chunk of the current gather
 };
 

@@ -120,6 +120,12 @@ __device__ __forceinline__ void wait_loads(u32x4 *v)
     for (int j = 0; j < N; ++j) asm volatile("" : "+v"(v[j]));
 }
 
+// The counters and error words of a call are zero between calls: the kernel
+// that stores the status words zeroes them, and a first pass whose second one
+// never ran leaves them zero too.  An error word holds ~p, max-reduced, of the
+// lowest failing position or entry p (below 2^32 - 1), 0 for none.
+__device__ __forceinline__ uint32_t error_word(uint32_t e) { return e == 0u ? 0u : row_error_code(~e); }
+
 // A status word cleared at the start of a launch: the last workgroup's word
 // follows it (its ticket comes after the clearing workgroup's wait).
 __device__ __forceinline__ void clear_status(uint64_t addr)
@@ -190,7 +196,7 @@ __global__ __launch_bounds__(256) void kvx_gather_prep(GatherParams P)
         if (threadIdx.x == 0) *x.chunkNext = 0u;
         for (uint32_t i = threadIdx.x; i < (n1 - n0) * 8u; i += blockDim.x) {
             x.counters[n0 * 8u + i] = 0u;
-            x.errs[n0 * 8u + i] = 0xFFFFFFFFu;  // lowest failing position, min-reduced
+            x.errs[n0 * 8u + i] = 0u;
         }
         if (a.status != 0) {
             for (uint32_t i = threadIdx.x; i < (n1 - n0) * x.statusWords; i += blockDim.x) {
@@ -282,7 +288,7 @@ __global__ __launch_bounds__(256) void kvx_gather_span(GatherParams P)
                         }
                         const uint64_t segRow = kvx_seg_row_of(row, a.stripeRows, a.nodeNum);
                         if (segRow >= a.perLayerSegRows) {  // row outside the segment: report, do not read
-                            atomicMin(&x.errs[key], static_cast<uint32_t>(p));
+                            atomicMax(&x.errs[key], ~static_cast<uint32_t>(p));
                             winner = false;
                         }
                         copy = winner;
@@ -333,12 +339,12 @@ __global__ __launch_bounds__(256) void kvx_gather_span(GatherParams P)
         const uint32_t node = n0 + i / 8u, b = i % 8u;
         const uint32_t q = __hip_atomic_load(&x.counters[node * 8u + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const uint32_t e = __hip_atomic_load(&x.errs[node * 8u + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        x.counters[node * 8u + b] = 0u;  // the one-launch import finds them zeroed
+        x.counters[node * 8u + b] = 0u;
         x.errs[node * 8u + b] = 0u;
         if (a.status == 0 || b >= x.statusWords) continue;
         uint64_t word = 1ull << 32;  // kvc_gather_rows.cpp:29-33, :93
         if (static_cast<int64_t>(b * ppc) < total) {
-            word |= (static_cast<uint64_t>(q) << 40) | (e == 0xFFFFFFFFu ? 0u : row_error_code(e));
+            word |= (static_cast<uint64_t>(q) << 40) | error_word(e);
         }
         store_status(a.status + node * 64ull + b * 8ull, word);
     }
@@ -574,7 +580,7 @@ __global__ __launch_bounds__(kOneThreads) void kvx_gather_one(GatherParams P)
         if (e != 0u) __hip_atomic_store(&x.errs[node * 8u + b], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (a.status == 0 || b >= x.statusWords) continue;
         uint64_t word = 1ull << 32;  // kvc_gather_rows.cpp:29-33, :93
-        if (static_cast<uint64_t>(b) * ppc < total) word |= (static_cast<uint64_t>(q) << 40) | (e == 0u ? 0u : row_error_code(~e));
+        if (static_cast<uint64_t>(b) * ppc < total) word |= (static_cast<uint64_t>(q) << 40) | error_word(e);
         store_status(a.status + node * 64ull + b * 8ull, word);
     }
 }
@@ -686,7 +692,7 @@ __global__ __launch_bounds__(256) void kvx_export_rows_prep(ExportRowsParams P)
         for (uint32_t k = threadIdx.x; k < (n1 - n0) * a.statusWords; k += blockDim.x) {
             const uint32_t node = n0 + k / a.statusWords, b = k % a.statusWords;
             P.counters[node * 8u + b] = 0u;
-            P.errs[node * 8u + b] = 0xFFFFFFFFu;  // lowest failing entry, min-reduced
+            P.errs[node * 8u + b] = 0u;
             if (a.status != 0) store_status(a.status + node * 64ull + b * 8ull, 0ull);
         }
     }
@@ -731,7 +737,7 @@ __global__ __launch_bounds__(256) void kvx_export_rows_copy(ExportRowsParams P)
             const uint32_t key = node * 8u + static_cast<uint32_t>(i) / ppc;
             atomicAdd(&P.counters[key], 1u);
             if (segRow >= a.perLayerSegRows) {  // outside the segment's layer region: report, do not write
-                atomicMin(&P.errs[key], static_cast<uint32_t>(i));
+                atomicMax(&P.errs[key], ~static_cast<uint32_t>(i));
             } else {
                 const uint64_t w = (a.fused ? static_cast<uint64_t>(node) * a.perLayerSegRows : 0ull) + segRow;
                 copy = w >= P.winEntries || win_load(P.win + w) == (tagHi | static_cast<unsigned long long>(i));
@@ -771,12 +777,12 @@ __global__ __launch_bounds__(256) void kvx_export_rows_copy(ExportRowsParams P)
         const uint32_t node = n0 + k / words, b = k % words;
         const uint32_t q = __hip_atomic_load(&P.counters[node * 8u + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const uint32_t e = __hip_atomic_load(&P.errs[node * 8u + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        P.counters[node * 8u + b] = 0u;  // the one-launch import finds them zeroed
+        P.counters[node * 8u + b] = 0u;
         P.errs[node * 8u + b] = 0u;
         if (a.status == 0) continue;
         uint64_t word = 1ull << 32;
         if (static_cast<int64_t>(b) * ppc < n) {
-            word |= (static_cast<uint64_t>(q) << 40) | (e == 0xFFFFFFFFu ? 0u : row_error_code(e));
+            word |= (static_cast<uint64_t>(q) << 40) | error_word(e);
         }
         store_status(a.status + node * 64ull + b * 8ull, word);
     }
@@ -896,7 +902,7 @@ __global__ __launch_bounds__(256) void kvx_export_rows_small(ExportRowsParams P)
         if (e != 0u) __hip_atomic_store(&P.errs[nd * 8u + b], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (a.status == 0 || b >= words) continue;
         uint64_t word = 1ull << 32;
-        if (static_cast<int64_t>(b) * ppc < n) word |= (static_cast<uint64_t>(q) << 40) | (e == 0u ? 0u : row_error_code(~e));
+        if (static_cast<int64_t>(b) * ppc < n) word |= (static_cast<uint64_t>(q) << 40) | error_word(e);
         store_status(a.status + nd * 64ull + b * 8ull, word);
     }
 }

@@ -446,3 +446,75 @@ def test_status_ring_blocks(kvops):
         assert _read_words(base + (N - 1) * 64, 1) == [DONE]
     finally:
         pool.destroy(close_ext=False)
+
+
+def _hip():
+    """The HIP runtime this process has loaded."""
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    return ctypes.CDLL(path)
+
+
+def _run_first_kernel_only(stream, call):
+    """Captures the two launches of `call` on `stream` and runs the first."""
+    hip = _hip()
+
+    def ok(rc):
+        assert rc == 0, rc
+
+    graph, exe, n = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_size_t(8)
+    s = ctypes.c_void_p(stream.cuda_stream)
+    ok(hip.hipStreamBeginCapture(s, ctypes.c_int(1)))
+    try:
+        call()
+    finally:
+        rc = hip.hipStreamEndCapture(s, ctypes.byref(graph))
+    ok(rc)
+    nodes, roots = (ctypes.c_void_p * 8)(), (ctypes.c_void_p * 8)()
+    ok(hip.hipGraphGetNodes(graph, nodes, ctypes.byref(n)))
+    r = ctypes.c_size_t(8)
+    ok(hip.hipGraphGetRootNodes(graph, roots, ctypes.byref(r)))
+    assert (n.value, r.value) == (2, 1)
+    (second,) = [x for x in nodes[:2] if x != roots[0]]
+    ok(hip.hipGraphDestroyNode(ctypes.c_void_p(second)))
+    ok(hip.hipGraphInstantiate(ctypes.byref(exe), graph, None, None, ctypes.c_size_t(0)))
+    ok(hip.hipGraphLaunch(exe, s))
+    stream.synchronize()
+    ok(hip.hipGraphExecDestroy(exe))
+    ok(hip.hipGraphDestroy(graph))
+
+
+@pytest.mark.parametrize("op", ["import", "export"])
+def test_first_pass_alone_leaves_no_error_behind(kvops, op):
+    """A two-launch import or export whose second launch never ran (here: taken
+    out of a captured graph) leaves the counters and error words zero: the next
+    one-launch call on the stream reports its own rows and no error."""
+    pool = HostSegPool(0, 1, 8192, ROW, stripe_rows=1, node_num=1)
+    pool.create_pool()
+    stream = torch.cuda.Stream()
+    try:
+        zero = torch.zeros(1, dtype=torch.int64, device="cuda")
+        rows = {"import": (8193, 1000), "export": (5000, 1000)}[op]  # a two-launch and a one-launch call
+        calls = []
+        for n in rows:
+            slots = torch.arange(n, dtype=torch.int32, device="cuda")
+            data = torch.zeros((n, ROW), dtype=torch.uint8, device="cuda")
+            if op == "import":
+                args = (0, slots % 8192, zero, zero, slots, torch.ones(n, dtype=torch.int8, device="cuda"),
+                        torch.ones(1, dtype=torch.int32, device="cuda"), data, 1, n)
+                f = pool.batch_read_fused
+            else:
+                args = (0, data, slots.to(torch.int64), torch.full((1,), n, dtype=torch.int32, device="cuda"), n)
+                f = pool.batch_export_rows_fused
+            calls.append(lambda f=f, args=args: f(*args, stream=stream.cuda_stream, block_dim=2))
+        torch.cuda.synchronize()
+        for c in calls:  # (sizes the stream's scratch)
+            pool.wait(c(), block_dim=2)
+        stream.synchronize()
+        _run_first_kernel_only(stream, calls[0])
+        status = calls[1]()
+        stream.synchronize()
+        assert _read_words(status, 2) == [DONE | 500 << 40] * 2
+    finally:
+        torch.cuda.synchronize()
+        pool.destroy(close_ext=False)
