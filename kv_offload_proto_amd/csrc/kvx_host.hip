@@ -291,7 +291,9 @@ StreamScratch &ScratchFor(uint64_t stream, const ScratchNeed &need, const char *
 // probes (1 = the single-lane HBM kernel, only when forced).  A row that fits
 // LDS but neither parallel layout (about 9000 to 15000 slots at 900 and more
 // positions) takes the batch kernel: 9 rows of 9370 slots and 1655 positions
-// 1060 us a call on the sequential one, 70 on the batch kernel.  With as many
+// 1060 us a call on the sequential one, 70 on the batch kernel (in both cases
+// without tokens past the batch kernel's map; with some the batch kernel runs
+// the sequential recurrence in LDS itself).  With as many
 // positions as slots a slot can be evicted twice in a step, which the batch
 // kernel leaves to a recurrence on HBM, so such a row stays on the sequential
 // LDS kernel; and so does a call whose stream has no scratch for the batch
@@ -301,7 +303,8 @@ struct SievePlan {
     size_t ldsLaunch = 0;   // dynamic LDS of the launch
     uint32_t invCap = 0;    // entries of the parallel kernel's token -> slot map
     bool rebuild = false;   // variant 5: a step's table changes by the rebuild kernels
-    size_t ldsInOrder = 0;  // variant 5: LDS of variant 0, which takes the row without scratch (0: it cannot)
+    size_t ldsInOrder = 0;  // variant 5: LDS of variant 0, which takes the row without scratch, and its in-order
+                            // steps inside the batch kernel (0: it cannot)
 };
 
 SievePlan PlanSieve(uint32_t top_k, uint32_t dbs, uint32_t padded, uint32_t visStrideB, uint32_t poolSize,
@@ -319,7 +322,7 @@ SievePlan PlanSieve(uint32_t top_k, uint32_t dbs, uint32_t padded, uint32_t visS
     const size_t ldsBatch = kvx::batch_layout(dbs, htSize, top_k).total;
     const bool batchOk = top_k >= 1 && top_k < (1u << 24) && dbs <= 65535 && htSize >= 1024 && ldsBatch <= g.ldsBatch;
     const bool inOrderOk = lds <= g.ldsLimit;
-    int v = fastOk ? 2 : (compactOk ? 4 : (inOrderOk && !(batchOk && top_k < dbs) ? 0 : (batchOk ? 5 : 3)));
+    int v = fastOk ? 2 : (compactOk ? 4 : (inOrderOk && !(batchOk && top_k < dbs && lds <= g.ldsBatch) ? 0 : (batchOk ? 5 : 3)));
     if (v == 5 && inOrderOk) p.ldsInOrder = lds;
     const int f = g.forcedSieveVariant;
     if (f == 0 && inOrderOk) v = 0;
@@ -973,7 +976,8 @@ int kvx_sieve_update(uint64_t topk_indices, uint64_t req_pool_indices, uint64_t 
             const StreamScratch &sc =
                 ScratchFor(stream, SieveScratchNeed(plan, max_num_reqs, static_cast<uint32_t>(htSize)), "sieve_update");
             hipCheck(kvx::launch_sieve_update_batch(a, reinterpret_cast<uint64_t>(g.overflow), sc.shadow, sc.aux,
-                                                    plan.rebuild ? sc.tbl : nullptr, AsStream(stream)),
+                                                    plan.rebuild ? sc.tbl : nullptr,
+                                                    static_cast<uint32_t>(plan.ldsInOrder), AsStream(stream)),
                      "hisp_sieve_update launch");
         } else {
             hipCheck(kvx::launch_sieve_update(a, reinterpret_cast<uint64_t>(g.overflow), plan.variant,

@@ -39,6 +39,10 @@ constexpr int32_t kHandStride = 16;
 // consistent with its tokens (every live token findable at its own slot, one
 // entry per live slot); any other writer of the row clears it.
 constexpr int32_t kCanonFlag = 0x4B565843;
+// The same word after an in-order step in LDS by the batch kernel on a row that
+// holds tokens past its map: the next step goes in order without the check,
+// which would find them again (every step sets the word anew).
+constexpr int32_t kInOrderFlag = 0x4B56584F;
 // sieve_hand[row][3]: written with the flag, the sum over slots [0, dbs) of
 // slot_token_mix(slot, token) (mod 2^32) of the tokens the kernel left.  A
 // flagged row is trusted only while its tokens still sum to it, so a token
@@ -361,9 +365,11 @@ hipError_t launch_sieve_update_wave(const HispSieveUpdateArgs &a, uint64_t overf
 hipError_t launch_sieve_update_fast(const HispSieveUpdateArgs &a, uint64_t overflowSlot, size_t ldsBytes,
                                     bool compact, hipStream_t stream);
 // tbl: the rebuild's scratch (rows of table_layout(htSize).words), or null
-// for the table changes applied inside the batch kernel.
+// for the table changes applied inside the batch kernel.  ldsRow: bytes of a
+// state row that LDS can hold (padded tokens, table, visited bits), whose
+// in-order steps then run there, or 0.
 hipError_t launch_sieve_update_batch(const HispSieveUpdateArgs &a, uint64_t overflowSlot, int32_t *shadow,
-                                     uint32_t *aux, uint32_t *tbl, hipStream_t stream);
+                                     uint32_t *aux, uint32_t *tbl, uint32_t ldsRow, hipStream_t stream);
 hipError_t sieve_batch_set_lds_limit(size_t bytes);
 // The table rebuild after the batch kernel (rows it left pending), on the
 // same stream; table_rebuild_ok: the shape's windows fit (htSize <= kTblMaxHt).

@@ -52,6 +52,10 @@
 //     with step 4 this is the table the in-order recurrence leaves, which
 //     equals inserting the live tokens in the order they were inserted.  The
 //     row's consistency flag is then set (cleared on the in-order path).
+//
+// The in-order recurrence runs on HBM, or in LDS for a row that fits there
+// (the sequential LDS kernel's); a row that holds tokens past the map is then
+// marked, so that its next step skips the check.
 #include "kvx_internal.h"
 #include "sieve_hbm.h"
 #include "sieve_local.h"
@@ -83,6 +87,7 @@ struct BatchParams {
     uint32_t *tbl;      // the rebuild's scratch [maxNumReqs][t.words], or null: a step with
                         // misses then applies its table changes here (phases 4, 5)
     TableLayout t;
+    uint32_t ldsRow;    // bytes of the state row where the launch's LDS holds it (0: it does not)
 };
 
 __device__ __forceinline__ int bit_get(const uint64_t *b, uint32_t i) { return (b[i >> 6] >> (i & 63)) & 1; }
@@ -814,6 +819,8 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
     // a row this kernel (or the LDS kernel) left consistent: the table scans
     // of the check are skipped, its live tokens and entries still counted
     const bool flagged = flagWord == kCanonFlag;
+    // a row known to need the in-order recurrence, which runs in LDS
+    const bool inOrder = P.ldsRow != 0u && flagWord == kInOrderFlag;
     const BatchLayout &y = P.lay;
     uint64_t *visB = reinterpret_cast<uint64_t *>(lds + y.vis);
     uint64_t *evB = reinterpret_cast<uint64_t *>(lds + y.ev);
@@ -839,7 +846,7 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
 #endif
     // ---- 1. check ------------------------------------------------------
     if (tid == 0) {
-        sBad = 0;
+        sBad = inOrder ? 1 : 0;
         sWrap = 0;
         sLive = 0;
         sOcc = 0;
@@ -877,7 +884,7 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
     }
     __syncthreads();
     const bool useBits = sBits != 0;
-    if (!useBits) {
+    if (!useBits && !inOrder) {
         // the map by plain stores; a token held by two slots is found when
         // the map is read back below (one of them reads the other's slot).
         // kMapUnroll slots' tokens are loaded before any is used (one memory
@@ -1284,7 +1291,7 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
 
     // the map and first-occurrence scratch are left zeroed (tokens still the
     // initial ones here)
-    for (int32_t s0 = tid; s0 < dbs && !useBits; s0 += BT * kMapUnroll) {
+    for (int32_t s0 = tid; s0 < dbs && !useBits && !inOrder; s0 += BT * kMapUnroll) {
         int32_t tv[kMapUnroll];
 #pragma unroll
         for (int q = 0; q < kMapUnroll; ++q) {
@@ -1316,6 +1323,40 @@ __global__ __launch_bounds__(BT) void kvx_sieve_update_batch(BatchParams P)
         // the in-order recurrence on the untouched row, which the next launch
         // checks in full
         if (tid == 0) gHand[1] = 0;
+        // On the row staged in LDS where it fits (a row that the sequential LDS
+        // kernel would take as well): 4 rows of 10000 slots and 2000 positions
+        // with tokens past the map 1222 us a call, 2823 in HBM, 1270 on that
+        // kernel.
+        if (P.ldsRow != 0u) {
+            int32_t *tok = reinterpret_cast<int32_t *>(lds);
+            uint16_t *ht = reinterpret_cast<uint16_t *>(lds + static_cast<size_t>(padded) * 4u);
+            uint8_t *vis = lds + static_cast<size_t>(padded) * 4u + static_cast<size_t>(H) * 2u;
+            sieve::block_copy16(tok, (const int32_t *)r.tok, static_cast<uint32_t>(padded) * 4u);
+            sieve::block_copy16(ht, (const uint16_t *)r.ht, static_cast<uint32_t>(H) * 2u);
+            sieve::block_copy16(vis, (const uint32_t *)r.vis32, static_cast<uint32_t>(visStrideB));
+            __syncthreads();
+            if (tid < 64) {
+                int32_t hand = hand0 < 0 || hand0 >= dbs ? 0 : hand0;
+                sieve::Guard g;
+                const bool dirty = sieve::sieve_row_wave((const int32_t *)rt, (int32_t *)rs, (int8_t *)rm, K, seqLen, prefill,
+                                                         dbs, padded, H - 1, tok, vis, ht, hand, g);
+                if (tid == 0) {
+                    gHand[0] = hand;
+                    sMisses = dirty ? 1 : 0;
+                    sieve::report_overflow(P.L.overflowSlot, g.code);
+                }
+            }
+            __syncthreads();
+            int32_t past = 0;
+            for (int32_t s = tid; s < dbs; s += BT) past |= tok[s] >= static_cast<int32_t>(P.mapCap) ? 1 : 0;
+            if (__syncthreads_or(past) && tid == 0) gHand[1] = kInOrderFlag;
+            sieve::block_copy16((uint32_t *)r.vis32, vis, static_cast<uint32_t>(visStrideB));
+            if (sMisses != 0) {
+                sieve::block_copy16((int32_t *)r.tok, tok, static_cast<uint32_t>(padded) * 4u);
+                sieve::block_copy16((uint16_t *)r.ht, ht, static_cast<uint32_t>(H) * 2u);
+            }
+            return;
+        }
         build_shadow(r);
         __threadfence_block();
         __syncthreads();
@@ -1880,7 +1921,7 @@ hipError_t sieve_batch_set_lds_limit(size_t bytes)
 }
 
 hipError_t launch_sieve_update_batch(const HispSieveUpdateArgs &a, uint64_t overflowSlot, int32_t *shadow,
-                                     uint32_t *aux, uint32_t *tbl, hipStream_t stream)
+                                     uint32_t *aux, uint32_t *tbl, uint32_t ldsRow, hipStream_t stream)
 {
     BatchParams P{};
     P.L = KvxLaunch<HispSieveUpdateArgs>{a, overflowSlot};
@@ -1895,7 +1936,9 @@ hipError_t launch_sieve_update_batch(const HispSieveUpdateArgs &a, uint64_t over
     hipLaunchKernelGGL(kvx_sieve_batch_slots, dim3(kPreSplit, a.maxNumReqs), dim3(kPreThreads), 0, stream, P);
     // the table update at the kernel's end takes the decisions' LDS again
     const uint32_t local = tbl == nullptr ? 0u : table_local::lds_bytes(a.htSize < table_local::kLocalCells ? a.htSize : table_local::kLocalCells);
-    const uint32_t ldsBytes = local > P.lay.total ? local : P.lay.total;
+    uint32_t ldsBytes = local > P.lay.total ? local : P.lay.total;
+    P.ldsRow = ldsRow;
+    if (ldsRow > ldsBytes) ldsBytes = ldsRow;
     hipLaunchKernelGGL(kvx_sieve_update_batch, dim3(a.maxNumReqs), dim3(BT), ldsBytes, stream, P);
     if (tbl != nullptr) {
         const hipError_t err = hipGetLastError();

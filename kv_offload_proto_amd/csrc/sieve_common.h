@@ -251,7 +251,7 @@ __device__ __forceinline__ void wave_shift_lds(uint16_t *ht, const int32_t *tok,
     g.code = kOverflowProbe;
 }
 
-__device__ bool sieve_row_wave(const int32_t *rt, int32_t *rs, int8_t *rm, int32_t topK, int32_t seqLen,
+__device__ __forceinline__ bool sieve_row_wave(const int32_t *rt, int32_t *rs, int8_t *rm, int32_t topK, int32_t seqLen,
                                int32_t prefill, int32_t dbs, int32_t padded, int32_t mask, int32_t *tok, uint8_t *vis,
                                uint16_t *ht, int32_t &hand, Guard &g)
 {
