@@ -289,9 +289,9 @@ StreamScratch &ScratchFor(uint64_t stream, const ScratchNeed &need, const char *
 // HBM-resident kernel (state in HBM, decisions and bitmaps in LDS), 0 =
 // sequential LDS kernel, 3 = sequential HBM-resident kernel with wave-wide
 // probes (1 = the single-lane HBM kernel, only when forced).  A row that fits
-// LDS but neither parallel layout (about 9000 to 15000 slots at 900 and more
-// positions) takes the batch kernel: 9 rows of 9370 slots and 1655 positions
-// 1060 us a call on the sequential one, 70 on the batch kernel (in both cases
+// LDS but neither parallel layout (about 9500 to 15000 slots at 900 and more
+// positions) takes the batch kernel: 9 rows of 10000 slots and 2000 positions
+// 998 us a call on the sequential one, 58 on the batch kernel (in both cases
 // without tokens past the batch kernel's map; with some the batch kernel runs
 // the sequential recurrence in LDS itself).  With as many
 // positions as slots a slot can be evicted twice in a step, which the batch

@@ -109,7 +109,7 @@ __host__ __device__ __forceinline__ uint64_t export_rows_win_entries(uint32_t pe
 constexpr int kFastThreads = KVX_FAST_THREADS;
 
 struct FastLayout {
-    uint32_t tok, ht, vis, ptok, pinf, vt, evslot, smKp, eseq, tb, smA, smB, vset, ber, occ, fin, nkb, cmask, emask,
+    uint32_t tok, ht, vis, ptok, pinf, vt, evslot, smKp, eseq, tb, smA, smB, vset, ber, occ, fin, rnk, cmask, emask,
         smask, rsn, rsm, total;
 };
 
@@ -125,8 +125,8 @@ __host__ __device__ __forceinline__ uint32_t align16(uint32_t x) { return (x + 1
 // cmask/emask/smask/rsn/rsm hold one 64-bit ballot per (wave, block of one
 // entry per lane).  ber, occ and fin are one bit per table cell: cells of
 // evicted tokens, the pre-step occupancy, the occupancy as the erase changes
-// it.  nkb (htSize / 8 bytes, at least 128): the event order of up to 64 slots
-// (rows decided in registers).
+// it.  rnk: the event order of up to 64 slots (rows decided in registers).
+constexpr uint32_t kRankBytes = 64u * 2u;
 __host__ __device__ __forceinline__ FastLayout fast_layout(uint32_t padded, uint32_t htSize, uint32_t topK,
                                                            uint32_t visStrideB, bool compact = false)
 {
@@ -157,7 +157,7 @@ __host__ __device__ __forceinline__ FastLayout fast_layout(uint32_t padded, uint
     l.rsn = o;     o += ringMaskBytes;
     l.rsm = o;     o += ringMaskBytes;
     l.fin = o;     o += align16(bmBytes);
-    l.nkb = o;     o += align16(bmBytes);
+    l.rnk = o;     o += kRankBytes;
     l.total = o;
     return l;
 }
@@ -208,12 +208,12 @@ __host__ __device__ __forceinline__ FastLayout fast_layout_fixed(uint32_t padded
     // the bitmap that the erase changes and the event orders take the
     // per-position classes' region, which the fixed kernels keep in registers
     // instead
-    if (2u * align16(htSize / 8u) <= Kx * 4u) {
+    if (align16(htSize / 8u) + kRankBytes <= Kx * 4u) {
         l.fin = l.pinf;
-        l.nkb = l.pinf + align16(htSize / 8u);
+        l.rnk = l.pinf + align16(htSize / 8u);
     } else {
         l.fin = o;  o += align16(htSize / 8u);
-        l.nkb = o;  o += align16(htSize / 8u);
+        l.rnk = o;  o += kRankBytes;
     }
     l.total = o;
     return l;

@@ -413,7 +413,7 @@ __global__ __launch_bounds__(NT) void kvx_sieve_update_fast(KvxLaunch<HispSieveU
     uint8_t *occ8 = smem + lay.occ;
     uint32_t *fin = reinterpret_cast<uint32_t *>(smem + lay.fin);   // occupied cells as the erase changes them
     uint8_t *fin8 = smem + lay.fin;
-    uint16_t *evRank = reinterpret_cast<uint16_t *>(smem + lay.nkb);  // rows decided in registers: the slots' event order
+    uint16_t *evRank = reinterpret_cast<uint16_t *>(smem + lay.rnk);  // rows decided in registers: the slots' event order
     uint64_t *cmask = reinterpret_cast<uint64_t *>(smem + lay.cmask);  // first occurrences of candidates
     uint64_t *emask = reinterpret_cast<uint64_t *>(smem + lay.emask);  // conversion positions
     uint64_t *smask = reinterpret_cast<uint64_t *>(smem + lay.smask);  // evicted SM slots

@@ -42,9 +42,10 @@ static void check_fast(uint32_t padded, uint32_t H, uint32_t K, uint32_t dbs, ui
     if (!finShared) {
         r.push_back({"pinf", l.pinf, Kx * 4u});
         r.push_back({"fin", l.fin, bm});
-        r.push_back({"nkb", l.nkb, bm});
+        r.push_back({"rnk", l.rnk, kvx::kRankBytes});
     } else {
-        CHECK(l.nkb + bm <= l.pinf + Kx * 4u);
+        CHECK(l.fin + bm <= l.rnk);
+        CHECK(l.rnk + kvx::kRankBytes <= l.pinf + Kx * 4u);
     }
     for (const Region &x : r) {
         CHECK(x.off % 16u == 0u);

@@ -1354,11 +1354,11 @@ def test_sieve_table_rebuild_cluster_edges(kvops, case):
     assert kvops.read_overflow() == 0
 
 
-@pytest.mark.parametrize("dbs,top_k,want", [(9370, 1655, 5), (10000, 2000, 5), (12000, 1200, 5), (15000, 1000, 5), (700, 16383, 0)])
+@pytest.mark.parametrize("dbs,top_k,want", [(9370, 1655, 4), (10000, 2000, 5), (12000, 1200, 4), (15000, 1000, 5), (700, 16383, 0)])
 def test_sieve_rows_between_the_layouts(kvops, dbs, top_k, want):
-    """Rows that fit LDS but neither layout of the parallel kernel: the batch
-    kernel, or the sequential one with as many positions as slots; full state
-    against the oracle after every step."""
+    """Rows about and past the end of the parallel kernel's layouts: that kernel's
+    compact layout, the batch kernel, or the sequential one with as many
+    positions as slots; full state against the oracle after every step."""
     rng = np.random.default_rng(dbs)
     req, prefill = 2, dbs + 3000
     st = orc.SieveState(1, req, dbs, top_k)
@@ -1387,7 +1387,7 @@ def _past_the_map(rng, dbs, top_k, req, prefill):
     return st, DevSieve(st)
 
 
-@pytest.mark.parametrize("dbs,top_k", [(9370, 1700), (10000, 2000), (15000, 1000)])
+@pytest.mark.parametrize("dbs,top_k", [(11000, 1500), (10000, 2000), (15000, 1000)])
 def test_sieve_between_the_layouts_past_the_map(kvops, dbs, top_k):
     """Rows between the layouts with tokens past the batch kernel's map (2^18):
     its in-order recurrence in LDS, full state against the oracle.  Steps: all
