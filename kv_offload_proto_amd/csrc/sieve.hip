@@ -282,7 +282,8 @@ __device__ __forceinline__ void init_table_lds(uint8_t *smem, const RowTokens<kI
 // one-wave sweep below, whose time does not depend on the distances.
 //
 // A token held twice, or one beyond the bitmap that finds those, sends the
-// row to the one-lane inserts.
+// row to the one-lane inserts.  Rows of more than 65535 slots are swept (two
+// of 70000 random tokens 7 ms; minutes with one lane on the table in HBM).
 //
 // Against the sweep alone: four tables of 65518 slots, admission pattern, 4541
 // -> 175 us with the calls around the build; 64 tables of 16000 random tokens
@@ -300,7 +301,7 @@ struct InitLargeLds {
     uint64_t occ[kInitWords], spill[kInitWords];
     uint64_t full[kInitWords / 64];
     uint32_t part[kInitThreads / 64 + 1];
-    int32_t inOrder, stop;
+    int32_t stop;
 };
 static_assert(kWaveInitTokenBits / 8 <= sizeof(InitLargeLds::cells), "the token bitmap takes the cells' place");
 static_assert(kInitWords == kInitThreads, "one bitmap word per lane");
@@ -400,7 +401,8 @@ __device__ void init_table_sweep(uint8_t *smem, const RowTokens<kIdentity> token
         const int32_t s = (bi << 6) + lane;
         const int32_t t = tNext;
         tNext = s + 64 < dbs ? token(s + 64) : -1;  // the next batch's tokens, in flight meanwhile
-        const bool valid = s < dbs && t >= 0;
+        // (an entry is slot + 1 in 16 bits: slot 65535 writes an empty cell)
+        const bool valid = s < dbs && t >= 0 && (s & 0xFFFF) != 0xFFFF;
         const uint64_t keys = __ballot(valid);
         if (keys == 0ull) continue;
         const int32_t h = valid ? static_cast<int32_t>(ht_hash(t)) & mask : 0;
@@ -565,16 +567,24 @@ __device__ __forceinline__ void init_table_large(uint8_t *smem, const RowTokens<
     InitLargeLds &l = *reinterpret_cast<InitLargeLds *>(smem);
     const int32_t tid = threadIdx.x;
     constexpr int32_t NT = kInitThreads;
-    const int32_t zeroEnd = H < kInitTailEnd ? H : kInitTailEnd;  // the helpers clear the rest
+    // rows past 16-bit slots (no helpers; never at admission)
+    const bool huge = !kIdentity && dbs >= kInitHomes;
+    const int32_t zeroEnd = H < kInitTailEnd || huge ? H : kInitTailEnd;  // the helpers clear the rest
     auto clear_cells = [&]() {
         for (int32_t i = tid; i < kInitHomes / 8; i += NT) reinterpret_cast<uint4 *>(l.cells)[i] = make_uint4(0, 0, 0, 0);
     };
     auto clear_table = [&]() {
         for (int32_t i = tid; i < zeroEnd / 8; i += NT) reinterpret_cast<GChunk *>(gHt)[i] = Chunk{0u, 0u, 0u, 0u};
     };
+    auto sweep = [&]() {
+        clear_table();
+        __threadfence_block();
+        __syncthreads();
+        if (tid < 64) init_table_sweep<kIdentity>(smem, token, gHt, dbs, H, overflowSlot);
+    };
     clear_cells();
     l.spill[tid] = 0ull;
-    if (tid == 0) l.inOrder = l.stop = 0;
+    if (tid == 0) l.stop = 0;
     __syncthreads();
     if constexpr (!kIdentity) {
         // repeated and out-of-range tokens
@@ -607,6 +617,10 @@ __device__ __forceinline__ void init_table_large(uint8_t *smem, const RowTokens<
                 }
                 report_overflow(overflowSlot, g.code);
             }
+            return;
+        }
+        if (huge) {
+            sweep();
             return;
         }
         clear_cells();
@@ -664,10 +678,7 @@ __device__ __forceinline__ void init_table_large(uint8_t *smem, const RowTokens<
         }
         __syncthreads();
         if (l.stop) {
-            clear_table();
-            __threadfence_block();
-            __syncthreads();
-            if (tid < 64) init_table_sweep<kIdentity>(smem, token, gHt, dbs, H, overflowSlot);
+            sweep();
             return;
         }
         done = end;
@@ -840,8 +851,8 @@ size_t sieve_ht_init_small_lds(uint32_t htSize, uint32_t dbs)
 
 size_t sieve_ht_init_large_lds(uint32_t htSize, uint32_t dbs)
 {
-    // slots below 65535: an entry is 16 bits
-    if (htSize < static_cast<uint32_t>(kInitHomes) || htSize > (1u << 20) || dbs > 65535u) return 0;
+    // fewer keys than cells
+    if (htSize < static_cast<uint32_t>(kInitHomes) || htSize > (1u << 20) || dbs >= htSize) return 0;
     const size_t sweep = htSize / 8u + htSize / 512u + 8u * ((htSize + 262143u) / 262144u);
     return sweep > sizeof(InitLargeLds) ? sweep : sizeof(InitLargeLds);
 }
@@ -867,7 +878,9 @@ hipError_t launch_sieve_ht_init(const HispSieveHtInitArgs &a, uint64_t overflowS
         const uint32_t threads = a.deviceBufferSize <= static_cast<uint32_t>(kInitSmallSlots) ? kInitSmallThreads : kInitThreads;
         hipLaunchKernelGGL(kvx_sieve_ht_init_par<false>, grid, dim3(threads), ldsBytes, stream, L);
     } else if (form == InitForm::kLarge) {
-        const uint32_t parts = a.htSize > static_cast<uint32_t>(kInitTailEnd) ? 1u + kInitHelpers : 1u;
+        // (the rows of more than 65535 slots may take cells past kInitTailEnd)
+        const bool tail = a.htSize > static_cast<uint32_t>(kInitTailEnd) && a.deviceBufferSize < static_cast<uint32_t>(kInitHomes);
+        const uint32_t parts = tail ? 1u + kInitHelpers : 1u;
         hipLaunchKernelGGL(kvx_sieve_ht_init_par<true>, dim3(grid.x, parts), dim3(kInitThreads), ldsBytes, stream, L);
     } else if (ldsBytes != 0) {
         hipLaunchKernelGGL(kvx_sieve_ht_init<true>, grid, block, ldsBytes, stream, L);

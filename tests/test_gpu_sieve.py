@@ -180,6 +180,33 @@ def test_ht_init_packed_homes(kvops, dbs, top_k, homes):
     assert kvops.read_overflow() == 0
 
 
+@pytest.mark.parametrize("homes", ["random", "packed"])
+@pytest.mark.parametrize("dbs,top_k", [(65535, 64), (65536, 64), (70000, 64)])
+def test_ht_init_full_rows(kvops, dbs, top_k, homes):
+    """Rows at and past 16-bit slots with every slot in use: random tokens, or
+    tokens homed in a sixteenth of the homes."""
+    rng = np.random.default_rng(dbs + len(homes))
+    st = orc.SieveState(1, 2, dbs, top_k)
+    t = np.arange(0, 1 << 20, dtype=np.int64)
+    near = t[_home(t, 65536) < 4096]
+    st.tokens[:] = -1
+    for r in range(2):
+        vals = rng.permutation(t)[:dbs]
+        if homes == "packed":
+            vals = np.full(dbs, -1)
+            n = min(dbs, len(near))
+            vals[rng.choice(dbs, size=n, replace=False)] = rng.permutation(near)[:n]
+        st.tokens[0, r, :dbs] = vals
+    dev = DevSieve(st)
+    dev.ht.fill_(77)
+    st.ht[:] = 77
+    orc.sieve_ht_init(st.tokens, st.ht, 0, 2, 1, 2, dbs, st.padded, st.ht_size)
+    kvops.sieve_ht_init(dev.tokens.data_ptr(), dev.ht.data_ptr(), dev.prefill.data_ptr(), 0, 2, 1, 2, dbs, st.padded,
+                        st.ht_size, 0, 0)
+    np.testing.assert_array_equal(dev.ht.cpu().numpy().view(np.uint16), st.ht)
+    assert kvops.read_overflow() == 0
+
+
 @pytest.mark.parametrize("dbs,top_k,prefills", [
     (1, 16, [0, 1, 5]), (64, 64, [63, 64, 256]), (1000, 333, [1, 999, 3777]), (8192, 2048, [8191, 8192, 16384]),
     (16370, 8, [16370, 40000]), (16384, 2048, [16383, 131072]), (65518, 8192, [300, 65518, 131072])])
@@ -1265,7 +1292,8 @@ def test_sieve_table_update_refused_late(kvops, kinds):
     assert st.ht_size == 65536
     order = np.argsort(_home(np.arange(prefill, dtype=np.int64), 65536), kind="stable")
     homes = _home(order, 65536)
-    by_home = [order[np.searchsorted(homes, h):np.searchsorted(homes, h, "right")] for h in range(65536)]
+    cut = np.searchsorted(homes, np.arange(65537))
+    by_home = [order[cut[h]:cut[h + 1]] for h in range(65536)]
     steps = 4
     batch = np.full((steps, req, top_k), -1, dtype=np.int32)
     for r, kind in enumerate(kinds):
