@@ -277,9 +277,20 @@ __device__ __forceinline__ void init_table_lds(uint8_t *smem, const RowTokens<kI
 // The slots go in increasing passes, each half of the cells left free, so
 // that the proposals of a pass stay few however full the table gets; a cell
 // taken in an earlier pass holds a smaller slot and is skipped by a bitmap
-// (occ, with a bit per full word in `full`).  A chain of more than
-// kInitMaxHops proposals (homes packed into few cells) sends the row to the
-// one-wave sweep below, whose time does not depend on the distances.
+// (occ, with a bit per full word in `full`).  A pass is at least one slot per
+// lane while the chains are short (homes spread evenly, as at admission), else
+// at least kInitSmallPass: with the last 1006 of 65518 random tokens on 1024
+// free cells in one pass, chains passed the limit below and the row was swept
+// after all (four tables 6705 us, 1142 so).
+//
+// Homes packed into few cells make the proposals many (the square of the keys
+// on one home): the row takes the one-wave sweep below, whose time does not
+// depend on the distances.  A sample of the slots (every fourth, over 4096) is
+// counted per 256 homes beforehand; more than twice the even share and 32 in
+// one of them sends the row there (random tokens: ten and more standard
+// deviations), and so does a chain of more than kInitMaxHops proposals.  (1024
+// keys on the last 64 homes of a 65536-cell table: 577 us swept, 2799 when
+// only the chains told.)
 //
 // A token held twice, or one beyond the bitmap that finds those, sends the
 // row to the one-lane inserts.  Rows of more than 65535 slots are swept (two
@@ -292,6 +303,9 @@ constexpr int32_t kWaveInitTokenBits = 1 << 20;
 constexpr int32_t kFreeCap = 4;  // free cells counted between neighbouring first-free cells
 constexpr int32_t kInitHomes = 65536;
 constexpr int32_t kInitMaxHops = 512;
+constexpr int32_t kInitLongChain = 16;                    // proposals past which later passes get smaller
+constexpr int32_t kInitSmallPass = 64;                    // their least slots
+constexpr int32_t kInitBuckets = 256;                     // sampled counts, of 256 homes each
 constexpr int32_t kInitWords = kInitHomes / 64;           // words of the occ and spill bitmaps
 constexpr int32_t kInitTailEnd = 2 * kInitHomes;          // no cell at or past it is ever taken
 constexpr int32_t kInitHelpers = 3;                       // workgroups per row beside the one that builds
@@ -301,7 +315,8 @@ struct InitLargeLds {
     uint64_t occ[kInitWords], spill[kInitWords];
     uint64_t full[kInitWords / 64];
     uint32_t part[kInitThreads / 64 + 1];
-    int32_t stop;
+    uint32_t bucket[kInitBuckets];
+    int32_t longChain, stop;
 };
 static_assert(kWaveInitTokenBits / 8 <= sizeof(InitLargeLds::cells), "the token bitmap takes the cells' place");
 static_assert(kInitWords == kInitThreads, "one bitmap word per lane");
@@ -584,10 +599,13 @@ __device__ __forceinline__ void init_table_large(uint8_t *smem, const RowTokens<
     };
     clear_cells();
     l.spill[tid] = 0ull;
-    if (tid == 0) l.stop = 0;
+    if (!kIdentity && tid < kInitBuckets) l.bucket[tid] = 0u;
+    if (tid == 0) l.longChain = l.stop = 0;
     __syncthreads();
     if constexpr (!kIdentity) {
-        // repeated and out-of-range tokens
+        // repeated and out-of-range tokens; packed homes among the sampled slots
+        const int32_t sampled = dbs <= kInitUnroll * NT ? (dbs < NT ? dbs : NT) : dbs / kInitUnroll;
+        const uint32_t packed = 32u + 2u * static_cast<uint32_t>(sampled / kInitBuckets);
         bool inOrder = false;
         for (int32_t s0 = tid; s0 < dbs; s0 += kInitUnroll * NT) {
             int32_t t[kInitUnroll];
@@ -596,6 +614,9 @@ __device__ __forceinline__ void init_table_large(uint8_t *smem, const RowTokens<
 #pragma unroll
             for (int q = 0; q < kInitUnroll; ++q) {
                 if (t[q] < 0) continue;
+                // (the last homes' keys leave a larger table's homes at once)
+                const uint32_t b = ht_hash(t[q]) / (kInitHomes / kInitBuckets);
+                if (q == 0 && (b < kInitBuckets - 1 || H == kInitHomes) && atomicAdd(&l.bucket[b], 1u) >= packed) l.stop = 1;
                 if (t[q] >= kWaveInitTokenBits) {
                     inOrder = true;
                     continue;
@@ -619,7 +640,7 @@ __device__ __forceinline__ void init_table_large(uint8_t *smem, const RowTokens<
             }
             return;
         }
-        if (huge) {
+        if (l.stop != 0 || huge) {
             sweep();
             return;
         }
@@ -642,10 +663,12 @@ __device__ __forceinline__ void init_table_large(uint8_t *smem, const RowTokens<
         }
         return kInitHomes;
     };
+    int32_t least = NT;  // slots of a pass (at admission the chains are short)
     for (int32_t done = 0; done < dbs;) {
         const int32_t half = (kInitHomes - done) / 2;
-        const int32_t end = min(dbs, done + (half > NT ? half : NT));
+        const int32_t end = min(dbs, done + (half > least ? half : least));
         const bool later = done > 0;
+        bool longChain = false;
         for (int32_t s0 = done + tid; s0 < end; s0 += kInitUnroll * NT) {
             int32_t t[kInitUnroll];
 #pragma unroll
@@ -655,7 +678,8 @@ __device__ __forceinline__ void init_table_large(uint8_t *smem, const RowTokens<
                 if (t[q] < 0) continue;
                 uint32_t v = static_cast<uint32_t>(s0 + q * NT) + 1u;
                 uint32_t c = ht_hash(t[q]);  // 16 bits: the home
-                for (int32_t hops = 0;; ++hops) {
+                int32_t hops = 0;
+                for (;; ++hops) {
                     if (later) c = next_free(c);
                     if (c >= static_cast<uint32_t>(kInitHomes)) {
                         if (!wraps) {
@@ -673,10 +697,18 @@ __device__ __forceinline__ void init_table_large(uint8_t *smem, const RowTokens<
                         break;
                     }
                 }
+                if constexpr (!kIdentity) longChain = longChain || hops > kInitLongChain;
             }
             if (*const_cast<volatile int32_t *>(&l.stop)) break;
         }
+        if constexpr (!kIdentity) {
+            if (longChain) l.longChain = 1;
+        }
         __syncthreads();
+        // (neither word is set again before the next barrier)
+        if constexpr (!kIdentity) {
+            if (l.longChain != 0) least = kInitSmallPass;
+        }
         if (l.stop) {
             sweep();
             return;

@@ -180,11 +180,13 @@ def test_ht_init_packed_homes(kvops, dbs, top_k, homes):
     assert kvops.read_overflow() == 0
 
 
-@pytest.mark.parametrize("homes", ["random", "packed"])
-@pytest.mark.parametrize("dbs,top_k", [(65535, 64), (65536, 64), (70000, 64)])
+@pytest.mark.parametrize("homes", ["random", "packed", "late"])
+@pytest.mark.parametrize("dbs,top_k", [(20000, 2048), (65518, 8192), (65535, 64), (65536, 64), (70000, 64)])
 def test_ht_init_full_rows(kvops, dbs, top_k, homes):
-    """Rows at and past 16-bit slots with every slot in use: random tokens, or
-    tokens homed in a sixteenth of the homes."""
+    """Large tables of rows with every slot in use: random tokens (at the slot
+    limit the last passes fill every home), tokens homed in a sixteenth of the
+    homes (the sampled counts send the row to the sweep), or such tokens only in
+    slots that are not sampled (its chains do); rows past 16-bit slots are swept."""
     rng = np.random.default_rng(dbs + len(homes))
     st = orc.SieveState(1, 2, dbs, top_k)
     t = np.arange(0, 1 << 20, dtype=np.int64)
@@ -196,6 +198,10 @@ def test_ht_init_full_rows(kvops, dbs, top_k, homes):
             vals = np.full(dbs, -1)
             n = min(dbs, len(near))
             vals[rng.choice(dbs, size=n, replace=False)] = rng.permutation(near)[:n]
+        elif homes == "late":
+            late = np.flatnonzero(np.arange(dbs) % 4096 >= 1024)[:len(near)]
+            vals = np.full(dbs, -1)
+            vals[late] = rng.permutation(near)[:len(late)]
         st.tokens[0, r, :dbs] = vals
     dev = DevSieve(st)
     dev.ht.fill_(77)
@@ -205,6 +211,34 @@ def test_ht_init_full_rows(kvops, dbs, top_k, homes):
                         st.ht_size, 0, 0)
     np.testing.assert_array_equal(dev.ht.cpu().numpy().view(np.uint16), st.ht)
     assert kvops.read_overflow() == 0
+
+
+def test_ht_init_random_tokens_at_the_slot_limit_stay_parallel(kvops):
+    """65518 random tokens take a few times as long as the admission pattern
+    (four tables: 6705 us when the row was swept after all, 1142 so, 76 for the
+    pattern)."""
+    import torch
+
+    dbs, top_k = 65518, 8192
+    best = {}
+    for kind in ("pattern", "random"):
+        st = orc.SieveState(1, 4, dbs, top_k)
+        for r in range(4):
+            st.tokens[0, r, :dbs] = np.arange(dbs) if kind == "pattern" else np.random.default_rng(r).permutation(1 << 20)[:dbs]
+        dev = DevSieve(st)
+        us = []
+        for _ in range(6):
+            t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            torch.cuda.synchronize()
+            t0.record()
+            kvops.sieve_ht_init(dev.tokens.data_ptr(), dev.ht.data_ptr(), dev.prefill.data_ptr(), 0, 4, 1, 4, dbs, st.padded,
+                                st.ht_size, 0, 0)
+            t1.record()
+            torch.cuda.synchronize()
+            us.append(t0.elapsed_time(t1) * 1e3)
+        best[kind] = min(us)
+    print("ht_init", best, flush=True)
+    assert best["random"] < 20 * best["pattern"], best
 
 
 @pytest.mark.parametrize("dbs,top_k,prefills", [
