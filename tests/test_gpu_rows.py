@@ -121,15 +121,20 @@ def test_gather_parity_after_sieve(kvops, stride_mode, fused):
 
 
 @pytest.mark.parametrize("req,top_k,num_real,S,N,stride_mode,fused,block_dim", [
-    (3, 1500, 2, 1, 2, "padded", True, 3),    # 4500 positions: 18 chunks, the last one partial
-    (3, 1500, 3, 64, 4, "zero", False, 2),    # stride 0: requests collide on hot rows
-    (5, 4096, 5, 1, 3, "padded", True, 8),    # 80 chunks over the 64 workgroups
-    (2, 2049, 1, 1, 1, "zero", True, 1),      # 4098 positions: just past the one-launch form
-    (3, 1500, 3, 1, 2, "wide", True, 2),      # stride 70000: winner rows spaced 65536 apart
+    (3, 1500, 2, 1, 2, "padded", True, 3),    # one launch: spans of 16, the last one of a request partial
+    (3, 1500, 3, 64, 4, "zero", False, 2),    # two launches (striped): requests collide on hot rows
+    (5, 4096, 5, 1, 3, "padded", True, 8),    # one launch: spans of 32 over the 256 workgroups
+    (2, 2049, 1, 1, 1, "zero", True, 1),      # one launch: one group of 4098 positions
+    (3, 1500, 3, 1, 2, "wide", True, 2),      # stride 70000: rows of a request spaced 65536 apart
+    (3, 1500, 2, 16, 2, "padded", True, 3),   # two launches: 18 chunks, the last one partial
+    (3, 3000, 3, 1, 2, "zero", True, 8),      # ... (stride 0 past 8192 positions)
+    (5, 8200, 4, 1, 3, "padded", True, 8),    # ... (requests past 8192 positions): 161 chunks over 64 workgroups
+    (2, 8200, 2, 1, 1, "wide", True, 2),      # ... winner rows spaced 65536 apart
 ])
 def test_gather_large_batch_parity(kvops, req, top_k, num_real, S, N, stride_mode, fused, block_dim):
-    """The large-batch import (winner tags, then workgroups claiming chunks of
-    positions) against the oracle on constructed inputs: duplicate and
+    """The import of larger batches, in one launch or in two (winner tags, then
+    workgroups claiming chunks of positions; the comments say which), against
+    the oracle on constructed inputs: duplicate and
     colliding destinations (the last valid miss wins), invalid tokens and
     slots, a request without a pool row, num_real below max_num_reqs, partial
     chunks; every hot byte and every node's status words."""
@@ -176,20 +181,18 @@ def test_gather_large_batch_parity(kvops, req, top_k, num_real, S, N, stride_mod
 
 
 @pytest.mark.parametrize("req,top_k,dbs,stride_mode,fused,block_dim", [
-    (12, 20, 16, "padded", True, 2),     # a workgroup's 32 positions straddle two requests
-    (40, 7, 8, "padded", False, 3),      # ... and five
+    (12, 20, 16, "padded", True, 2),     # a span of 16 positions and one of 4 per request
+    (40, 7, 8, "padded", False, 3),      # spans longer than a request
     (10, 48, 32, "half", True, 1),       # stride 16 < slots in use: neighbouring requests share rows
     (6, 100, 64, "zero", False, 2),      # stride 0: every request on the same rows
-    (1, 4096, 4096, "padded", True, 8),  # the largest one-launch call: one request of 4096 positions
+    (1, 4096, 4096, "padded", True, 8),  # one request of 4096 positions: every slot in use once
 ])
 def test_gather_small_batch_winners(kvops, req, top_k, dbs, stride_mode, fused, block_dim):
-    """The one-launch import (max_num_reqs * top_k <= 4096) against the oracle
-    on constructed inputs with many misses on one destination row: within a
-    request (the winner decided in LDS from the workgroup's own requests,
-    whose positions may straddle workgroups) and across requests (a stride
-    below the slots in use: device-scope tags of every position); invalid
-    tokens and slots, a request without a pool row; every hot byte and every
-    node's status words."""
+    """The one-launch import against the oracle on constructed inputs with many
+    misses on one destination row: within a request (whose positions lie in
+    several spans) and across requests (a stride below the slots in use: later
+    requests searched for the row); invalid tokens and slots, a request without
+    a pool row; every hot byte and every node's status words."""
     print("small import case", req, top_k, dbs, stride_mode, fused, block_dim, flush=True)
     L, layer, prefill, S, N = 2, 1, 512, 1, 2
     padded = (dbs + 15) // 16 * 16
@@ -292,9 +295,26 @@ def test_gather_empty_step_costs_no_more_for_a_larger_batch(kvops):
         pool.destroy(close_ext=False)
 
 
-@pytest.mark.parametrize("top_k", [1000, 3000])   # 3 x 1000 positions: one-launch form; 3 x 3000: two launches
+@pytest.mark.parametrize("top_k", [1000, 3000])   # one launch both
 @pytest.mark.parametrize("fused", [False, True])    # import_seg per segment, or import_all
 def test_gather_rows_past_layer_region(kvops, top_k, fused):
+    _past_layer_region(top_k, fused)
+
+
+@pytest.mark.parametrize("top_k,stripe,shared", [
+    (8200, 1, False),   # requests past 8192 positions
+    (3000, 1, True),    # stride 0 past 8192 positions
+    (1500, 2, False),   # striped past 4096 positions
+])
+@pytest.mark.parametrize("fused", [False, True])
+def test_gather_rows_past_layer_region_two_launches(kvops, top_k, stripe, shared, fused):
+    """The same where the import takes two launches, each followed by a
+    one-launch call on the stream that reports its own errors: the forms share
+    the counters and error words."""
+    _past_layer_region(top_k, fused, stripe, shared, then=700)
+
+
+def _past_layer_region(top_k, fused, stripe=1, shared=False, then=None):
     """Host rows whose segment row lies past the layer region (host base +
     token >= N * per_layer_seg_rows): the reference would read the next
     layer's region, or past the segment's end for the last layer
@@ -302,36 +322,41 @@ def test_gather_rows_past_layer_region(kvops, top_k, fused):
     as queued and still competes for its destination, and its block's status
     word carries 0x200 + (p & 0xFF) + (1 << 16) for the lowest such position
     p; the oracle applies the same rule.  Every hot byte and status word."""
-    print("past-region case", top_k, fused, flush=True)
+    print("past-region case", top_k, fused, stripe, shared, flush=True)
     req, L, prefill, dbs, N, block_dim = 3, 2, 4096, 2048, 2, 3
     padded = dbs
     layer_rows = req * prefill
-    pool = HostSegPool(0, L, layer_rows, ROW, stripe_rows=1, node_num=N)
+    pool = HostSegPool(0, L, layer_rows, ROW, stripe_rows=stripe, node_num=N)
     pool.create_pool()
     try:
         plsr = pool.per_layer_seg_rows
-        assert plsr * N == layer_rows
+        end = plsr * N * stripe  # the first host row past the region
+        assert stripe > 1 or end == layer_rows
         rng = np.random.default_rng(top_k + fused)
         views = pool.segment_views()
         for v in views:
             v[...] = rng.integers(0, 256, size=v.shape, dtype=np.uint8)
         segs = [v.reshape(-1) for v in views]
-        # request 2's run starts 1000 rows before the end of the layer, so its
+        # request 2's run starts 1000 rows before the end of the region, so its
         # tokens >= 1000 name rows past the region of either layer
-        host_base = np.array([0, prefill, layer_rows - 1000], dtype=np.int64)
-        topk = rng.integers(0, prefill, size=(req, top_k)).astype(np.int32)
-        slots = rng.integers(0, dbs, size=(req, top_k)).astype(np.int32)
-        miss = (rng.random((req, top_k)) < 0.6).astype(np.int8)
+        host_base = np.array([0, prefill, end - 1000], dtype=np.int64)
         pool_idx = np.arange(req, dtype=np.int64)
-        outside = (miss[2] != 0) & (host_base[2] + topk[2] >= layer_rows)
-        assert outside.sum() > 100
-        for layer in (0, L - 1):
+        stride = 0 if shared else padded
+        cases = []
+        for k in [top_k] if then is None else [top_k, then]:
+            topk = rng.integers(0, prefill, size=(req, k)).astype(np.int32)
+            slots = rng.integers(0, dbs, size=(req, k)).astype(np.int32)
+            miss = (rng.random((req, k)) < 0.6).astype(np.int8)
+            outside = (miss[2] != 0) & (host_base[2] + topk[2] >= end)
+            assert outside.sum() > 100
+            cases.append((k, topk, slots, miss))
+        for layer, (k, topk, slots, miss) in [(layer, c) for layer in (0, L - 1) for c in cases]:
             hot_np = rng.integers(0, 256, size=(req * padded, ROW), dtype=np.uint8)
             hot = torch.from_numpy(hot_np.copy()).cuda()
             args = (layer, to_dev(topk), to_dev(pool_idx), to_dev(host_base), to_dev(slots), to_dev(miss),
-                    to_dev(np.array([req], dtype=np.int32)), hot, req, top_k)
+                    to_dev(np.array([req], dtype=np.int32)), hot, req, k)
             read = pool.batch_read_fused if fused else pool.batch_read
-            status = read(*args, block_dim=block_dim, hot_req_stride_rows=padded)
+            status = read(*args, block_dim=block_dim, hot_req_stride_rows=stride)
             # the blocks that report the rows past the region fail the wait
             with pytest.raises(RuntimeError, match="kv op failed on node"):
                 pool.wait(status, block_dim=block_dim)
@@ -339,10 +364,10 @@ def test_gather_rows_past_layer_region(kvops, top_k, fused):
             errs = 0
             for s in range(N):
                 _, words = orc.gather_rows(segs, hot_np.reshape(-1), layer * plsr, ROW, topk, pool_idx, host_base,
-                                           slots, miss, req, top_k, req, 1, N, s, hot_req_stride_rows=padded,
+                                           slots, miss, req, k, req, stripe, N, s, hot_req_stride_rows=stride,
                                            block_dim=block_dim, per_layer_seg_rows=plsr)
                 got = _read_words(status + s * 64, block_dim)
-                assert got == [int(w) for w in words], (layer, s, [hex(w) for w in got], [hex(w) for w in words])
+                assert got == [int(w) for w in words], (layer, k, s, [hex(w) for w in got], [hex(w) for w in words])
                 errs += sum(1 for w in words if int(w) & 0xFFFFFFFF)
             assert errs >= 1, "no block reported the rows past the region"
             np.testing.assert_array_equal(hot.cpu().numpy(), hot_np, err_msg="layer {}".format(layer))
