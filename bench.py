@@ -785,8 +785,9 @@ def main():
             total += sum(hits)
         return total
 
-    # the library imports up to 4096 positions in one launch, larger batches in two
-    gather_kernels = ("kvx_gather_small",) if positions <= 4096 else ("kvx_gather_prep", "kvx_gather_span")
+    # the library imports in one launch, but requests past 8192 positions and striped batches past 4096 in two
+    one_launch = cfg.top_k <= 8192 and (cfg.stripe_rows <= 1 or positions <= 4096)
+    gather_kernels = ("kvx_gather_one",) if one_launch else ("kvx_gather_prep", "kvx_gather_span")
     gather_roof = {"kernel": "+".join(gather_kernels), "bound": "host-link", "achieved": link_gbps,
                    "peak": link["peak_GBps"], "unit": "GB/s", "frac": link_gbps / link["peak_GBps"],
                    "traffic": traffic_of(*gather_kernels), "traffic_source": traffic_src,

@@ -285,7 +285,7 @@ __host__ __device__ __forceinline__ BatchLayout batch_layout(uint32_t dbs, uint3
 //   newk [H/2]         new keys in event order: (home << 16) | (slot + 1)
 //   evict [H/32]       the step's evicted slots (bitmap)
 //   chunkA [H/kTblChunkCells]  per cell chunk: start of its cluster, or -1
-//   (cellw and chunkA hold min(H, kTblCells) cells)
+//   (of cellw and chunkA the first min(H, kTblCells) cells are used)
 constexpr uint32_t kTblChunkCells = 1024;    // survivors' cells per chunk
 constexpr uint32_t kTblChunkKeys = 1024;     // new keys per chunk
 // A hash has 16 bits, so homes lie in the first 2^16 cells, and fewer than

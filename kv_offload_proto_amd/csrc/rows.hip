@@ -15,8 +15,9 @@
 //
 // Completion: the last workgroup to finish (atomicInc ticket) stores the
 // status words with a system-scope release, after every workgroup fenced its
-// own row stores, or waited for stores that go through the caches.  The reference's per-block Commit/Drain + MTE3 flush has the
-// same meaning: all rows of the launch have landed.
+// own row stores, or waited for stores that go through the caches.  The
+// reference's per-block Commit/Drain + MTE3 flush has the same meaning: all
+// rows of the launch have landed.
 #include <cstddef>
 
 #include "kvx_internal.h"
@@ -373,8 +374,8 @@ __global__ __launch_bounds__(256) void kvx_gather_span(GatherParams P)
 // 651, 1024 662; spans of 128: 654 from 256).  Against a launch that marked
 // the winners in memory and one that listed and moved the rows: 8192 positions
 // 56 -> 47 us, 1665 positions in the earlier one-launch form, where every
-// workgroup counted all positions, 29 -> 19; 131072 positions 639 -> 633 (the
-// link).  The spans are those of the positions in use: a call, or a captured
+// workgroup counted all positions, 29 -> 19; 131072 positions 639 -> 633 (0.2
+// misses: the link).  The spans are those of the positions in use: a call, or a captured
 // graph's replay, with fewer requests than it was made for does nothing for
 // the others (256 requests of 1024 positions with 16 in use 102 us when every
 // span of the largest batch was walked, 77 so; with none 20 and 7).
@@ -383,8 +384,11 @@ constexpr uint32_t kOneMaxGroup = 8192;  // positions of a group (each workgroup
 constexpr uint32_t kOneMaxBlocks = 256;  // workgroups; more spans are taken in turn
 // Rows of a stripe share one segment row, whose repeats an XCD's L2 serves
 // when neighbouring positions meet there: larger calls of that kind keep the
-// two launches, whose 64 workgroups take 256 positions each (32768 positions,
-// stripes of 16: 178 us, 238 in short spans; 3600 positions: 64 and 37).
+// two launches, whose 64 workgroups take 256 positions each.  The line lies
+// where no stripe loses (0.3 misses, us in two launches and in one): 4096
+// positions 41.7 and 38.3 at stripes of 2, 38.6 and 38.3 at 64; 8192 66.7 and
+// 59.5 at 2, 61.3 and 58.9 at 16, 49.9 and 57.3 at 64; 32768 221 and 211 at 2,
+// 193 and 205 at 16, 142 and 185 at 64.
 constexpr uint32_t kOneMaxStriped = 4096;
 constexpr int kOneThreads = 256;
 
@@ -796,8 +800,8 @@ __global__ __launch_bounds__(256) void kvx_export_rows_copy(ExportRowsParams P)
 // the last workgroup (ticket) stores the status words and leaves the call's
 // counters zeroed.  The bound is latency: three dependent reads, a row's way
 // over the link and back.  Entries go to many workgroups (4 each up to 1024:
-// 64 rows, one
-// layer: 9.7 us from 2 workgroups ending in system-scope fences, 7.2 now).
+// 64 rows, one layer: 9.7 us from 2 workgroups ending in system-scope fences,
+// 6.8 now).
 constexpr uint32_t kExportSmallMax = 4096;
 constexpr uint32_t kExportSpanRows = 1024;  // up to here 4 entries a workgroup, else 16
 constexpr uint32_t kExportMaxSpan = 16;

@@ -30,7 +30,7 @@
 //     here), a cell empty before and after the step that starts the cell
 //     order, and per chunk of cells the start of its cluster and whether a
 //     deleted cell precedes it in the cluster (otherwise its survivors stay);
-//  3. chunks (one workgroup per chunk of 256 cells or 256 new keys): the
+//  3. chunks (one workgroup per chunk of 1024 cells or 1024 new keys): the
 //     chunk's free cells, then its keys in order; a survivor that lands on
 //     another cell, and every new key, writes its entry there.
 //
@@ -479,14 +479,14 @@ __device__ __forceinline__ void chunk_free_cells(uint32_t x0, uint32_t x1, uint3
     __syncthreads();
 }
 
-// The chunk's n <= 256 keys, in insertion order (home h, window-relative;
+// The chunk's n <= 1024 keys, in insertion order (home h, window-relative;
 // entry; own cell, window-relative, or kNoOwn), each into the first free cell
 // of win[] at or after its home, one after another.  The set of cells they
 // take does not depend on that order: going in in home order, key j (sorted)
 // takes the free cell of index r_j = max(p_j, r_{j-1} + 1), p_j the free cells
 // before its home, i.e. r_j = j + max_{i<=j} (p_i - i); z_j its cell.  In
 // insertion order each key then takes the first of those cells at or after
-// its home not taken before it: an index search in a 256-bit mask.
+// its home not taken before it (match_cells).
 constexpr uint32_t kNoOwn = 0xFFFFFFFFu;
 
 struct PlaceLds {
@@ -516,10 +516,11 @@ __device__ __forceinline__ uint32_t select_bit64(uint64_t x, uint32_t r)  // off
 // to L.sortedH[i].  By halving: the cells that the first half of the keys take
 // do not depend on their order (the backlog of their counts); those cells, in
 // order, and the rest are two problems of half the size, and a key's first
-// candidate in its half is the number of that half's cells before it.  Eight
-// levels of a scan in place of 256 searches one after another on one wave
-// (100k of a chunk's 130k cycles in a long cluster): the launch 315 -> 176 us at
-// 4 rows of 65518 slots in long clusters.  All threads call it; n <= kTblChunkCells,
+// candidate in its half is the number of that half's cells before it.  A scan a
+// level, ten of them (chunks of 256 keys, eight levels in place of 256 searches
+// one after another on one wave, 100k of a chunk's 130k cycles in a long
+// cluster: the launch 315 -> 176 us at 4 rows of 65518 slots in long clusters;
+// chunks of 1024: 62).  All threads call it; n <= kTblChunkCells,
 // the arrays are padded with keys that each take a cell of their own.
 __device__ __forceinline__ void match_cells(const PlaceLds &L, uint32_t n)
 {
@@ -761,7 +762,7 @@ __global__ __launch_bounds__(kTT) void kvx_sieve_table_chunks(TblParams P)
     bool survivors = blk < nS;
     uint32_t s0 = 0;
     if (survivors) {
-        // survivors of positions [s0, s0 + 256), after those of [A, s0) in the same cluster
+        // survivors of positions [s0, s0 + kTblChunkCells), after those of [A, s0) in the same cluster
         const int32_t a0 = reinterpret_cast<const KVX_GM int32_t *>(tb + P.t.chunkA)[blk];
         if (a0 < 0) return;
         s0 = blk * kTblChunkCells;
@@ -801,7 +802,7 @@ __global__ __launch_bounds__(kTT) void kvx_sieve_table_chunks(TblParams P)
 #ifdef KVX_BATCH_STAMPS
         t2 = __builtin_amdgcn_s_memtime();
 #endif
-        // the chunk's survivors in cell order (its cells are threads 0..255: whole waves)
+        // the chunk's survivors in cell order (a cell per thread)
         __shared__ uint32_t sWaveCnt[kTblChunkCells / 64];
         const bool surv = tid < kTblChunkCells && (cw & 0xFFFFu) != 0u;
         const uint64_t bm = __ballot(surv);
