@@ -125,7 +125,11 @@ __host__ __device__ __forceinline__ uint32_t align16(uint32_t x) { return (x + 1
 // cmask/emask/smask/rsn/rsm hold one 64-bit ballot per (wave, block of one
 // entry per lane).  ber, occ and fin are one bit per table cell: cells of
 // evicted tokens, the pre-step occupancy, the occupancy as the erase changes
-// it.  rnk: the event order of up to 64 slots (rows decided in registers).
+// it.  rnk: the event order of up to 64 slots (rows decided in registers); the
+// full form, whose direct map takes what is left anyway, gives it a bitmap's
+// room: with 128 bytes there too the registers of its kernels fall otherwise,
+// and rows decided in order lose 2 to 4 % (8 rows of 700 slots and 512
+// positions 476 and 485 us).
 constexpr uint32_t kRankBytes = 64u * 2u;
 __host__ __device__ __forceinline__ FastLayout fast_layout(uint32_t padded, uint32_t htSize, uint32_t topK,
                                                            uint32_t visStrideB, bool compact = false)
@@ -157,7 +161,7 @@ __host__ __device__ __forceinline__ FastLayout fast_layout(uint32_t padded, uint
     l.rsn = o;     o += ringMaskBytes;
     l.rsm = o;     o += ringMaskBytes;
     l.fin = o;     o += align16(bmBytes);
-    l.rnk = o;     o += kRankBytes;
+    l.rnk = o;     o += compact ? kRankBytes : align16(bmBytes);
     l.total = o;
     return l;
 }
@@ -208,12 +212,13 @@ __host__ __device__ __forceinline__ FastLayout fast_layout_fixed(uint32_t padded
     // the bitmap that the erase changes and the event orders take the
     // per-position classes' region, which the fixed kernels keep in registers
     // instead
-    if (align16(htSize / 8u) + kRankBytes <= Kx * 4u) {
+    const uint32_t rankBytes = compact ? kRankBytes : align16(htSize / 8u);
+    if (align16(htSize / 8u) + rankBytes <= Kx * 4u) {
         l.fin = l.pinf;
         l.rnk = l.pinf + align16(htSize / 8u);
     } else {
         l.fin = o;  o += align16(htSize / 8u);
-        l.rnk = o;  o += kRankBytes;
+        l.rnk = o;  o += rankBytes;
     }
     l.total = o;
     return l;
